@@ -225,25 +225,31 @@ __global__ void k_fill64(uint64_t* v, uint64_t n, uint64_t x) {
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix sort, 8 bits per pass: per-tile digit histograms, one scan
-// of the [digit][tile] matrix, then the scatter.  A tile is RS_TILE elements;
-// wave w of the block holds tile elements [w*RS_WSPAN, (w+1)*RS_WSPAN),
-// lane-minor, so (wave, item, lane) order is input order.  The scatter ranks
-// every element within its digit (ballots inside a wave, a per-wave LDS
-// counter across its items, a prefix over waves), sorts the tile in LDS, and
-// writes it out digit run by digit run, so consecutive lanes store to
-// consecutive addresses.
+// Stable LSD radix sort, three launches per pass: per-tile digit histograms,
+// the scan of each digit's row of the [digit][tile] matrix (one block per
+// digit), then the scatter, whose blocks scan the 256 digit totals
+// themselves.  The key bits are split evenly over ceil(bits / 8) passes
+// (20 bits: 7 + 7 + 6), which shortens the per-item ballot loop and
+// lengthens each digit's run.  A tile is 256 x RS_ITEMS elements; wave w of the
+// block holds tile elements [w*RS_WSPAN, (w+1)*RS_WSPAN), lane-minor, so
+// (wave, item, lane) order is input order.  The scatter ranks every element
+// within its digit (ballots inside a wave, a per-wave LDS counter across its
+// items, a prefix over waves), sorts the tile in LDS, and writes it out digit
+// run by digit run, so consecutive lanes store to consecutive addresses.
+// Bound: the stores of the digit runs (a pass over 2^24 u32 pairs moves 335
+// MB in about 120 us, 2.8 TB/s) and, below 2^20 pairs, launch latency (about
+// 4 us each).  Sort of u32 pairs by 24 bits against 5 launches a pass on
+// 4,096-element tiles: 2^24 pairs 370 -> 368 us, 2^20 90 -> 73 us, 180,000 80 ->
+// 39 us.
 // ---------------------------------------------------------------------------
 constexpr int RS_BT = 256;
-constexpr int RS_ITEMS = 16;
-constexpr int RS_TILE = RS_BT * RS_ITEMS;
 constexpr int RS_WAVES = RS_BT / 64;
-constexpr int RS_WSPAN = RS_ITEMS * 64;
 
-template <class KT>
+template <class KT, int RS_ITEMS>
 __global__ __launch_bounds__(RS_BT) void k_rs_hist(const KT* keys, uint64_t n, int shift, uint32_t dmask,
                                                    uint32_t* hist, uint32_t nb) {
   __shared__ uint32_t h[256];
+  constexpr int RS_TILE = RS_BT * RS_ITEMS;
   h[threadIdx.x] = 0;
   const uint64_t base = (uint64_t)blockIdx.x * RS_TILE;
   uint32_t d[RS_ITEMS];
@@ -257,21 +263,75 @@ __global__ __launch_bounds__(RS_BT) void k_rs_hist(const KT* keys, uint64_t n, i
   for (int i = 0; i < RS_ITEMS; ++i)
     if (d[i] < 256u) atomicAdd(&h[d[i]], 1u);
   __syncthreads();
-  hist[(uint64_t)threadIdx.x * nb + blockIdx.x] = h[threadIdx.x];
+  if (threadIdx.x <= dmask) {
+    hist[(uint64_t)threadIdx.x * nb + blockIdx.x] = h[threadIdx.x];
+    if (blockIdx.x + 1 == gridDim.x)  // the row's padding
+      for (uint32_t b = gridDim.x; b < nb; ++b) hist[(uint64_t)threadIdx.x * nb + b] = 0;
+  }
 }
 
-// offs[d * nb + b]: where tile b's first element of digit d goes; the digit
-// is (key >> shift) & dmask (dmask < 0xff only on a last, narrower pass)
-template <class KT>
+// Columns of a row of the [digit][tile] matrix: padded to whole 16-byte loads.
+inline uint32_t rs_stride(uint64_t nb) { return (uint32_t)((nb + 3) & ~3ull); }
+
+// offs[d][0..nb) <- exclusive scan of itself, totals[d] <- its sum; block d.
+// A thread takes 4 consecutive entries of each 1,024; the loads of 4,096
+// entries (16.8M elements) are issued before the first is used.
+__global__ __launch_bounds__(RS_BT) void k_rs_rowscan(uint32_t* offs, uint32_t nb, uint32_t* totals) {
+  constexpr int CH = 4;  // chunks of 4 * RS_BT entries per step
+  __shared__ uint32_t wsum[2][RS_WAVES];
+  uint4* row = reinterpret_cast<uint4*>(offs + (uint64_t)blockIdx.x * nb);
+  const uint32_t t = threadIdx.x, lane = dev::lane_id(), wave = t / 64, n4 = nb / 4;
+  uint32_t carry = 0;
+  int buf = 0;
+  for (uint32_t b0 = 0; b0 < n4; b0 += CH * RS_BT) {
+    uint4 v[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const uint32_t i = b0 + c * RS_BT + t;
+      v[c] = i < n4 ? row[i] : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (b0 + c * RS_BT >= n4) break;  // the same for the whole block
+      const uint32_t mine = v[c].x + v[c].y + v[c].z + v[c].w;
+      uint32_t x = mine;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)x, d, 64);
+        if (lane >= (uint32_t)d) x += o;
+      }
+      if (lane == 63) wsum[buf][wave] = x;
+      __syncthreads();  // one per chunk: the two halves of wsum alternate
+      uint32_t p = carry + x - mine;
+#pragma unroll
+      for (uint32_t w = 0; w < RS_WAVES; ++w) {
+        const uint32_t q = wsum[buf][w];
+        p += w < wave ? q : 0u;
+        carry += q;
+      }
+      buf ^= 1;
+      const uint32_t i = b0 + c * RS_BT + t;
+      if (i < n4) row[i] = make_uint4(p, p + v[c].x, p + v[c].x + v[c].y, p + v[c].x + v[c].y + v[c].z);
+    }
+  }
+  if (t == 0) totals[blockIdx.x] = carry;
+}
+
+// offs[d * nb + b]: where tile b's first element of digit d goes within the
+// digit, totals[d] the elements of digit d; the digit is the `width` bits of
+// the key from `shift` up
+template <class KT, int RS_ITEMS>
 __global__ __launch_bounds__(RS_BT) void k_rs_scatter(const KT* kin, const uint32_t* vin, KT* kout,
-                                                      uint32_t* vout, uint64_t n, int shift, uint32_t dmask,
-                                                      const uint32_t* offs, uint32_t nb) {
+                                                      uint32_t* vout, uint64_t n, int shift, int width,
+                                                      const uint32_t* offs, uint32_t nb, const uint32_t* totals) {
+  constexpr int RS_TILE = RS_BT * RS_ITEMS, RS_WSPAN = RS_ITEMS * 64;
   __shared__ KT skey[RS_TILE];
   __shared__ uint32_t sval[RS_TILE];
   __shared__ uint32_t wcnt[RS_WAVES][256];  // digit counts per wave, then each wave's start in the digit
   __shared__ uint32_t dstart[256];          // tile-local start of each digit
   __shared__ uint32_t gbase[256];           // global start of each digit's run from this tile
-  __shared__ uint32_t wsum[RS_WAVES];
+  __shared__ uint32_t wsum[RS_WAVES], wtot[RS_WAVES];
+  const uint32_t dmask = (1u << width) - 1u;
   const uint32_t t = threadIdx.x, lane = dev::lane_id(), wave = t / 64;
   const uint64_t base = (uint64_t)blockIdx.x * RS_TILE;
   const uint32_t cnt = n - base < (uint64_t)RS_TILE ? (uint32_t)(n - base) : (uint32_t)RS_TILE;
@@ -292,14 +352,18 @@ __global__ __launch_bounds__(RS_BT) void k_rs_scatter(const KT* kin, const uint3
   for (int i = 0; i < RS_ITEMS; ++i) {
     const bool valid = wave * RS_WSPAN + i * 64 + lane < cnt;
     const uint32_t d = (uint32_t)(k[i] >> shift) & dmask;
-    uint64_t peers = dev::ballot(valid);
+    const uint64_t act = dev::ballot(valid);
+    uint32_t plo = (uint32_t)act, phi = (uint32_t)(act >> 32);
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      const bool bit = (d >> b) & 1u;
-      const uint64_t bb = dev::ballot(bit);
-      peers &= bit ? bb : ~bb;
+      if (b >= width) break;
+      const uint64_t bb = dev::ballot((d >> b) & 1u);
+      const uint32_t m = (uint32_t)((int32_t)(d << (31 - b)) >> 31);  // all ones where the bit is set
+      plo &= ~((uint32_t)bb ^ m);
+      phi &= ~((uint32_t)(bb >> 32) ^ m);
     }
-    const uint32_t below = (uint32_t)__popcll(peers & dev::lanemask_lt());
+    const uint64_t peers = plo | ((uint64_t)phi << 32);
+    const uint32_t below = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, 0u));
     uint32_t old = 0;
     if (valid && below == 0) old = atomicAdd(&wcnt[wave][d], (uint32_t)__popcll(peers));
     const int leader = peers ? __ffsll((unsigned long long)peers) - 1 : (int)lane;
@@ -315,18 +379,30 @@ __global__ __launch_bounds__(RS_BT) void k_rs_scatter(const KT* kin, const uint3
     wcnt[w][t] = tot;
     tot += c;
   }
-  uint32_t x = tot;
+  const uint32_t all = t <= dmask ? totals[t] : 0u;
+  const uint32_t in_digit = t <= dmask ? offs[(uint64_t)t * nb + blockIdx.x] : 0u;
+  uint32_t x = tot, y = all;
 #pragma unroll
   for (int dd = 1; dd < 64; dd <<= 1) {
     const uint32_t o = (uint32_t)__shfl_up((int)x, dd, 64);
-    if (lane >= (uint32_t)dd) x += o;
+    const uint32_t q = (uint32_t)__shfl_up((int)y, dd, 64);
+    if (lane >= (uint32_t)dd) {
+      x += o;
+      y += q;
+    }
   }
-  if (lane == 63) wsum[wave] = x;
-  gbase[t] = offs[(uint64_t)t * nb + blockIdx.x];
+  if (lane == 63) {
+    wsum[wave] = x;
+    wtot[wave] = y;
+  }
   __syncthreads();
-  uint32_t carry = 0;
-  for (uint32_t w = 0; w < wave; ++w) carry += wsum[w];
+  uint32_t carry = 0, gcarry = 0;
+  for (uint32_t w = 0; w < wave; ++w) {
+    carry += wsum[w];
+    gcarry += wtot[w];
+  }
   dstart[t] = carry + x - tot;
+  gbase[t] = gcarry + y - all + in_digit;  // the digit's start, then this tile's place in it
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < RS_ITEMS; ++i) {
@@ -487,7 +563,7 @@ hipError_t scan_impl(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tm
   return hipGetLastError();
 }
 
-template <class KT>
+template <class KT, int ITEMS>
 hipError_t radix_impl(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, int key_bits,
                       uint32_t* tmp, KT** kout, uint32_t** vout, hipStream_t s) {
   KT* ka = k0;
@@ -495,17 +571,21 @@ hipError_t radix_impl(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, in
   KT* kb = k1;
   uint32_t* vb = v1;
   if (n > 1 && key_bits > 0) {
-    const uint64_t nb = (n + RS_TILE - 1) / RS_TILE;
+    const uint64_t nb = (n + RS_BT * ITEMS - 1) / (RS_BT * ITEMS);
+    const uint32_t stride = rs_stride(nb);
     uint32_t* hist = tmp;
-    uint32_t* stmp = tmp + 256 * nb;
-    for (int shift = 0; shift < key_bits; shift += 8) {
-      const uint32_t dmask = key_bits - shift >= 8 ? 0xffu : (1u << (key_bits - shift)) - 1u;
-      hipLaunchKernelGGL((k_rs_hist<KT>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, n, shift, dmask, hist,
-                         (uint32_t)nb);
-      hipError_t e = scan_impl<OpAdd, false>(hist, hist, 256 * nb, stmp, s);
+    uint32_t* totals = tmp + 256ull * stride;
+    const int passes = (key_bits + 7) / 8;
+    for (int p = 0, shift = 0; p < passes; ++p) {
+      const int width = (key_bits - shift + passes - p - 1) / (passes - p);  // what is left, evenly
+      const uint32_t dmask = (1u << width) - 1u;
+      hipLaunchKernelGGL((k_rs_hist<KT, ITEMS>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, n, shift, dmask, hist, stride);
+      hipLaunchKernelGGL(k_rs_rowscan, dim3(dmask + 1), dim3(RS_BT), 0, s, hist, stride, totals);
+      hipLaunchKernelGGL((k_rs_scatter<KT, ITEMS>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, va, kb, vb, n, shift, width,
+                         hist, stride, totals);
+      const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
-      hipLaunchKernelGGL((k_rs_scatter<KT>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, va, kb, vb, n,
-                         shift, dmask, hist, (uint32_t)nb);
+      shift += width;
       KT* tk = ka;
       ka = kb;
       kb = tk;
@@ -517,6 +597,20 @@ hipError_t radix_impl(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, in
   *kout = ka;
   *vout = va;
   return hipGetLastError();
+}
+
+// Items per thread (a tile is 256 x items).  Up to 2^20 elements a 4,096-element
+// tile leaves at most one block per CU, whose 16 items per wave then rank one
+// after another with nothing to hide their latency; above, the longer tile's
+// longer digit runs win.  24-bit sort, 16 / 4 items: 180,000 pairs 64 / 39 us,
+// 2^20 73 / 71 us, 2^21 84 / 107 us, 2^24 363 / 741 us.
+constexpr int RS_LONG = 16, RS_SHORT = 4;
+constexpr uint64_t RS_SHORT_MAX = 1ull << 20;
+template <class KT>
+hipError_t radix_sort(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, int key_bits, uint32_t* tmp, KT** kout,
+                      uint32_t** vout, hipStream_t s) {
+  return n <= RS_SHORT_MAX ? radix_impl<KT, RS_SHORT>(k0, v0, k1, v1, n, key_bits, tmp, kout, vout, s)
+                         : radix_impl<KT, RS_LONG>(k0, v0, k1, v1, n, key_bits, tmp, kout, vout, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -967,18 +1061,18 @@ hipError_t fill_u64(uint64_t* v, uint64_t n, uint64_t x, hipStream_t s) { GC_LAU
 
 uint64_t scan_tmp_words(uint64_t n) { return (n + SC_TILE - 1) / SC_TILE + 64; }
 uint64_t radix_sort_tmp_words(uint64_t n) {
-  const uint64_t nb = (n + RS_TILE - 1) / RS_TILE;
-  return 256 * nb + scan_tmp_words(256 * nb) + 64;
+  const uint64_t nb = (n + RS_BT * RS_SHORT - 1) / (RS_BT * RS_SHORT);
+  return 256ull * rs_stride(nb) + 256 + 64;
 }
 hipError_t radix_sort_u32(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint64_t n,
                           int key_bits, uint32_t* tmp, uint32_t** keys_out, uint32_t** vals_out,
                           hipStream_t s) {
-  return radix_impl<uint32_t>(k0, v0, k1, v1, n, key_bits, tmp, keys_out, vals_out, s);
+  return radix_sort<uint32_t>(k0, v0, k1, v1, n, key_bits, tmp, keys_out, vals_out, s);
 }
 hipError_t radix_sort_u64(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint64_t n,
                           int key_bits, uint32_t* tmp, uint64_t** keys_out, uint32_t** vals_out,
                           hipStream_t s) {
-  return radix_impl<uint64_t>(k0, v0, k1, v1, n, key_bits, tmp, keys_out, vals_out, s);
+  return radix_sort<uint64_t>(k0, v0, k1, v1, n, key_bits, tmp, keys_out, vals_out, s);
 }
 hipError_t inclusive_sum_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s) {
   return scan_impl<OpAdd, true>(in, out, n, tmp, s);
