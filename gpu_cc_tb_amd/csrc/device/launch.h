@@ -64,7 +64,6 @@ hipError_t radix_sort_u64(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1
 
 // --- scans (u32) --- tmp must hold scan_tmp_words(n) u32.
 uint64_t scan_tmp_words(uint64_t n);
-hipError_t inclusive_sum_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s);
 hipError_t inclusive_max_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s);
 
 // --- ordered-execution preprocessing ---
@@ -72,20 +71,27 @@ hipError_t inclusive_max_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint
 // flags (p or 0) and, when rowstart is given, row-start flags (p or 0).
 hipError_t access_group_flags(const uint32_t* srow, const uint32_t* sop, uint64_t n, uint32_t* flags,
                               hipStream_t s, uint32_t* rowstart = nullptr);
-// need[op] = gstart[p] + pos_base for op = sop[p] & OPID_MASK;
-// counters[row_slot(srow[p])] = p + pos_base at row starts.
-hipError_t access_need(const uint32_t* srow, const uint32_t* sop, const uint32_t* gstart,
-                       uint64_t n, uint32_t pos_base, uint32_t* need, uint32_t* counters,
-                       uint64_t nrows, hipStream_t s);
-// need[op] = gstart[p] - segstart[p] for op = sop[p] & OPID_MASK: the turn
-// relative to the row's first access, for counters that start at zero.
-// With comb_min > 0 it also lists every row queue of at least comb_min
-// accesses as (first position, length) in segs (seg_ctr counts them; at most
-// seg_cap are kept).
-hipError_t access_need_rel(const uint32_t* sop, const uint32_t* gstart, const uint32_t* segstart, uint64_t n,
-                           uint32_t* need, hipStream_t s, const uint32_t* srow = nullptr, uint64_t nrows = 0,
-                           uint32_t comb_min = 0, uint2* segs = nullptr, uint32_t* seg_ctr = nullptr,
-                           uint32_t seg_cap = 0);
+// From accesses sorted by (row, order): key[p] >> rb is the row, val[p] an
+// op id (op_ids).  need[op] (NEED_*) of every access that waits for another or
+// is waited for (the caller fills need with NEED_FREE first), counters[row] =
+// 0 for the rows where that happens.  With comb_min > 0 every row queue of at
+// least comb_min accesses is listed as (first position, length) in segs
+// (seg_ctr counts them; at most seg_cap are kept).  conflicts (may be null):
+// neighbours with equal keys where either writes, added to CONFLICT_SLOTS
+// counters 16 words apart.  tmp holds seg_tmp_words(n) u32.
+constexpr uint32_t CONFLICT_SLOTS = 16;
+uint64_t seg_tmp_words(uint64_t n);
+hipError_t seg_turns(const uint32_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
+                     uint32_t* counters, uint64_t nrows, uint32_t comb_min, uint2* segs, uint32_t* seg_ctr,
+                     uint32_t seg_cap, uint64_t* conflicts, hipStream_t s);
+hipError_t seg_turns64(const uint64_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
+                       uint32_t* counters, uint64_t nrows, uint64_t* conflicts, hipStream_t s);
+// GPUTx one-pass rank (src/gputx.cu:5-27) from accesses sorted by (row, tx),
+// val[p] the access's transaction with its write flag in bit 31: rank[tx] =
+// max over tx's accesses of the access-group boundaries of their rows up to
+// them (the caller zeroes rank and max_rank); max_rank = max.
+hipError_t seg_ranks(const uint32_t* row, const uint32_t* val, uint64_t n, uint32_t* tmp, uint64_t nrows,
+                     uint32_t* rank, uint32_t* max_rank, hipStream_t s);
 // GaccO, persistent form: run each listed row queue in order on the row's
 // cells (cols <= 64), store its reads' results, mark its ops need = NEED_DONE
 // and add the ops run to *combined.  wvals (nops u64) receives every op's
@@ -101,31 +107,12 @@ hipError_t access_need_open(const uint32_t* srow, const uint32_t* sop, const uin
                             uint64_t n, uint64_t nrows, const uint32_t* base, uint32_t* need, hipStream_t s);
 hipError_t row_base_add(const uint32_t* srow, const uint32_t* rstart, uint64_t n, uint64_t nrows, uint32_t* base,
                         hipStream_t s);
-// GPUTx: *conflicts += adjacent same-row, same-rank accesses where either
-// writes, from the (row << rank_bits | rank) sorted keys and the group flags.
-hipError_t gtx_conflicts(const uint64_t* skey, const uint32_t* flags, uint64_t n, uint64_t* conflicts,
-                         hipStream_t s);
-hipError_t gtx_conflicts32(const uint32_t* skey, const uint32_t* flags, uint64_t n, uint64_t* conflicts,
-                           hipStream_t s);
-// GPUTx one-pass rank (src/gputx.cu:5-27).  boundary[p] = 1 if p is not the
-// first access of its row and (p-1 or p) is a write; rowstart[p] = p at row
-// starts else 0.
-hipError_t gtx_flags(const uint32_t* srow, const uint32_t* sop, uint64_t n, uint64_t nrows, uint32_t* boundary,
-                     uint32_t* rowstart, hipStream_t s);
-// local rank = S[p] - S[SS[p]]; rank[tx] = max over tx's accesses, where
-// stx[p] is the transaction at sorted position p (write flag in bit 31);
-// max_rank = max.
-hipError_t gtx_rank(const uint32_t* stx, const uint32_t* S, const uint32_t* SS, uint64_t n,
-                    uint32_t* rank, uint32_t* max_rank, hipStream_t s);
 // composite key (row << rank_bits) | rank[op_tx[op]] for ops [0, n)
 hipError_t gtx_exec_keys(const uint32_t* rows, const uint32_t* op_tx, const uint32_t* rank,
                          uint64_t n, int rank_bits, uint64_t* keys, hipStream_t s);
 // the same key cut to 32 bits, for row_bits + rank_bits <= 32
 hipError_t gtx_exec_keys32(const uint32_t* rows, const uint32_t* op_tx, const uint32_t* rank,
                            uint64_t n, int rank_bits, uint32_t* keys, hipStream_t s);
-// out[i] = keys[i] >> shift
-hipError_t u64_key_high(const uint64_t* keys, uint64_t n, int shift, uint32_t* out, hipStream_t s);
-hipError_t u32_key_high(const uint32_t* keys, uint64_t n, int shift, uint32_t* out, hipStream_t s);
 hipError_t rank_hist(const uint32_t* rank, uint64_t ntx, uint32_t nranks, uint32_t* hist, hipStream_t s);
 
 // --- memory-system ceilings (microbench.hip) ---

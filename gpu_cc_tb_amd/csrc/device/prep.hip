@@ -426,17 +426,13 @@ __global__ __launch_bounds__(RS_BT) void k_rs_scatter(const KT* kin, const uint3
 }
 
 // ---------------------------------------------------------------------------
-// Scans over u32 with + or max.  Three kernels: block totals, a single-block
+// Inclusive scans over u32 (max).  Three kernels: block totals, a single-block
 // scan of the totals, and the block-local scan with its carry-in.
 // ---------------------------------------------------------------------------
 constexpr int SC_BT = 256;
 constexpr int SC_ITEMS = 16;
 constexpr int SC_TILE = SC_BT * SC_ITEMS;
 
-struct OpAdd {
-  static __device__ __forceinline__ uint32_t id() { return 0u; }
-  static __device__ __forceinline__ uint32_t f(uint32_t a, uint32_t b) { return a + b; }
-};
 struct OpMax {
   static __device__ __forceinline__ uint32_t id() { return 0u; }
   static __device__ __forceinline__ uint32_t f(uint32_t a, uint32_t b) { return a > b ? a : b; }
@@ -507,7 +503,7 @@ __global__ __launch_bounds__(SC_BT) void k_scan_top(uint32_t* sums, uint32_t nb)
 // of LDS.  Element j sits at LDS word j + j / 16, so the 16 consecutive words
 // of thread t start at 17 t and a wave's reads fall in distinct banks.  The
 // whole tile is loaded before any of it is stored, so in may equal out.
-template <class Op, bool INCLUSIVE>
+template <class Op>
 __global__ __launch_bounds__(SC_BT) void k_scan_down(const uint32_t* in, uint32_t* out, uint64_t n,
                                                      const uint32_t* sums) {
   static_assert(SC_ITEMS == 16, "the LDS padding assumes 16 items per thread");
@@ -536,13 +532,8 @@ __global__ __launch_bounds__(SC_BT) void k_scan_down(const uint32_t* in, uint32_
   uint32_t c = Op::f(sums[blockIdx.x], t == 0 ? Op::id() : tincl[t - 1]);
 #pragma unroll
   for (int i = 0; i < SC_ITEMS; ++i) {
-    if (INCLUSIVE) {
-      c = Op::f(c, vals[i]);
-      tile[t * 17 + i] = c;
-    } else {
-      tile[t * 17 + i] = c;
-      c = Op::f(c, vals[i]);
-    }
+    c = Op::f(c, vals[i]);
+    tile[t * 17 + i] = c;
   }
   __syncthreads();
 #pragma unroll
@@ -552,13 +543,13 @@ __global__ __launch_bounds__(SC_BT) void k_scan_down(const uint32_t* in, uint32_
   }
 }
 
-template <class Op, bool INCLUSIVE>
+template <class Op>
 hipError_t scan_impl(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s) {
   if (n == 0) return hipSuccess;
   const uint64_t nb = (n + SC_TILE - 1) / SC_TILE;
   hipLaunchKernelGGL((k_scan_reduce<Op>), dim3((unsigned)nb), dim3(SC_BT), 0, s, in, n, tmp);
   hipLaunchKernelGGL((k_scan_top<Op>), dim3(1), dim3(SC_BT), 0, s, tmp, (uint32_t)nb);
-  hipLaunchKernelGGL((k_scan_down<Op, INCLUSIVE>), dim3((unsigned)nb), dim3(SC_BT), 0, s, in, out, n,
+  hipLaunchKernelGGL((k_scan_down<Op>), dim3((unsigned)nb), dim3(SC_BT), 0, s, in, out, n,
                      tmp);
   return hipGetLastError();
 }
@@ -627,35 +618,288 @@ __global__ void k_access_group_flags(const uint32_t* srow, const uint32_t* sop, 
     if (rowstart) rowstart[p] = row0 ? (uint32_t)p : 0u;
   }
 }
-__global__ void k_access_need(const uint32_t* srow, const uint32_t* sop, const uint32_t* gstart,
-                              uint64_t n, uint32_t pos_base, uint32_t* need, uint32_t* counters,
-                              uint64_t nrows) {
-  const uint32_t shift = slot_shift(nrows);
-  for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
-       p += (uint64_t)gridDim.x * blockDim.x) {
-    need[sop[p] & OPID_MASK] = gstart[p] + pos_base;
-    // an index miss probes to the index length; such ops never execute
-    if (((p == 0) || srow[p] != srow[p - 1]) && srow[p] < nrows)
-      counters[row_slot(srow[p], shift)] = (uint32_t)p + pos_base;
+// ---------------------------------------------------------------------------
+// Turns and local ranks from accesses sorted by (row, order): val[p] carries
+// the access's write flag, key[p] >> rb is its row.  Position p starts a row
+// (EV_ROW), or a new access group of its row (EV_GROUP: it or the access
+// before it writes), or continues a run of reads (0).
+//
+// Two passes over tiles of TT elements, 8 consecutive ones per thread:
+// k_seg_tiles leaves each tile's last row start, last group start and the
+// group starts after its last row start; then a tile's carry-in is found by
+// reading the summaries before it backwards, 64 at a time (one step unless a
+// row spans more than 64 tiles), and everything else lies inside the tile.
+// This replaces group flags, two max-scans and a scatter over whole arrays
+// (and, for GPUTx, a sum-scan, a key shift and a conflict pass): on 2^24
+// accesses, theta 0.1, read ratio 0.9, GaccO's turns 432 -> 131 us (26 tiles,
+// 86 turns, 19 fill), GPUTx's ranks 290 -> 128 us and turns 500 -> 138 us.
+// Bound: the scattered need stores, which only accesses that meet another one
+// still make (the others keep NEED_FREE from a streaming fill).
+// ---------------------------------------------------------------------------
+constexpr int TT_ITEMS = 8;
+constexpr int TT = BT * TT_ITEMS;
+constexpr uint32_t EV_ROW = 1u, EV_GROUP = 2u;
+
+template <class KT>
+struct SegTile {
+  KT k[TT_ITEMS];
+  uint32_t v[TT_ITEMS];
+  KT pk;         // the access before the thread's first
+  uint32_t pv;
+  uint64_t p0;   // position of the thread's first access
+  uint32_t cnt;  // how many it has
+
+  __device__ __forceinline__ void load(const KT* key, const uint32_t* val, uint64_t n) {
+    p0 = (uint64_t)blockIdx.x * TT + (uint64_t)threadIdx.x * TT_ITEMS;
+    cnt = p0 >= n ? 0u : n - p0 < (uint64_t)TT_ITEMS ? (uint32_t)(n - p0) : (uint32_t)TT_ITEMS;
+    if (cnt == (uint32_t)TT_ITEMS) {
+      constexpr int Q = (int)sizeof(KT) * TT_ITEMS / 16;
+      uint4 q[Q], w[2];
+#pragma unroll
+      for (int i = 0; i < Q; ++i) q[i] = reinterpret_cast<const uint4*>(key + p0)[i];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) w[i] = reinterpret_cast<const uint4*>(val + p0)[i];
+      __builtin_memcpy(k, q, sizeof k);
+      __builtin_memcpy(v, w, sizeof v);
+    } else {
+#pragma unroll
+      for (int i = 0; i < TT_ITEMS; ++i) {
+        k[i] = (uint32_t)i < cnt ? key[p0 + i] : (KT)0;
+        v[i] = (uint32_t)i < cnt ? val[p0 + i] : 0u;
+      }
+    }
+    pk = cnt && p0 ? key[p0 - 1] : (KT)0;
+    pv = cnt && p0 ? val[p0 - 1] : 0u;
   }
+  // event of the thread's access i (0 past the end)
+  __device__ __forceinline__ uint32_t event(int i, int rb) const {
+    if ((uint32_t)i >= cnt) return 0u;
+    const KT a = i ? k[i - 1] : pk;
+    const uint32_t b = i ? v[i - 1] : pv;
+    if (p0 + i == 0 || (k[i] >> rb) != (a >> rb)) return EV_ROW;
+    return ((v[i] | b) & OPID_WRITE) ? EV_GROUP : 0u;
+  }
+};
+
+// exclusive max / sum over the block's threads before this one (all lanes of
+// the block take part); total: over the whole block
+struct SegScan {
+  uint32_t row, group;  // last row / group start + 1 (0: none)
+  uint32_t cnt;         // group starts since the last row start (or since the tile's first access)
+};
+__device__ __forceinline__ SegScan seg_join(const SegScan& a, const SegScan& b) {  // a before b
+  SegScan r;
+  r.row = b.row ? b.row : a.row;
+  r.group = b.group ? b.group : a.group;
+  r.cnt = b.row ? b.cnt : a.cnt + b.cnt;
+  return r;
+}
+__device__ __forceinline__ SegScan seg_block_scan(const SegScan& mine, SegScan* total) {
+  __shared__ SegScan ws[BT / 64];
+  const uint32_t lane = dev::lane_id(), wave = threadIdx.x / 64;
+  SegScan x = mine;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    SegScan o;
+    o.row = (uint32_t)__shfl_up((int)x.row, d, 64);
+    o.group = (uint32_t)__shfl_up((int)x.group, d, 64);
+    o.cnt = (uint32_t)__shfl_up((int)x.cnt, d, 64);
+    if (lane >= (uint32_t)d) x = seg_join(o, x);
+  }
+  if (lane == 63) ws[wave] = x;
+  SegScan e;
+  e.row = (uint32_t)__shfl_up((int)x.row, 1, 64);
+  e.group = (uint32_t)__shfl_up((int)x.group, 1, 64);
+  e.cnt = (uint32_t)__shfl_up((int)x.cnt, 1, 64);
+  if (lane == 0) e = SegScan{0, 0, 0};
+  __syncthreads();
+  SegScan before{0, 0, 0}, all{0, 0, 0};
+#pragma unroll
+  for (uint32_t w = 0; w < BT / 64; ++w) {
+    if (w < wave) before = seg_join(before, ws[w]);
+    all = seg_join(all, ws[w]);
+  }
+  *total = all;
+  return seg_join(before, e);
+}
+// what the thread's own accesses add to the scan
+template <class KT>
+__device__ __forceinline__ SegScan seg_own(const SegTile<KT>& t, int rb) {
+  SegScan s{0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < TT_ITEMS; ++i) {
+    const uint32_t e = t.event(i, rb);
+    const uint32_t p = (uint32_t)(t.p0 + i) + 1u;
+    if (e) s.group = p;
+    if (e == EV_ROW) {
+      s.row = p;
+      s.cnt = 0;
+    } else if (e == EV_GROUP) {
+      s.cnt++;
+    }
+  }
+  return s;
+}
+// Carry-in of tile b: the join of the summaries before it, read backwards by
+// the block's first wave until a row start is seen (the first access of all
+// starts a row).  Every thread of the block calls it.
+__device__ __forceinline__ SegScan seg_carry(const uint4* summ) {
+  __shared__ SegScan in;
+  if (threadIdx.x < 64) {
+    SegScan c{0, 0, 0};
+    const uint32_t lane = threadIdx.x;
+    for (uint32_t b = blockIdx.x; b > 0 && c.row == 0;) {
+      const bool has = lane < b;
+      const uint4 s = has ? summ[b - 1 - lane] : make_uint4(0, 0, 0, 0);
+      const uint64_t rows = dev::ballot(has && s.x != 0), groups = dev::ballot(has && s.y != 0);
+      // the tiles from the nearest one with a row start on (all, if none has)
+      const int rl = rows ? __ffsll((unsigned long long)rows) - 1 : 63;
+      uint32_t n = lane <= (uint32_t)rl ? s.z : 0u;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) n += (uint32_t)__shfl_xor((int)n, d, 64);
+      c.cnt += n;
+      if (rows) c.row = (uint32_t)__shfl((int)s.x, rl, 64);
+      if (groups && c.group == 0) c.group = (uint32_t)__shfl((int)s.y, __ffsll((unsigned long long)groups) - 1, 64);
+      b = b > 64 ? b - 64 : 0;
+    }
+    if (lane == 0) in = c;
+  }
+  __syncthreads();
+  return in;
 }
 
-__global__ void k_access_need_rel(const uint32_t* sop, const uint32_t* gstart, const uint32_t* segstart,
-                                  uint64_t n, uint32_t* need, const uint32_t* srow, uint64_t nrows,
-                                  uint32_t comb_min, uint2* segs, uint32_t* seg_ctr, uint32_t seg_cap) {
-  for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
-       p += (uint64_t)gridDim.x * blockDim.x) {
-    need[sop[p] & OPID_MASK] = gstart[p] - segstart[p];
-    // the last access of a row queue at least comb_min long lists the queue
-    // for a combiner
-    if (comb_min && (p + 1 == n || segstart[p + 1] != segstart[p])) {
-      const uint32_t len = (uint32_t)p + 1 - segstart[p];
-      if (len >= comb_min && srow[p] < nrows) {
-        const uint32_t i = atomicAdd(seg_ctr, 1u);
-        if (i < seg_cap) segs[i] = make_uint2(segstart[p], len);
+template <class KT>
+__global__ __launch_bounds__(BT) void k_seg_tiles(const KT* key, const uint32_t* val, uint64_t n, int rb, uint4* summ) {
+  SegTile<KT> t;
+  t.load(key, val, n);
+  SegScan total;
+  seg_block_scan(seg_own(t, rb), &total);
+  if (threadIdx.x == 0) summ[blockIdx.x] = make_uint4(total.row, total.group, total.cnt, 0u);
+}
+
+// need[op] (op = val & OPID_MASK) of every access that waits or is waited
+// for; the others keep NEED_FREE.  The counter of a row where that happens is
+// set to 0 at the row's first access.  comb_min > 0: every row queue of at
+// least comb_min accesses is listed as (first position, length) in segs.
+// conflicts (GPUTx): same-row neighbours of equal key (row and rank) where
+// either writes, added to CONFLICT_SLOTS counters on lines of their own.
+template <class KT>
+__global__ __launch_bounds__(BT) void k_seg_turns(const KT* key, const uint32_t* val, uint64_t n, int rb,
+                                                  const uint4* summ, uint32_t* need, uint32_t* counters,
+                                                  uint64_t nrows, uint32_t comb_min, uint2* segs, uint32_t* seg_ctr,
+                                                  uint32_t seg_cap, unsigned long long* conflicts) {
+  __shared__ uint32_t wnext[BT / 64];
+  SegTile<KT> t;
+  t.load(key, val, n);
+  const uint32_t lane = dev::lane_id(), wave = threadIdx.x / 64;
+  SegScan total, at = seg_block_scan(seg_own(t, rb), &total);
+  at = seg_join(seg_carry(summ), at);
+  // the first event at or after this thread's chunk, from the chunks after
+  // it in the wave, then in the block, then the next tile's first access (a
+  // run of reads that goes on there counts as followed: an unneeded
+  // increment changes nothing)
+  uint32_t first = 0;
+#pragma unroll
+  for (int i = TT_ITEMS - 1; i >= 0; --i) {
+    const uint32_t e = t.event(i, rb);
+    first = e ? e : first;
+  }
+  if (t.cnt < (uint32_t)TT_ITEMS && first == 0) first = EV_ROW;  // the end of the accesses
+  const uint64_t some = dev::ballot(first != 0), grp = dev::ballot(first == EV_GROUP);
+  if (lane == 0) wnext[wave] = some ? ((grp >> (__ffsll((unsigned long long)some) - 1)) & 1u ? EV_GROUP : EV_ROW) : 0u;
+  __syncthreads();
+  const uint64_t later = lane == 63 ? 0ull : some & (~0ull << (lane + 1));
+  uint32_t next = 0;
+  if (later) {
+    next = (grp >> (__ffsll((unsigned long long)later) - 1)) & 1u ? EV_GROUP : EV_ROW;
+  } else {
+#pragma unroll
+    for (uint32_t w = 0; w < BT / 64; ++w)
+      if (w > wave && next == 0) next = wnext[w];
+    if (next == 0) {
+      const uint64_t e = (uint64_t)(blockIdx.x + 1) * TT;
+      next = e >= n || (key[e] >> rb) != (key[e - 1] >> rb) ? EV_ROW : EV_GROUP;
+    }
+  }
+  // does the chunk's last access end its row queue?
+  KT nk = 0;
+  {
+    const uint32_t lo = (uint32_t)__shfl_down((int)(uint32_t)t.k[0], 1, 64);
+    nk = (KT)lo;
+    if constexpr (sizeof(KT) == 8)
+      nk |= (KT)((uint64_t)(uint32_t)__shfl_down((int)(uint32_t)((uint64_t)t.k[0] >> 32), 1, 64) << 32);
+    const uint64_t e = t.p0 + TT_ITEMS;
+    if (lane == 63) nk = e < n ? key[e] : (KT)0;
+  }
+  // what follows each access: walk backwards
+  uint32_t nx[TT_ITEMS];
+#pragma unroll
+  for (int i = TT_ITEMS - 1; i >= 0; --i) {
+    if (i + 1 < TT_ITEMS) {
+      const uint32_t e = t.event(i + 1, rb);
+      nx[i] = e ? e : (uint32_t)i + 1 < t.cnt ? nx[i + 1] : (uint32_t)EV_ROW;
+    } else {
+      nx[i] = next;
+    }
+  }
+  uint64_t same = 0;
+#pragma unroll
+  for (int i = 0; i < TT_ITEMS; ++i) {
+    if ((uint32_t)i >= t.cnt) break;
+    const uint32_t e = t.event(i, rb), p = (uint32_t)(t.p0 + i);
+    if (e) at.group = p + 1;
+    if (e == EV_ROW) at.row = p + 1;
+    const uint64_t row = (uint64_t)(t.k[i] >> rb);
+    if (e == EV_GROUP && conflicts) same += t.k[i] == (i ? t.k[i - 1] : t.pk) ? 1u : 0u;
+    if (row >= nrows) continue;  // an index miss never executes
+    const uint32_t wait = at.group - at.row;
+    const bool followed = nx[i] == EV_GROUP;
+    if (wait || followed) need[t.v[i] & OPID_MASK] = wait | (followed ? 0u : NEED_LAST);
+    if (e == EV_ROW && followed) counters[row_slot((uint32_t)row, slot_shift(nrows))] = 0u;
+    if (comb_min) {
+      const uint64_t q = t.p0 + i + 1;
+      const KT k1 = i + 1 < TT_ITEMS ? t.k[i + 1] : nk;
+      if (q == n || (k1 >> rb) != (t.k[i] >> rb)) {
+        const uint32_t len = p + 2 - at.row;
+        if (len >= comb_min) {
+          const uint32_t s = atomicAdd(seg_ctr, 1u);
+          if (s < seg_cap) segs[s] = make_uint2(at.row - 1, len);
+        }
       }
     }
   }
+  if (conflicts) {
+    same = block_reduce_u64<false>(same);
+    if (threadIdx.x == 0 && same)
+      atomicAdd(conflicts + 16 * (blockIdx.x % launch::CONFLICT_SLOTS), (unsigned long long)same);
+  }
+}
+
+// GPUTx one-pass rank (src/gputx.cu:5-27): an access's local rank is the
+// number of group starts in its row up to it; rank[tx] = max over tx's
+// accesses, tx = val & OPID_MASK here; max_rank = max.
+__global__ __launch_bounds__(BT) void k_seg_ranks(const uint32_t* key, const uint32_t* val, uint64_t n,
+                                                  const uint4* summ, uint64_t nrows, uint32_t* rank,
+                                                  uint32_t* max_rank) {
+  SegTile<uint32_t> t;
+  t.load(key, val, n);
+  SegScan total, at = seg_block_scan(seg_own(t, 0), &total);
+  at = seg_join(seg_carry(summ), at);
+  uint32_t mx = 0;
+#pragma unroll
+  for (int i = 0; i < TT_ITEMS; ++i) {
+    const uint32_t e = t.event(i, 0);
+    if (e == EV_ROW) at.cnt = 0;
+    if (e == EV_GROUP) at.cnt++;
+    // index misses (IDX_MISS sorts last) never execute and raise no rank
+    if ((uint32_t)i < t.cnt && at.cnt && t.k[i] < nrows) {
+      atomicMax(&rank[t.v[i] & OPID_MASK], at.cnt);  // ranks start at 0
+      mx = at.cnt > mx ? at.cnt : mx;
+    }
+  }
+  mx = (uint32_t)block_reduce_u64<true>(mx);
+  // few blocks raise the maximum: look before the one-address atomic
+  if (threadIdx.x == 0 && mx > dev::ld32(max_rank)) atomicMax(max_rank, mx);
 }
 
 // ---------------------------------------------------------------------------
@@ -790,59 +1034,12 @@ __global__ void k_row_base_add(const uint32_t* srow, const uint32_t* rstart, uin
   }
 }
 
-// GPUTx same-rank conflicts: adjacent accesses of one row with equal rank
-// where either writes.  In the (row << rank_bits | rank) sorted keys, same
-// row and rank means equal keys; flags[p] (access_group_flags) is non-zero
-// at a non-row-start position exactly when either access writes.
-template <class KT>
-__global__ void k_gtx_conflicts(const KT* skey, const uint32_t* flags, uint64_t n,
-                                unsigned long long* conflicts) {
-  uint64_t local = 0;
-  for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x + 1; p < n;
-       p += (uint64_t)gridDim.x * blockDim.x)
-    local += (skey[p] == skey[p - 1] && flags[p] != 0u) ? 1u : 0u;
-  // one atomic per block (launched with reduce_blocks)
-  local = block_reduce_u64<false>(local);
-  if (threadIdx.x == 0 && local) atomicAdd(conflicts, (unsigned long long)local);
-}
-
-__global__ void k_gtx_flags(const uint32_t* srow, const uint32_t* sop, uint64_t n, uint64_t nrows,
-                            uint32_t* boundary, uint32_t* rowstart) {
-  for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
-       p += (uint64_t)gridDim.x * blockDim.x) {
-    const bool start = (p == 0) || srow[p] != srow[p - 1];
-    rowstart[p] = start ? (uint32_t)p : 0u;
-    // index misses (IDX_MISS sorts last) never execute and raise no rank
-    boundary[p] = (!start && srow[p] < nrows &&
-                   ((sop[p] | sop[p - 1]) & OPID_WRITE) != 0u) ? 1u : 0u;
-  }
-}
-// stx[p]: the transaction of sorted position p (write flag in bit 31)
-__global__ void k_gtx_rank(const uint32_t* stx, const uint32_t* S, const uint32_t* SS, uint64_t n,
-                           uint32_t* rank, uint32_t* max_rank) {
-  uint32_t mx = 0;
-  for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
-       p += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t local = S[p] - S[SS[p]];
-    if (local) atomicMax(&rank[stx[p] & OPID_MASK], local);  // ranks start at 0
-    mx = local > mx ? local : mx;
-  }
-  // one atomic per block (launched with reduce_blocks)
-  mx = (uint32_t)block_reduce_u64<true>(mx);
-  if (threadIdx.x == 0 && mx) atomicMax(max_rank, mx);
-}
 template <class KT>
 __global__ void k_gtx_exec_keys(const uint32_t* rows, const uint32_t* op_tx, const uint32_t* rank,
                                 uint64_t n, int rank_bits, KT* keys) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
     keys[i] = (KT)(((uint64_t)rows[i] << rank_bits) | rank[op_tx[i]]);
-}
-template <class KT>
-__global__ void k_key_high(const KT* keys, uint64_t n, int shift, uint32_t* out) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    out[i] = (uint32_t)(keys[i] >> shift);
 }
 // Histogram of ranks (gputx_pre3, src/gputx.cu:30-38).  There are usually few
 // ranks, so each block counts into LDS and adds its non-zero bins once.
@@ -1074,25 +1271,44 @@ hipError_t radix_sort_u64(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1
                           hipStream_t s) {
   return radix_sort<uint64_t>(k0, v0, k1, v1, n, key_bits, tmp, keys_out, vals_out, s);
 }
-hipError_t inclusive_sum_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s) {
-  return scan_impl<OpAdd, true>(in, out, n, tmp, s);
-}
 hipError_t inclusive_max_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s) {
-  return scan_impl<OpMax, true>(in, out, n, tmp, s);
+  return scan_impl<OpMax>(in, out, n, tmp, s);
 }
 hipError_t access_group_flags(const uint32_t* srow, const uint32_t* sop, uint64_t n, uint32_t* flags,
                               hipStream_t s, uint32_t* rowstart) {
   GC_LAUNCH(k_access_group_flags, n, srow, sop, n, flags, rowstart);
 }
-hipError_t access_need(const uint32_t* srow, const uint32_t* sop, const uint32_t* gstart,
-                       uint64_t n, uint32_t pos_base, uint32_t* need, uint32_t* counters,
-                       uint64_t nrows, hipStream_t s) {
-  GC_LAUNCH(k_access_need, n, srow, sop, gstart, n, pos_base, need, counters, nrows);
+uint64_t seg_tmp_words(uint64_t n) { return 4 * ((n + TT - 1) / TT); }
+template <class KT>
+static hipError_t seg_turns_impl(const KT* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
+                                 uint32_t* counters, uint64_t nrows, uint32_t comb_min, uint2* segs, uint32_t* seg_ctr,
+                                 uint32_t seg_cap, uint64_t* conflicts, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  const unsigned nb = (unsigned)((n + TT - 1) / TT);
+  uint4* summ = reinterpret_cast<uint4*>(tmp);
+  hipLaunchKernelGGL((k_seg_tiles<KT>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ);
+  hipLaunchKernelGGL((k_seg_turns<KT>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, need, counters, nrows, comb_min,
+                     segs, seg_ctr, seg_cap, (unsigned long long*)conflicts);
+  return hipGetLastError();
 }
-hipError_t access_need_rel(const uint32_t* sop, const uint32_t* gstart, const uint32_t* segstart, uint64_t n,
-                           uint32_t* need, hipStream_t s, const uint32_t* srow, uint64_t nrows, uint32_t comb_min,
-                           uint2* segs, uint32_t* seg_ctr, uint32_t seg_cap) {
-  GC_LAUNCH(k_access_need_rel, n, sop, gstart, segstart, n, need, srow, nrows, comb_min, segs, seg_ctr, seg_cap);
+hipError_t seg_turns(const uint32_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
+                     uint32_t* counters, uint64_t nrows, uint32_t comb_min, uint2* segs, uint32_t* seg_ctr,
+                     uint32_t seg_cap, uint64_t* conflicts, hipStream_t s) {
+  return seg_turns_impl(key, val, n, rb, tmp, need, counters, nrows, comb_min, segs, seg_ctr, seg_cap, conflicts, s);
+}
+hipError_t seg_turns64(const uint64_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
+                       uint32_t* counters, uint64_t nrows, uint64_t* conflicts, hipStream_t s) {
+  return seg_turns_impl(key, val, n, rb, tmp, need, counters, nrows, 0u, (uint2*)nullptr, (uint32_t*)nullptr, 0u,
+                        conflicts, s);
+}
+hipError_t seg_ranks(const uint32_t* row, const uint32_t* val, uint64_t n, uint32_t* tmp, uint64_t nrows,
+                     uint32_t* rank, uint32_t* max_rank, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  const unsigned nb = (unsigned)((n + TT - 1) / TT);
+  uint4* summ = reinterpret_cast<uint4*>(tmp);
+  hipLaunchKernelGGL((k_seg_tiles<uint32_t>), dim3(nb), dim3(BT), 0, s, row, val, n, 0, summ);
+  hipLaunchKernelGGL(k_seg_ranks, dim3(nb), dim3(BT), 0, s, row, val, n, summ, nrows, rank, max_rank);
+  return hipGetLastError();
 }
 hipError_t gacco_combine(const uint2* segs, const uint32_t* seg_ctr, uint32_t seg_cap, const uint32_t* srow,
                          const uint32_t* sop, const uint64_t* ops, const uint32_t* op_tx, const uint64_t* tx_off,
@@ -1109,22 +1325,6 @@ hipError_t gacco_combine(const uint2* segs, const uint32_t* seg_ctr, uint32_t se
                      cells, cols, reads, need, combined);
   return hipGetLastError();
 }
-hipError_t gtx_conflicts(const uint64_t* skey, const uint32_t* flags, uint64_t n, uint64_t* conflicts,
-                         hipStream_t s) {
-  GC_LAUNCH_REDUCE(k_gtx_conflicts<uint64_t>, n, skey, flags, n, (unsigned long long*)conflicts);
-}
-hipError_t gtx_conflicts32(const uint32_t* skey, const uint32_t* flags, uint64_t n, uint64_t* conflicts,
-                           hipStream_t s) {
-  GC_LAUNCH_REDUCE(k_gtx_conflicts<uint32_t>, n, skey, flags, n, (unsigned long long*)conflicts);
-}
-hipError_t gtx_flags(const uint32_t* srow, const uint32_t* sop, uint64_t n, uint64_t nrows, uint32_t* boundary,
-                     uint32_t* rowstart, hipStream_t s) {
-  GC_LAUNCH(k_gtx_flags, n, srow, sop, n, nrows, boundary, rowstart);
-}
-hipError_t gtx_rank(const uint32_t* stx, const uint32_t* S, const uint32_t* SS, uint64_t n,
-                    uint32_t* rank, uint32_t* max_rank, hipStream_t s) {
-  GC_LAUNCH_REDUCE(k_gtx_rank, n, stx, S, SS, n, rank, max_rank);
-}
 hipError_t gtx_exec_keys(const uint32_t* rows, const uint32_t* op_tx, const uint32_t* rank,
                          uint64_t n, int rank_bits, uint64_t* keys, hipStream_t s) {
   GC_LAUNCH(k_gtx_exec_keys<uint64_t>, n, rows, op_tx, rank, n, rank_bits, keys);
@@ -1132,12 +1332,6 @@ hipError_t gtx_exec_keys(const uint32_t* rows, const uint32_t* op_tx, const uint
 hipError_t gtx_exec_keys32(const uint32_t* rows, const uint32_t* op_tx, const uint32_t* rank,
                            uint64_t n, int rank_bits, uint32_t* keys, hipStream_t s) {
   GC_LAUNCH(k_gtx_exec_keys<uint32_t>, n, rows, op_tx, rank, n, rank_bits, keys);
-}
-hipError_t u64_key_high(const uint64_t* keys, uint64_t n, int shift, uint32_t* out, hipStream_t s) {
-  GC_LAUNCH(k_key_high<uint64_t>, n, keys, n, shift, out);
-}
-hipError_t u32_key_high(const uint32_t* keys, uint64_t n, int shift, uint32_t* out, hipStream_t s) {
-  GC_LAUNCH(k_key_high<uint32_t>, n, keys, n, shift, out);
 }
 hipError_t rank_hist(const uint32_t* rank, uint64_t ntx, uint32_t nranks, uint32_t* hist, hipStream_t s) {
   uint64_t blocks = (ntx + 4095) / 4096;

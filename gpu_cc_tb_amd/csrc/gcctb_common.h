@@ -56,7 +56,13 @@ constexpr uint32_t OPID_MASK = 0x7fffffffu;
 // The key bucket of the hot-key counts (Fibonacci hash into 2^16 buckets).
 constexpr uint32_t DEFER_BUCKET_BITS = 16;
 GC_HD uint32_t defer_bucket(uint32_t key) { return (key * 2654435761u) >> (32 - DEFER_BUCKET_BITS); }
-// need[op] of an op that a row's combiner already executed (GaccO, persistent form)
+// GaccO / GPUTx: need[op] is the count of completed accesses to its row that
+// the op waits for (0: nothing to wait for), with NEED_LAST set when no later
+// access to the row waits for anything, so that the op's own completion need
+// not be counted.  NEED_FREE is an op that meets no other: it neither polls
+// nor counts.  NEED_DONE: a row's combiner already executed the op (GaccO).
+constexpr uint32_t NEED_LAST = 0x80000000u;
+constexpr uint32_t NEED_FREE = NEED_LAST;
 constexpr uint32_t NEED_DONE = 0xffffffffu;
 
 // ---------------------------------------------------------------------------
@@ -296,7 +302,7 @@ struct ExecArgs {
   uint64_t pool_cap;       // MVCC: node capacity
   uint32_t* counters;      // gacco/gputx: per-row completed-access counter, at the row's slot
   uint32_t slot_shift;     // slot_shift(rows)
-  const uint32_t* need;    // gacco/gputx: per-op access-group start
+  const uint32_t* need;    // gacco/gputx: per-op turn (NEED_*)
   uint64_t* ctrs;          // ticket, pool top and timestamp shards (CTR_* word offsets)
   // outputs
   uint32_t* rows_out;      // per op: row the index returned

@@ -144,7 +144,7 @@ struct gcctb_ctx {
   gcctb::DevBuf<uint32_t> tx_aborts;
   gcctb::DevBuf<gcctb::Metrics> metrics;
   // preprocessing scratch
-  gcctb::DevBuf<uint32_t> sk0, sv0, sk1, sv1, flags, gstart, sort_tmp, S, SS;
+  gcctb::DevBuf<uint32_t> sk0, sv0, sk1, sv1, flags, gstart, sort_tmp;
   gcctb::DevBuf<uint64_t> sk64a, sk64b;
   gcctb::DevBuf<uint32_t> rank, tx_map, max_rank;
   // hot-writer deferral: sampled counts and state, slot -> transaction map;
@@ -398,14 +398,14 @@ class GaccoHost : public SchemeHost {
   using SchemeHost::SchemeHost;
   void Init(int batch_id, uint64_t batch_st) override {
     const uint64_t n_tx = batches[batch_id];
-    prep_range(ctx.h_tx_off[batch_st], ctx.h_tx_off[batch_st + n_tx]);
+    prep_range(ctx.h_tx_off[batch_st], ctx.h_tx_off[batch_st + n_tx], false);
   }
   // The persistent form queues every row's accesses of the whole stream in
   // transaction-id order: the outcome is that of the serial run in id order,
   // the same as batch after batch.
   void PrepStream() override { prep_range(0, ctx.nops, true); }
   void PostStream() override {}
-  void PrepLaunch(uint64_t o0, uint64_t o1) override { prep_range(o0, o1); }
+  void PrepLaunch(uint64_t o0, uint64_t o1) override { prep_range(o0, o1, false); }
   bool ProbesRows() const override { return true; }
   // Open launch: every row's queue starts empty; each admitted batch's
   // accesses queue behind those of the batches admitted before it, in
@@ -432,12 +432,9 @@ class GaccoHost : public SchemeHost {
   }
   bool OpenRowsProbed() const override { return true; }
   // per-row access queues for ops [o0, o1) in (row, transaction id) order;
-  // the rows also land in rows_out[o0, o1).  relative: turns count from the
-  // row's first access and the counters start from one dense zero fill (the
-  // whole stream at once); otherwise each touched row's counter is set to
-  // its first position, which costs a random store per row but no fill of
-  // the whole array (one batch at a time).
-  void prep_range(uint64_t o0, uint64_t o1, bool relative = false) {
+  // the rows also land in rows_out[o0, o1).  stream: the whole stream at
+  // once, whose long row queues go to combiners (column mode).
+  void prep_range(uint64_t o0, uint64_t o1, bool stream) {
     const uint64_t n = o1 - o0;
     if (n == 0) return;
     hipStream_t s = ctx.stream;
@@ -446,33 +443,18 @@ class GaccoHost : public SchemeHost {
     // rows are below cfg.rows; a miss (IDX_MISS) has all row bits set and sorts last
     HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, bits_for(ctx.cfg.rows),
                                    ctx.sort_tmp.p, &srow, &sop, s));
-    if (relative) {
-      // the sort's other key and value buffers are free now: row-start flags
-      // and the row start of every position
-      uint32_t* rflags = srow == ctx.sk0.p ? ctx.sk1.p : ctx.sk0.p;
-      uint32_t* rstart = sop == ctx.sv0.p ? ctx.sv1.p : ctx.sv0.p;
-      HIP_TRY(launch::access_group_flags(srow, sop, n, ctx.flags.p, s, rflags));
-      HIP_TRY(launch::inclusive_max_u32(ctx.flags.p, ctx.gstart.p, n, ctx.sort_tmp.p, s));
-      HIP_TRY(launch::inclusive_max_u32(rflags, rstart, n, ctx.sort_tmp.p, s));
-      // rows with long queues go to combiners (whole stream, column mode)
-      const bool comb = ctx.scheme == SCHEME_GACCO && ctx.comb_min && ctx.comb_cap && ctx.cfg.cols <= 64 &&
-                        o0 == 0 && !ctx.cfg.row_ops && !ctx.tpcc;
-      if (comb) HIP_TRY(launch::fill_u64(ctx.comb_ctr.p, 2, 0, s));
-      uint2* segs = reinterpret_cast<uint2*>(ctx.comb_segs.p);
-      uint32_t* nseg = reinterpret_cast<uint32_t*>(ctx.comb_ctr.p);
-      HIP_TRY(launch::access_need_rel(sop, ctx.gstart.p, rstart, n, ctx.need.p, s, srow, ctx.cfg.rows,
-                                      comb ? ctx.comb_min : 0u, segs, nseg, (uint32_t)ctx.comb_cap));
-      if (comb)
-        HIP_TRY(launch::gacco_combine(segs, nseg, (uint32_t)ctx.comb_cap, srow, sop, ctx.ops.p, ctx.op_tx.p,
-                                      ctx.tx_off.p, ctx.nops, ctx.cells.p, ctx.cfg.cols, ctx.cfg.seed, ctx.comb_wv.p,
-                                      ctx.reads.p, ctx.need.p, ctx.comb_ctr.p + 1, s));
-      combined_ = comb;
-      HIP_TRY(launch::fill_u32(ctx.counters.p, ctx.counters.n, 0, s));
-      return;
-    }
-    HIP_TRY(launch::access_group_flags(srow, sop, n, ctx.flags.p, s));
-    HIP_TRY(launch::inclusive_max_u32(ctx.flags.p, ctx.gstart.p, n, ctx.sort_tmp.p, s));
-    HIP_TRY(launch::access_need(srow, sop, ctx.gstart.p, n, 0, ctx.need.p, ctx.counters.p, ctx.cfg.rows, s));
+    const bool comb = stream && ctx.comb_min && ctx.comb_cap && ctx.cfg.cols <= 64 && !ctx.cfg.row_ops && !ctx.tpcc;
+    if (comb) HIP_TRY(launch::fill_u64(ctx.comb_ctr.p, 2, 0, s));
+    uint2* segs = reinterpret_cast<uint2*>(ctx.comb_segs.p);
+    uint32_t* nseg = reinterpret_cast<uint32_t*>(ctx.comb_ctr.p);
+    HIP_TRY(launch::fill_u32(ctx.need.p + o0, n, NEED_FREE, s));
+    HIP_TRY(launch::seg_turns(srow, sop, n, 0, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows,
+                              comb ? ctx.comb_min : 0u, segs, nseg, (uint32_t)ctx.comb_cap, nullptr, s));
+    if (comb)
+      HIP_TRY(launch::gacco_combine(segs, nseg, (uint32_t)ctx.comb_cap, srow, sop, ctx.ops.p, ctx.op_tx.p,
+                                    ctx.tx_off.p, ctx.nops, ctx.cells.p, ctx.cfg.cols, ctx.cfg.seed, ctx.comb_wv.p,
+                                    ctx.reads.p, ctx.need.p, ctx.comb_ctr.p + 1, s));
+    if (stream) combined_ = comb;
   }
   void Launch(int b, uint64_t lo, uint64_t hi, bool persist) override {
     const ExecArgs a = args(b, lo, hi);
@@ -537,12 +519,9 @@ class GPUTxHost : public SchemeHost {
     HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, row_bits, ctx.sort_tmp.p,
                                    &srow, &stx_ops, s));
     // one-pass local ranks and rank[tx] = max (src/gputx.cu:5-27)
-    HIP_TRY(launch::gtx_flags(srow, stx_ops, n, ctx.cfg.rows, ctx.flags.p, ctx.gstart.p, s));
-    HIP_TRY(launch::inclusive_sum_u32(ctx.flags.p, ctx.S.p, n, ctx.sort_tmp.p, s));
-    HIP_TRY(launch::inclusive_max_u32(ctx.gstart.p, ctx.SS.p, n, ctx.sort_tmp.p, s));
     HIP_TRY(launch::fill_u32(ctx.rank.p, ntx, 0, s));
     HIP_TRY(launch::fill_u32(ctx.max_rank.p, 1, 0, s));
-    HIP_TRY(launch::gtx_rank(stx_ops, ctx.S.p, ctx.SS.p, n, ctx.rank.p, ctx.max_rank.p, s));
+    HIP_TRY(launch::seg_ranks(srow, stx_ops, n, ctx.sort_tmp.p, ctx.cfg.rows, ctx.rank.p, ctx.max_rank.p, s));
     uint32_t max_rank = 0;
     HIP_TRY(hipMemcpyAsync(&max_rank, ctx.max_rank.p, 4, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
@@ -558,43 +537,26 @@ class GPUTxHost : public SchemeHost {
     HIP_TRY(hipMemcpyAsync(ctx.tx_map.p, stx, ntx * 4, hipMemcpyDeviceToDevice, s));
     // execution order of every row: (row, rank, tx); 32-bit composite keys
     // when row and rank fit, else 64-bit
-    if (n && row_bits + rank_bits <= 32) {
+    if (!n) return;
+    HIP_TRY(launch::fill_u64(ctx.conflicts.p, ctx.conflicts.n, 0, s));
+    HIP_TRY(launch::fill_u32(ctx.need.p, n, NEED_FREE, s));
+    HIP_TRY(launch::op_ids(ctx.ops.p, n, 0, ctx.sv0.p, s));
+    uint32_t* sop2;
+    if (row_bits + rank_bits <= 32) {
       HIP_TRY(launch::gtx_exec_keys32(ctx.rows_out.p, ctx.op_tx.p, ctx.rank.p, n, rank_bits, ctx.sk0.p, s));
-      HIP_TRY(launch::op_ids(ctx.ops.p, n, 0, ctx.sv0.p, s));
-      uint32_t *skey, *sop2;
+      uint32_t* skey;
       HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, row_bits + rank_bits,
                                      ctx.sort_tmp.p, &skey, &sop2, s));
-      uint32_t* srow2 = ctx.S.p;  // free once the ranks are made
-      HIP_TRY(launch::u32_key_high(skey, n, rank_bits, srow2, s));
-      ordered_need(srow2, sop2);
-      HIP_TRY(launch::fill_u64(ctx.conflicts.p, 1, 0, s));
-      HIP_TRY(launch::gtx_conflicts32(skey, ctx.flags.p, n, ctx.conflicts.p, s));
-    } else if (n) {
+      HIP_TRY(launch::seg_turns(skey, sop2, n, rank_bits, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows, 0u,
+                                nullptr, nullptr, 0u, ctx.conflicts.p, s));
+    } else {
       HIP_TRY(launch::gtx_exec_keys(ctx.rows_out.p, ctx.op_tx.p, ctx.rank.p, n, rank_bits, ctx.sk64a.p, s));
-      HIP_TRY(launch::op_ids(ctx.ops.p, n, 0, ctx.sv0.p, s));
       uint64_t* skey;
-      uint32_t* sop2;
       HIP_TRY(launch::radix_sort_u64(ctx.sk64a.p, ctx.sv0.p, ctx.sk64b.p, ctx.sv1.p, n, row_bits + rank_bits,
                                      ctx.sort_tmp.p, &skey, &sop2, s));
-      HIP_TRY(launch::u64_key_high(skey, n, rank_bits, ctx.sk0.p, s));
-      ordered_need(ctx.sk0.p, sop2);
-      HIP_TRY(launch::fill_u64(ctx.conflicts.p, 1, 0, s));
-      HIP_TRY(launch::gtx_conflicts(skey, ctx.flags.p, n, ctx.conflicts.p, s));
+      HIP_TRY(launch::seg_turns64(skey, sop2, n, rank_bits, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows,
+                                  ctx.conflicts.p, s));
     }
-  }
-  // need[] from accesses in execution order (group flags in ctx.flags, which
-  // the conflict count reads afterwards).  A row occupies the same positions
-  // in the (row, tx) and (row, rank, tx) orders, so ctx.SS (the row start of
-  // every position, made for the ranks) makes each turn relative to its row,
-  // and the counters start at zero: one dense fill instead of a random store
-  // per row.
-  void ordered_need(const uint32_t* srow, const uint32_t* sop) {
-    const uint64_t n = ctx.nops;
-    hipStream_t s = ctx.stream;
-    HIP_TRY(launch::access_group_flags(srow, sop, n, ctx.flags.p, s));
-    HIP_TRY(launch::inclusive_max_u32(ctx.flags.p, ctx.gstart.p, n, ctx.sort_tmp.p, s));
-    HIP_TRY(launch::access_need_rel(sop, ctx.gstart.p, ctx.SS.p, n, ctx.need.p, s));
-    HIP_TRY(launch::fill_u32(ctx.counters.p, ctx.counters.n, 0, s));
   }
   void Init(int, uint64_t) override {}
   // the persistent form runs every rank level in one launch: it needs no
@@ -1016,9 +978,12 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
       c->sv0.alloc(n);
       c->sk1.alloc(n);
       c->sv1.alloc(n);
-      c->flags.alloc(n);
-      c->gstart.alloc(n);
-      c->sort_tmp.alloc(std::max(launch::radix_sort_tmp_words(n), launch::scan_tmp_words(n)));
+      if (c->scheme == SCHEME_GACCO) {  // the serving form's admitted batches
+        c->flags.alloc(n);
+        c->gstart.alloc(n);
+      }
+      c->sort_tmp.alloc(
+          std::max({launch::radix_sort_tmp_words(n), launch::scan_tmp_words(n), launch::seg_tmp_words(n)}));
       if (c->scheme == SCHEME_GACCO && c->comb_min) {
         // at most nops / comb_min queues reach comb_min accesses
         c->comb_cap = std::min<uint64_t>(nops / c->comb_min + 1, 0x7fffffffull);
@@ -1027,14 +992,12 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
         c->comb_wv.alloc(nops);  // every op's write value, for the combiners
       }
       if (c->scheme == SCHEME_GPUTX) {
-        c->S.alloc(n);
-        c->SS.alloc(n);
         c->sk64a.alloc(n);
         c->sk64b.alloc(n);
         c->rank.alloc(ntx);
         c->tx_map.alloc(ntx);
         c->max_rank.alloc(1);
-        c->conflicts.alloc(1);
+        c->conflicts.alloc(16 * launch::CONFLICT_SLOTS);
       }
     }
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1250,7 +1213,11 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
     if (m.error_flags) clear_cc_state(*c);
     if (c->scheme == SCHEME_GPUTX) {
       st.ranks = c->nranks;
-      if (c->nops) HIP_TRY(hipMemcpy(&st.same_rank_conflicts, c->conflicts.p, 8, hipMemcpyDeviceToHost));
+      if (c->nops) {
+        uint64_t slot[16 * launch::CONFLICT_SLOTS];
+        HIP_TRY(hipMemcpy(slot, c->conflicts.p, sizeof slot, hipMemcpyDeviceToHost));
+        for (uint32_t i = 0; i < launch::CONFLICT_SLOTS; ++i) st.same_rank_conflicts += slot[16 * i];
+      }
     }
     if (form == FORM_PERSIST) st.combined = c->host->Combined();
     if (defer && c->ntx) {

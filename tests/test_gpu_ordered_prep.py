@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import gpu_cc_tb_amd as g
+import oracle_lib as orc
 
 SHORT_MAX = 1 << 20  # pairs up to which the sort uses its short tile (1,024)
 
@@ -20,3 +21,62 @@ def test_sort_tile_sizes(n, dtype, bits):
     k, v, _ = g.sort_pairs(keys, vals, key_bits=bits)
     order = np.argsort(keys & dtype((1 << bits) - 1), kind="stable")
     assert np.array_equal(v, order.astype(np.uint32)) and np.array_equal(k, keys[order])
+
+
+def _one_row_stream(ntx, writes, rows, seed):
+    """ntx transactions of 2 ops: row 0, read or (at the given transactions)
+    written, and a row of their own, so one queue runs through the sorted
+    accesses and every other row is met once."""
+    rng = np.random.default_rng(seed)
+    keys = np.zeros((ntx, 2), dtype=np.uint64)
+    keys[:, 1] = 1 + rng.permutation(rows - 1)[:ntx]
+    wr = np.zeros((ntx, 2), dtype=np.uint64)
+    wr[writes, 0] = 1
+    wr[:, 1] = rng.integers(0, 2, ntx)
+    ops = g.make_ops(keys.reshape(-1), rng.integers(0, 10, 2 * ntx), wr.reshape(-1))
+    return g.Ops(ops, np.arange(ntx + 1, dtype=np.uint64) * np.uint64(2))
+
+
+TURN_TILE = 2048  # accesses per tile of the turn kernels; carries look back 64 tiles a step
+TURN_CASES = {
+    # name: (ntx, transactions that write row 0)
+    "no_writes": (TURN_TILE, []),
+    "tile_edges": (2 * TURN_TILE + 1, [TURN_TILE - 1, TURN_TILE, 2 * TURN_TILE]),
+    "first_and_last": (TURN_TILE + 7, [0, TURN_TILE + 6]),
+    "past_64_tiles": (66 * TURN_TILE + 5, [0, 3, 66 * TURN_TILE + 1]),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", list(TURN_CASES))
+@pytest.mark.parametrize("scheme", ["gacco", "gputx"])
+@pytest.mark.parametrize("form", ["plain", "persistent"])
+def test_turns_of_a_long_queue(scheme, case, form, monkeypatch):
+    """One row's queue across tile edges and beyond one look-back step, turn
+    by turn (no combiner): the serial replay in the reported order."""
+    monkeypatch.setenv("GCCTB_COMBINE_MIN", "0")
+    ntx, writes = TURN_CASES[case]
+    rows = ntx + 1
+    w = _one_row_stream(ntx, writes, rows, ntx)
+    print(f"[turns] scheme={scheme} case={case} form={form}", flush=True)
+    with g.Context(scheme, rows=rows, warp_density=1, block_size=8, batch_size=1 << 20) as ctx:
+        ctx.seed_table()
+        ctx.load_ops(w)
+        st = ctx.run(form)
+        res = ctx.fetch()
+        rank = ctx.fetch_ranks()[0] if scheme == "gputx" else None
+    assert st["committed"] == ntx and st["error_flags"] == 0
+    init = orc.seed_table(g.SEED, rows, 10)
+    exp_t, exp_r, ties = orc.replay(rows, 10, g.SEED, init, w.ops, w.tx_off, res["order"])
+    isr = ~g.op_is_write(w.ops)
+    assert ties == 0 and np.array_equal(res["table"], exp_t) and np.array_equal(res["reads"][isr], exp_r[isr])
+    if scheme == "gacco":
+        t2, r2 = orc.replay_txid(rows, 10, g.SEED, init, w.ops, w.tx_off)
+        assert np.array_equal(res["table"], t2) and np.array_equal(res["reads"][isr], r2[isr])
+    else:
+        # group starts of row 0's queue up to each transaction
+        wr = np.zeros(ntx, dtype=bool)
+        wr[writes] = True
+        start = np.zeros(ntx, dtype=np.int64)
+        start[1:] = wr[1:] | wr[:-1]
+        assert np.array_equal(rank, np.cumsum(start).astype(np.uint32))
