@@ -100,6 +100,7 @@ struct TxCtx {
   uint32_t nops = 0;
   uint32_t ph = PH_START;
   uint32_t attempts = 0;   // aborted attempts
+  uint32_t backoff = 0;    // exponent of the retry delay
   bool live = false;
   bool done = true;
   uint64_t ts = 0;         // attempt timestamp (T/O, MVCC) or commit timestamp
@@ -258,12 +259,25 @@ __device__ __forceinline__ void ev_commit(const TxCtx<G>& c, const ExecArgs& a) 
 // transactions of one wave that restart in the same round collide again in the
 // same order; an immediate retry (benchmark/ycsb.cu:99-104) can then repeat
 // forever.  The restart is delayed by a random number of units in
-// [0, 2^min(attempts, backoff_exp)) (backoff_exp 10 unless configured), where
+// [0, 2^min(e, backoff_exp)) (e: the aborts so far; backoff_exp 10 unless configured), where
 // a unit is the duration of the failed attempt
 // (at least backoff_ticks, at most BACKOFF_UNIT_MAX): retries spread over
 // rounds, not just over ticks.  The cap matters for attempts that waited
 // (wait-die, T/O reads of uncommitted rows): their duration includes the
 // wait, and 1024 such units would idle a transaction for seconds.
+//
+// A young plain launch (until 300 us + 4 ns per transaction after its
+// counters were reset) spans at most 4 units and does not raise e: the
+// conflicts of a low-contention batch are over within that time, and delays
+// that had already grown to 8 and 16 units of the first, crowded attempt were
+// half of such a launch (65,536 transactions of 16 ops on 1,048,576 rows,
+// theta 0.1, read ratio 0.9, 8 lanes each: 2PL 800 -> 350 us, T/O 290 -> 215,
+// MVCC 420 -> 350, Silo 520 -> 330, TicToc 510 -> 375; 6,007 transactions of 4
+// to 32 ops on 131,071 rows, read ratio 0.5: 390-910 -> 140-290 us).  A
+// contended launch runs for tens of ms, so the aborts of its first 300 us do
+// not count (theta 0.99, read ratio 0.5 and 0.9: within 2% either way).  By
+// the age of the transaction instead, the waves that start late would each
+// bring a burst of retries of their own: 2PL 1.5x slower at theta 0.99.
 // Urgent state (persistent form).  A transaction that has aborted
 // ExecArgs::urgent_attempts times (256 by default: a safety net, far beyond
 // the abort counts of a healthy run) adds itself to the urgent count of every
@@ -290,7 +304,8 @@ __device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, ui
   uint64_t unit = dur > a.backoff_ticks ? dur : a.backoff_ticks;
   if (unit > BACKOFF_UNIT_MAX) unit = BACKOFF_UNIT_MAX;
   const uint64_t h = hash3(a.seed ^ TAG_BACKOFF, c.tx, c.attempts);
-  const uint32_t span = 1u << (c.attempts < a.backoff_exp ? c.attempts : a.backoff_exp);
+  if (c.backoff < 2 || !a.young_ticks || t - ld(a.ctrs + CTR_T0) >= a.young_ticks) c.backoff++;
+  const uint32_t span = 1u << (c.backoff < a.backoff_exp ? c.backoff : a.backoff_exp);
   c.t_resume = t + (h % span) * unit;
   c.ph = PH_START;
 }
@@ -1402,6 +1417,7 @@ __device__ __forceinline__ void load_tx(TxCtx<G>& c, const ExecArgs& a, uint64_t
   c.done = !c.live;
   c.ph = PH_START;
   c.attempts = 0;
+  c.backoff = 0;
   c.t_resume = 0;
   c.t_start = now;
   c.nops = 0;

@@ -244,6 +244,7 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
       a.batch_id = (uint32_t)b;
       a.slot_lo = st0;
       a.slot_hi = st0 + n;
+      a.young_ticks = young_ticks(n);
       NA_TRY(launch::batch_begin(ctrs, s));
       NA_TRY(launch_exec(sch, G, a, n, threads, s));
       if (sch != SCHEME_TPL_NW && sch != SCHEME_TPL_WD)

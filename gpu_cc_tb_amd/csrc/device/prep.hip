@@ -1080,6 +1080,7 @@ __global__ void k_batch_begin(uint64_t* ctrs) {
   if (threadIdx.x == 0) {
     dev::st(ctrs + CTR_TICKET, 0);  // commit tickets
     dev::st(ctrs + CTR_POOL, 0);    // MVCC pool bump pointer
+    dev::st(ctrs + CTR_T0, wall_clock64());
     // timestamp allocators restart at 1 (timestamp.cuh:76-80)
     for (int s = 0; s < TS_SHARDS; ++s) dev::st(ctrs + CTR_TS0 + 16 * s, 1);
   }

@@ -205,6 +205,7 @@ constexpr int CTR_GATE0 = CTR_SLOT + 16;
 constexpr int GATE_SHARDS = 16;
 constexpr int CTR_ADMIT0 = CTR_GATE0 + 16 * GATE_SHARDS;
 constexpr int CTR_EVENT = CTR_ADMIT0 + 16 * GATE_SHARDS;  // event-log stamps (a whole run)
+constexpr int CTR_T0 = CTR_EVENT + 8;  // wall clock at the batch's counter reset, before its launch
 constexpr int CTR_WORDS = CTR_EVENT + 16;
 constexpr uint32_t ADMIT_CLOSED = 1u << 31;
 // Waves add their totals into one of METRIC_SLOTS 128-byte slots (by block
@@ -324,12 +325,17 @@ struct ExecArgs {
   uint32_t persist;        // 1 in persistent launches (slots from CTR_SLOT, gates, urgent state)
   uint32_t urgent_attempts; // persistent form: aborts that make a transaction urgent (0 = never)
   uint32_t backoff_exp;     // retry delay spans at most 2^backoff_exp units
+  uint32_t young_ticks;     // plain form: until this long after CTR_T0 it spans at most 4 units (young_ticks())
   uint32_t poll_ticks;      // ordered schemes: expected ticks per handoff on a row (rest pacing)
   uint64_t* tcommit;       // optional, per tx: wall-clock tick of its commit (serving form)
   uint64_t* ev_op;         // event-log kernels: per op, the stamp of its access (0 = none)
   uint64_t* ev_commit;     // event-log kernels: per tx, the stamp of its commit (0 = none)
   const uint32_t* op_param; // TPC-C kernels: per op, the update's parameter
 };
+
+// How long a plain launch over n transactions counts as young (10 ns ticks):
+// 300 us and 4 ns per transaction, about twice what it takes without conflicts.
+constexpr uint32_t young_ticks(uint64_t n) { return 30000u + (uint32_t)(n < (1ull << 31) ? n * 2 / 5 : 0); }
 
 // ---------------------------------------------------------------------------
 // TPC-C (benchmark/tpcc.cu, include/tpcc.cuh): payment and new_order over the

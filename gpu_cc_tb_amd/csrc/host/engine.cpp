@@ -308,6 +308,7 @@ class SchemeHost {
     a.watchdog_ticks = ctx.watchdog_ticks;
     a.urgent_attempts = ctx.urgent_attempts;
     a.backoff_exp = ctx.backoff_exp;
+    a.young_ticks = young_ticks(slot_hi - slot_lo);
     a.poll_ticks = ctx.poll_ticks;
     a.dbg = ctx.dbg.p;
     a.persist_groups = ctx.cfg.persist_window;
