@@ -375,6 +375,7 @@ template <bool WAIT_DIE>
 struct TwoPL {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
   static constexpr bool kBulkRefill = true;
+  static constexpr bool kSlotStash = false;
   // lock_shared (twopl.cuh:233-267), continuing from an observed word `cur`
   // (the round's first CAS guessed a free word and returned it).
   static __device__ StepResult lock_shared(uint64_t* w, uint64_t self, uint64_t cur) {
@@ -614,6 +615,7 @@ __device__ __forceinline__ void ts_head_reads(const TxCtx<G>& c, const ExecArgs&
 struct TimestampOrdering {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
   static constexpr bool kBulkRefill = true;
+  static constexpr bool kSlotStash = false;
   static __device__ StepResult write_mark(uint64_t* w, uint64_t ts, uint64_t& prev, uint64_t& seen) {
     uint64_t cur = w_ld(w);
 #pragma unroll 1
@@ -737,6 +739,7 @@ __device__ __forceinline__ uint64_t mvcc_stride(const ExecArgs& a) { return kRow
 struct Mvcc {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
   static constexpr bool kBulkRefill = true;
+  static constexpr bool kSlotStash = false;
   static __device__ StepResult read(const ExecArgs& a, uint32_t row, uint32_t col, uint64_t ts,
                                     uint64_t& val) {
     uint64_t* w = cc_word(a, row);
@@ -1015,6 +1018,7 @@ __device__ __forceinline__ void occ_lock(const TxCtx<G>& c, const ExecArgs& a, u
 struct Silo {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
   static constexpr bool kBulkRefill = true;
+  static constexpr bool kSlotStash = false;
   // Read: the word, then the cell (silo.cuh:223-259 loads the word a second
   // time after the data).  The commit validation re-reads every read word
   // and aborts unless it still holds the TID seen here, unlocked; a writer
@@ -1158,6 +1162,7 @@ struct Silo {
 struct Tictoc {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
   static constexpr bool kBulkRefill = true;
+  static constexpr bool kSlotStash = false;
   template <int G>
   static __device__ void round(TxCtx<G>& c, const ExecArgs& a) {
     constexpr int K = TxCtx<G>::K;
@@ -1392,6 +1397,7 @@ struct Ordered {
   // Refill at once: a done group that waited for its wave would idle behind
   // groups queued on hot rows (measured: 29% slower on the batched stream).
   static constexpr bool kBulkRefill = false;
+  static constexpr bool kSlotStash = true;
   static constexpr uint64_t POLL_REST_MAX = 12800;     // 128 us
 };
 
@@ -1534,12 +1540,24 @@ __device__ void watchdog_stop(const TxCtx<G>& c, const ExecArgs& a) {
 
 // ---------------------------------------------------------------------------
 // Persistent form.  Groups take stream slots, in stream order, from one
-// wave-aggregated counter as soon as their transaction commits, so a group
-// held up by a slow transaction never holds back later slots, and the lowest
-// unfinished slot always belongs to a running group (which the ordered
-// schemes need: they wait on lower slots only).  The grid holds the
-// admission window: at most that many groups, so at most that many
-// transactions in flight.
+// counter as soon as their transaction commits, so a group held up by a slow
+// transaction never holds back later slots, and the lowest unfinished slot
+// always belongs to a running group or to the next one of its block that
+// frees up (which the ordered schemes need: they wait on lower slots only).
+// The grid holds the admission window: at most that many groups, so at most
+// that many transactions in flight.
+//
+// One address serves 83 M atomics/s, and the ordered schemes refill a group
+// at a time, so their launch took the draws' 12 ns each (GaccO, 1,048,576
+// transactions of 16 ops, theta 0.1: 0.69 / 0.96 / 1.77 / 3.34 ms at 2 / 4 / 8
+// / 16 lanes per transaction).  Their blocks therefore draw as many slots as
+// they have groups at once and hand them out in order from LDS (SlotStash;
+// 0.73 / 0.67 / 0.66 / 0.95 ms with 256 threads); within one grid's worth of
+// slots of the end they draw no more than they start.  A block's running
+// slots are all below its stashed ones, so the stash never holds the lowest
+// unfinished slot while its groups wait.  The other schemes refill a wave at
+// once and are not bound by the draws; there slots held back move
+// transactions against each other for nothing (Silo: same time).
 //
 // Open form (a.open, the serving loop): the launch starts before its
 // transactions have arrived.  The host admits them batch by batch while the
@@ -1579,11 +1597,65 @@ __device__ __forceinline__ void scheme_round(TxCtx<G>& c, const ExecArgs& a) {
   }
 }
 
+// Slots a block has drawn and not started, [next, end), under a lock that a
+// wave holds for one draw at most (its holder never waits for another wave).
+struct SlotStash {
+  uint32_t lock;
+  uint64_t next, end;
+};
+// A slot for every lane with `take` (the wave's first such lane draws for
+// all; every lane of the wave calls it).
+__device__ __forceinline__ uint64_t stash_take(SlotStash& s, uint64_t* ctr, bool take, uint32_t chunk, uint64_t tail) {
+  const uint64_t m = ballot(take);
+  const int first = __ffsll((unsigned long long)m) - 1;
+  const uint32_t want = (uint32_t)__popcll(m);
+  uint64_t lo = 0, hi = 0;
+  uint32_t had = 0;  // slots from the stash; the others follow hi
+  if ((int)lane_id() == first) {
+    uint32_t open_lock = 0;
+    while (!__hip_atomic_compare_exchange_strong(&s.lock, &open_lock, 1u, __ATOMIC_ACQUIRE, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP)) {
+      open_lock = 0;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    lo = s.next;
+    const uint64_t left = s.end - lo;
+    had = left < want ? (uint32_t)left : want;
+    s.next = lo + had;
+    if (had < want) {
+      const uint32_t rest = want - had;
+      const uint32_t n = s.end < tail && chunk > rest ? chunk : rest;
+      hi = fetch_add(ctr, n);
+      s.next = hi + rest;
+      s.end = hi + n;
+    }
+    __hip_atomic_store(&s.lock, 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  lo = shfl64(lo, first);
+  hi = shfl64(hi, first);
+  had = shfl32(had, first);
+  const uint32_t r = (uint32_t)__popcll(m & lanemask_lt());
+  return r < had ? lo + r : hi + (r - had);
+}
+
 template <class S, int G>
 __device__ void run_persistent(TxCtx<G>& c, const ExecArgs& a) {
+  __shared__ SlotStash stash;
+  if constexpr (S::kSlotStash) {
+    if (threadIdx.x == 0) {
+      stash.lock = 0;
+      stash.next = stash.end = 0;
+    }
+    __syncthreads();
+  }
+  const bool stashing = S::kSlotStash && a.open == 0;
+  const uint32_t chunk = blockDim.x / G;  // one slot per group of the block
   const bool leader = (lane_id() & (G - 1)) == 0;
   const uint64_t nslots = a.slot_hi - a.slot_lo;
   const bool open = a.open != 0;
+  // draws of whole chunks stop one grid's worth of slots before the end
+  const uint64_t all_groups = (uint64_t)chunk * gridDim.x;
+  const uint64_t tail = nslots > all_groups ? nslots - all_groups : 0;
   uint64_t* slot_ctr = a.ctrs + CTR_SLOT;
   const uint32_t shard = blockIdx.x & (GATE_SHARDS - 1);
   const uint64_t* gate = a.ctrs + CTR_GATE0 + 16 * shard;
@@ -1633,10 +1705,12 @@ __device__ void run_persistent(TxCtx<G>& c, const ExecArgs& a) {
           }
         }
       }
-      if (handed_out && need && held == NO_SLOT) finished = true;
+      if (!stashing && handed_out && need && held == NO_SLOT) finished = true;
       const bool take = need && !finished && urgent == 0 && held == NO_SLOT;
       if (ballot(take) != 0) {
-        const uint64_t got = group_bcast64<G>(wave_fetch_inc(slot_ctr, take && leader));
+        uint64_t got = stashing ? stash_take(stash, slot_ctr, take && leader, chunk, tail)
+                                : wave_fetch_inc(slot_ctr, take && leader);
+        got = group_bcast64<G>(got);
         if (take) {
           if (got < nslots) {
             held = got;
@@ -1674,7 +1748,7 @@ __device__ void run_persistent(TxCtx<G>& c, const ExecArgs& a) {
         next_stall = now + STALL_TICKS;
         const uint64_t cur = ld(slot_ctr);
         if (cur >= nslots) {
-          if (parked) finished = true;
+          if (parked) finished = true;  // (an ordered scheme, the only one to stash, never parks: it never aborts)
         } else if (cur != seen_slot) {
           seen_slot = cur;
           seen_at = now;

@@ -80,3 +80,29 @@ def test_turns_of_a_long_queue(scheme, case, form, monkeypatch):
         start = np.zeros(ntx, dtype=np.int64)
         start[1:] = wr[1:] | wr[:-1]
         assert np.array_equal(rank, np.cumsum(start).astype(np.uint32))
+
+
+# (warp_density, block_size, window, ntx): blocks of 64, 64, 1 and 16 groups;
+# streams of one slot past a block, many chunks, and none to stash
+STASH_CASES = [(2, 8, 64, 65), (2, 8, 128, 2001), (5, 1, 4, 33), (4, 8, 32, 32), (4, 8, 32, 515)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wd,bs,window,ntx", STASH_CASES)
+@pytest.mark.parametrize("scheme", ["gacco", "gputx"])
+def test_slot_stash(scheme, wd, bs, window, ntx):
+    """Blocks that draw their slots in chunks run every transaction once, in
+    an order that the waits on lower slots allow, down to the stream's end."""
+    rows = 256
+    w = g.generate(rows, ntx, theta=0.8, read_ratio=0.5, len_min=1, len_max=8)
+    print(f"[stash] scheme={scheme} wd={wd} bs={bs} window={window} ntx={ntx}", flush=True)
+    with g.Context(scheme, rows=rows, warp_density=wd, block_size=bs, batch_size=1 << 20,
+                   persist_window=window) as ctx:
+        ctx.seed_table()
+        ctx.load_ops(w)
+        st = ctx.run("persistent")
+        res = ctx.fetch()
+    assert st["committed"] == ntx and st["error_flags"] == 0
+    exp_t, exp_r, ties = orc.replay(rows, 10, g.SEED, orc.seed_table(g.SEED, rows, 10), w.ops, w.tx_off, res["order"])
+    isr = ~g.op_is_write(w.ops)
+    assert ties == 0 and np.array_equal(res["table"], exp_t) and np.array_equal(res["reads"][isr], exp_r[isr])
