@@ -74,16 +74,39 @@ hipError_t access_group_flags(const uint32_t* srow, const uint32_t* sop, uint64_
 // From accesses sorted by (row, order): key[p] >> rb is the row, val[p] an
 // op id (op_ids).  need[op] (NEED_*) of every access that waits for another or
 // is waited for (the caller fills need with NEED_FREE first), counters[row] =
-// 0 for the rows where that happens.  With comb_min > 0 every row queue of at
-// least comb_min accesses is listed as (first position, length) in segs
-// (seg_ctr counts them; at most seg_cap are kept).  conflicts (may be null):
-// neighbours with equal keys where either writes, added to CONFLICT_SLOTS
-// counters 16 words apart.  tmp holds seg_tmp_words(n) u32.
+// 0 for the rows where that happens.  With comb.min > 0 every row queue of at
+// least comb.min accesses is listed for gacco_combine.  conflicts (may be
+// null): neighbours with equal keys where either writes, added to
+// CONFLICT_SLOTS counters 16 words apart.  tmp holds seg_tmp_words(n) u32.
 constexpr uint32_t CONFLICT_SLOTS = 16;
 uint64_t seg_tmp_words(uint64_t n);
+// GaccO's row combiners: what they read, and the lists that seg_turns files
+// queues in (ctr: COMB_WORDS u32, zero before).  chunks[i]: {first position,
+// length, its summary + 1 (0: the queue's only chunk), 0}; multi[i], queues
+// of several chunks: {first position, first summary, chunks, 0}.
+struct CombArgs {
+  uint32_t min;          // shortest queue to combine (0: none)
+  uint32_t chunk_cap, multi_cap;
+  uint4* chunks;
+  uint4* multi;
+  uint64_t* sums;        // cols values and a mask of the columns written, per chunk
+  uint32_t* ctr;
+  const uint64_t* ops;
+  const uint32_t* op_tx;
+  const uint64_t* tx_off;
+  uint64_t* cells;
+  uint32_t cols;
+  uint64_t seed;
+  uint64_t* reads;
+  uint32_t* need;
+  unsigned long long* combined;
+};
+constexpr uint32_t COMB_CHUNKS = 0, COMB_SUMS = 1, COMB_MULTI = 2, COMB_WORDS = 4;
+uint64_t comb_chunk_cap(uint64_t nops, uint32_t min);
+uint64_t comb_multi_cap(uint64_t nops);
+uint64_t comb_sum_words(uint64_t nops, uint32_t cols);
 hipError_t seg_turns(const uint32_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
-                     uint32_t* counters, uint64_t nrows, uint32_t comb_min, uint2* segs, uint32_t* seg_ctr,
-                     uint32_t seg_cap, uint64_t* conflicts, hipStream_t s);
+                     uint32_t* counters, uint64_t nrows, const CombArgs& comb, uint64_t* conflicts, hipStream_t s);
 hipError_t seg_turns64(const uint64_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
                        uint32_t* counters, uint64_t nrows, uint64_t* conflicts, hipStream_t s);
 // GPUTx one-pass rank (src/gputx.cu:5-27) from accesses sorted by (row, tx),
@@ -94,12 +117,8 @@ hipError_t seg_ranks(const uint32_t* row, const uint32_t* val, uint64_t n, uint3
                      uint32_t* rank, uint32_t* max_rank, hipStream_t s);
 // GaccO, persistent form: run each listed row queue in order on the row's
 // cells (cols <= 64), store its reads' results, mark its ops need = NEED_DONE
-// and add the ops run to *combined.  wvals (nops u64) receives every op's
-// write value first, when any queue is listed.
-hipError_t gacco_combine(const uint2* segs, const uint32_t* seg_ctr, uint32_t seg_cap, const uint32_t* srow,
-                         const uint32_t* sop, const uint64_t* ops, const uint32_t* op_tx, const uint64_t* tx_off,
-                         uint64_t nops, uint64_t* cells, uint32_t cols, uint64_t seed, uint64_t* wvals, uint64_t* reads,
-                         uint32_t* need, uint64_t* combined, hipStream_t s);
+// and add the ops run to *combined.  srow, sop: the sorted accesses.
+hipError_t gacco_combine(const CombArgs& c, const uint32_t* srow, const uint32_t* sop, hipStream_t s);
 // Open form, one admitted batch sorted by (row, op) with group starts gstart
 // and row starts rstart: need[op] = base[row] + gstart[p] - rstart[p]; then
 // row_base_add adds the batch's accesses of each row to base[row].

@@ -779,15 +779,41 @@ __global__ __launch_bounds__(BT) void k_seg_tiles(const KT* key, const uint32_t*
 
 // need[op] (op = val & OPID_MASK) of every access that waits or is waited
 // for; the others keep NEED_FREE.  The counter of a row where that happens is
-// set to 0 at the row's first access.  comb_min > 0: every row queue of at
-// least comb_min accesses is listed as (first position, length) in segs.
+// set to 0 at the row's first access.  comb.min > 0: every row queue of at
+// least comb.min accesses is listed for its combiner (comb_list).
 // conflicts (GPUTx): same-row neighbours of equal key (row and rank) where
 // either writes, added to CONFLICT_SLOTS counters on lines of their own.
+// The row queues of a thread's accesses that end in it, filed block by block:
+// one add per counter and block (a queue per atomic would pile onto them).
+__device__ __forceinline__ uint32_t block_file(uint32_t n, uint32_t* ctr) {  // n places for this thread
+  __shared__ uint32_t wsum[BT / 64], base;
+  const uint32_t lane = dev::lane_id(), wave = threadIdx.x / 64;
+  uint32_t x = n;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t o = (uint32_t)__shfl_up((int)x, d, 64);
+    if (lane >= (uint32_t)d) x += o;
+  }
+  __syncthreads();  // the call before has read wsum and base
+  if (lane == 63) wsum[wave] = x;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < BT / 64; ++w) {
+    before += w < wave ? wsum[w] : 0u;
+    all += wsum[w];
+  }
+  if (threadIdx.x == 0) base = all ? atomicAdd(ctr, all) : 0u;
+  __syncthreads();
+  return base + before + x - n;
+}
+constexpr uint32_t CB_BT = 256;  // accesses per combiner chunk, one per thread
+
 template <class KT>
 __global__ __launch_bounds__(BT) void k_seg_turns(const KT* key, const uint32_t* val, uint64_t n, int rb,
                                                   const uint4* summ, uint32_t* need, uint32_t* counters,
-                                                  uint64_t nrows, uint32_t comb_min, uint2* segs, uint32_t* seg_ctr,
-                                                  uint32_t seg_cap, unsigned long long* conflicts) {
+                                                  uint64_t nrows, launch::CombArgs comb,
+                                                  unsigned long long* conflicts) {
   __shared__ uint32_t wnext[BT / 64];
   SegTile<KT> t;
   t.load(key, val, n);
@@ -843,6 +869,7 @@ __global__ __launch_bounds__(BT) void k_seg_turns(const KT* key, const uint32_t*
     }
   }
   uint64_t same = 0;
+  uint32_t qlen[TT_ITEMS] = {};  // length of the row queue that ends at access i
 #pragma unroll
   for (int i = 0; i < TT_ITEMS; ++i) {
     if ((uint32_t)i >= t.cnt) break;
@@ -856,14 +883,41 @@ __global__ __launch_bounds__(BT) void k_seg_turns(const KT* key, const uint32_t*
     const bool followed = nx[i] == EV_GROUP;
     if (wait || followed) need[t.v[i] & OPID_MASK] = wait | (followed ? 0u : NEED_LAST);
     if (e == EV_ROW && followed) counters[row_slot((uint32_t)row, slot_shift(nrows))] = 0u;
-    if (comb_min) {
+    if (comb.min) {
       const uint64_t q = t.p0 + i + 1;
       const KT k1 = i + 1 < TT_ITEMS ? t.k[i + 1] : nk;
-      if (q == n || (k1 >> rb) != (t.k[i] >> rb)) {
-        const uint32_t len = p + 2 - at.row;
-        if (len >= comb_min) {
-          const uint32_t s = atomicAdd(seg_ctr, 1u);
-          if (s < seg_cap) segs[s] = make_uint2(at.row - 1, len);
+      if (q == n || (k1 >> rb) != (t.k[i] >> rb)) qlen[i] = p + 2 - at.row;
+    }
+  }
+  if (comb.min) {
+    // file the queues long enough: their chunks, and those of more than one
+    // chunk once more for the carry between their chunks
+    uint32_t nch = 0, nmc = 0, nms = 0;
+#pragma unroll
+    for (int i = 0; i < TT_ITEMS; ++i) {
+      if (qlen[i] < comb.min) qlen[i] = 0;
+      const uint32_t c = (qlen[i] + CB_BT - 1) / CB_BT;
+      nch += c;
+      nmc += c > 1 ? c : 0u;
+      nms += c > 1 ? 1u : 0u;
+    }
+    if (__syncthreads_or((int)nch)) {
+      uint32_t ci = block_file(nch, comb.ctr + launch::COMB_CHUNKS);
+      uint32_t si = block_file(nmc, comb.ctr + launch::COMB_SUMS);
+      uint32_t mi = block_file(nms, comb.ctr + launch::COMB_MULTI);
+#pragma unroll
+      for (int i = 0; i < TT_ITEMS; ++i) {
+        if (!qlen[i]) continue;
+        const uint32_t first = (uint32_t)(t.p0 + i) + 1u - qlen[i], c = (qlen[i] + CB_BT - 1) / CB_BT;
+        if (c > 1 && mi < comb.multi_cap) comb.multi[mi] = make_uint4(first, si, c, 0u);
+        for (uint32_t x = 0; x < c; ++x)
+          if (ci + x < comb.chunk_cap)
+            comb.chunks[ci + x] = make_uint4(first + x * CB_BT, x + 1 < c ? CB_BT : qlen[i] - x * CB_BT,
+                                             c > 1 ? si + x + 1u : 0u, 0u);
+        ci += c;
+        if (c > 1) {
+          si += c;
+          ++mi;
         }
       }
     }
@@ -904,109 +958,171 @@ __global__ __launch_bounds__(BT) void k_seg_ranks(const uint32_t* key, const uin
 
 // ---------------------------------------------------------------------------
 // GaccO, persistent form: a row whose access queue (its accesses in
-// transaction-id order) holds at least comb_min accesses is run by one
-// workgroup, the row's combiner, before the launch.  The combiner keeps the
-// row's cells in LDS and applies the queue in order, so every read returns
-// the value of the last write to its column before it in transaction-id
-// order, or the cell's value before the stream, and the row ends with the
-// last write of each column: what the queue's turns produce one handoff at a
-// time.  Its ops are marked done (need = NEED_DONE) and the launch skips
-// them; no other op touches the row.  Column mode, cols <= 64.
+// transaction-id order) holds at least comb.min accesses is run in queue
+// order by the row's combiner before the launch.  Every read returns the
+// value of the last write to its column before it in transaction-id order,
+// or the cell's value before the stream, and the row ends with the last write
+// of each column: what the queue's turns produce one handoff at a time.  Its
+// ops are marked done (need = NEED_DONE) and the launch skips them; no other
+// op touches the row.  Column mode, cols <= 64.
 //
-// Steps of CB_BT queue entries, one per thread, all 16 waves at once:
-//  1. every thread gathers its entry (column, write flag, written value);
-//  2. each wave resolves its own 64 entries: per column written among them
-//     (one ballot each), a read finds the last write below it, and the last
-//     write of each column is kept as the wave's summary;
-//  3. lane c of wave 0 carries column c through the 16 summaries in order,
-//     which gives every wave the value each column holds at its start;
-//  4. the reads with no write below them in their wave take that value, and
-//     every thread stores its read's result and the done mark.
-// Written values come precomputed per op (k_gacco_wvals), so the gather is
-// two dependent loads deep.
-constexpr int CB_BT = 1024;
+// The queue is cut into chunks of CB_BT accesses that workgroups resolve
+// independently, as a scan does:
+//  1. k_comb_sums: the last write of each column in a chunk (queues of more
+//     than one chunk only);
+//  2. k_comb_carry, one workgroup per such queue: each column's value at the
+//     start of every chunk, and the row's final cells;
+//  3. k_comb_resolve: a chunk's reads.  Each wave resolves its own 64
+//     accesses: per column written among them (one ballot each), a read
+//     finds the last write below it, and the last write of each column is
+//     the wave's summary; lane c of wave 0 carries column c through the
+//     summaries from the chunk's start; the reads with no write below them
+//     in their wave take that value.
+// One workgroup per queue, chunk after chunk, took 3.4 us per 1,024 accesses,
+// and the hottest row's queue was the whole time: 262,144 transactions of 4 to
+// 32 ops at theta 0.99 (270,000 accesses to row 0) 944 us, now 178 us (26 + 36
+// + 116; bound: the resolve pass's random op loads and result stores).
+// ---------------------------------------------------------------------------
 constexpr int CB_WAVES = CB_BT / 64;
-// wv[op] = the value op would write, for every op (the combiners read those
-// of their writes); nothing to do when no queue is listed
-__global__ void k_gacco_wvals(const uint32_t* op_tx, const uint64_t* tx_off, uint64_t nops, uint64_t seed,
-                              const uint32_t* seg_ctr, uint64_t* wv) {
-  if (*seg_ctr == 0) return;  // the same for every thread of the grid
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nops;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t t = op_tx[i];
-    wv[i] = write_value(seed, t, (uint32_t)(i - tx_off[t]));
+// the value that op writes
+__device__ __forceinline__ uint64_t comb_value(const launch::CombArgs& c, uint32_t opid) {
+  const uint32_t tx = c.op_tx[opid];
+  return write_value(c.seed, tx, (uint32_t)(opid - c.tx_off[tx]));
+}
+
+__global__ __launch_bounds__(CB_BT) void k_comb_sums(launch::CombArgs c, const uint32_t* sop) {
+  __shared__ int last[64];
+  const uint32_t nc = min(c.ctr[launch::COMB_CHUNKS], c.chunk_cap), tid = threadIdx.x;
+  for (uint32_t x = blockIdx.x; x < nc; x += gridDim.x) {
+    const uint4 ch = c.chunks[x];
+    if (ch.z == 0) continue;  // the queue's only chunk
+    if (tid < 64) last[tid] = -1;
+    __syncthreads();
+    if (tid < ch.y) {
+      const uint32_t so = sop[ch.x + tid];
+      if (so & OPID_WRITE) atomicMax(&last[op_col(c.ops[so & OPID_MASK])], (int)tid);
+    }
+    __syncthreads();
+    if (tid < 64) {
+      const int l = tid < c.cols ? last[tid] : -1;
+      uint64_t* sum = c.sums + (uint64_t)(ch.z - 1) * (c.cols + 1);
+      const uint64_t written = dev::ballot(l >= 0);
+      if (tid == 0) sum[c.cols] = written;
+      if (l >= 0) sum[tid] = comb_value(c, sop[ch.x + (uint32_t)l] & OPID_MASK);
+    }
+    __syncthreads();  // last is rewritten by the next chunk
   }
 }
-__global__ __launch_bounds__(CB_BT) void k_gacco_combine(const uint2* segs, const uint32_t* seg_ctr, uint32_t seg_cap,
-                                                         const uint32_t* srow, const uint32_t* sop, const uint64_t* ops,
-                                                         const uint64_t* wvals, uint64_t* cells, uint32_t cols,
-                                                         uint64_t* reads, uint32_t* need, uint64_t* combined) {
-  __shared__ uint64_t val[CB_BT];            // written values, by entry
-  __shared__ uint64_t sum[CB_WAVES][64];     // per wave: the last value it wrote to each column
-  __shared__ uint64_t cin[CB_WAVES][64];     // per wave: each column's value at its first entry
-  __shared__ uint64_t wmask[CB_WAVES];       // per wave: the columns it wrote
-  __shared__ uint64_t cell[64];              // the row between steps
-  const uint32_t nseg = min(*seg_ctr, seg_cap);
+
+// Wave w takes the w-th part of the queue's chunks: the last write of each
+// column in it, then (with the parts before it known) every chunk's carry-in
+// in place of its summary.  Lane c holds column c.
+constexpr int CC_WAVES = 16;
+__global__ __launch_bounds__(CC_WAVES * 64) void k_comb_carry(launch::CombArgs c, const uint32_t* srow) {
+  __shared__ uint64_t part[CC_WAVES][64];
+  __shared__ uint64_t mask[CC_WAVES];
+  const uint32_t nm = min(c.ctr[launch::COMB_MULTI], c.multi_cap);
+  const uint32_t w = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const bool col = lane < c.cols;
+  for (uint32_t x = blockIdx.x; x < nm; x += gridDim.x) {
+    const uint4 q = c.multi[x];
+    uint64_t* rc = c.cells + (uint64_t)srow[q.x] * c.cols;
+    const uint32_t per = (q.z + CC_WAVES - 1) / CC_WAVES;
+    const uint32_t k0 = min(w * per, q.z), k1 = min(k0 + per, q.z);
+    uint64_t* sum = c.sums + (uint64_t)q.y * (c.cols + 1);
+    uint64_t cur = 0, seen = 0;
+#pragma unroll 4
+    for (uint32_t k = k0; k < k1; ++k) {
+      const uint64_t m = sum[(uint64_t)k * (c.cols + 1) + c.cols];
+      const uint64_t v = col ? sum[(uint64_t)k * (c.cols + 1) + lane] : 0;
+      if ((m >> lane) & 1ull) cur = v;
+      seen |= m;
+    }
+    part[w][lane] = cur;
+    if (lane == 0) mask[w] = seen;
+    __syncthreads();
+    cur = col ? rc[lane] : 0;
+    for (uint32_t y = 0; y < w; ++y)
+      if ((mask[y] >> lane) & 1ull) cur = part[y][lane];
+    if (w == CC_WAVES - 1 && col) {
+      const uint64_t end = (mask[w] >> lane) & 1ull ? part[w][lane] : cur;
+      part[w][lane] = end;  // the row's final cells, stored once every wave has read it
+    }
+#pragma unroll 4
+    for (uint32_t k = k0; k < k1; ++k) {
+      uint64_t* s = sum + (uint64_t)k * (c.cols + 1);
+      const uint64_t m = s[c.cols];
+      const uint64_t v = col ? s[lane] : 0;
+      if (col) s[lane] = cur;
+      if ((m >> lane) & 1ull) cur = v;
+    }
+    __syncthreads();
+    if (w == CC_WAVES - 1 && col) rc[lane] = part[w][lane];
+    __syncthreads();  // part and mask are rewritten by the next queue
+  }
+}
+
+__global__ __launch_bounds__(CB_BT) void k_comb_resolve(launch::CombArgs c, const uint32_t* srow, const uint32_t* sop) {
+  __shared__ uint64_t val[CB_BT];         // written values, by access
+  __shared__ uint64_t sum[CB_WAVES][64];  // per wave: the last value it wrote to each column
+  __shared__ uint64_t cin[CB_WAVES][64];  // per wave: each column's value at its first access
+  __shared__ uint64_t wmask[CB_WAVES];    // per wave: the columns it wrote
+  const uint32_t nc = min(c.ctr[launch::COMB_CHUNKS], c.chunk_cap);
   const uint32_t tid = threadIdx.x, w = tid / 64, lane = tid % 64;
   uint64_t done_ops = 0;
-  for (uint32_t sg = blockIdx.x; sg < nseg; sg += gridDim.x) {
-    const uint2 seg = segs[sg];
-    const uint32_t p0 = seg.x, len = seg.y;
-    uint64_t* rc = cells + (uint64_t)srow[p0] * cols;
-    if (tid < cols) cell[tid] = rc[tid];
-    for (uint32_t b = 0; b < len; b += CB_BT) {
-      const uint32_t i = b + tid;
-      const bool valid = i < len;
-      uint32_t opid = 0, col = 0;
-      bool isw = false;
-      uint64_t wv = 0;
-      if (valid) {
-        const uint32_t so = sop[p0 + i];
-        opid = so & OPID_MASK;
-        isw = (so & OPID_WRITE) != 0;
-        col = op_col(ops[opid]);
-        if (isw) wv = wvals[opid];
-      }
-      int src = -1;  // the lane (of this wave) whose write this read sees
-      uint64_t written = 0;
-      uint64_t wm = dev::ballot(valid && isw);
-      while (wm) {  // the columns written among the wave's 64 entries
-        const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)col, __ffsll((unsigned long long)wm) - 1);
-        const uint64_t wc = dev::ballot(valid && isw && col == c);
-        if (valid && col == c) {
-          if (isw) {
-            if ((wc >> lane) >> 1 == 0) sum[w][c] = wv;  // the wave's last write of c
-          } else {
-            const uint64_t below = wc & dev::lanemask_lt();
-            if (below) src = 63 - __clzll((long long)below);
-          }
-        }
-        written |= 1ull << c;
-        wm &= ~wc;
-      }
-      val[tid] = wv;
-      if (lane == 0) wmask[w] = written;
-      __syncthreads();
-      if (tid < cols) {
-        uint64_t cur = cell[tid];
-        for (int x = 0; x < CB_WAVES; ++x) {
-          cin[x][tid] = cur;
-          if ((wmask[x] >> tid) & 1ull) cur = sum[x][tid];
-        }
-        cell[tid] = cur;
-      }
-      __syncthreads();
-      if (valid) {
-        if (!isw) reads[opid] = src >= 0 ? val[w * 64 + (uint32_t)src] : cin[w][col];
-        need[opid] = NEED_DONE;
-      }
-      __syncthreads();  // val / sum / cin / wmask are rewritten by the next step
+  for (uint32_t x = blockIdx.x; x < nc; x += gridDim.x) {
+    const uint4 ch = c.chunks[x];
+    const bool valid = tid < ch.y;
+    uint32_t opid = 0, col = 0;
+    bool isw = false;
+    uint64_t wv = 0;
+    if (valid) {
+      const uint32_t so = sop[ch.x + tid];
+      opid = so & OPID_MASK;
+      isw = (so & OPID_WRITE) != 0;
+      col = op_col(c.ops[opid]);
+      if (isw) wv = comb_value(c, opid);
     }
-    if (tid < cols) rc[tid] = cell[tid];
-    done_ops += len;
-    __syncthreads();  // cell is reloaded for the next row
+    uint64_t* rc = c.cells + (uint64_t)srow[ch.x] * c.cols;
+    const uint64_t* from = ch.z ? c.sums + (uint64_t)(ch.z - 1) * (c.cols + 1) : rc;
+    const uint64_t start = tid < c.cols ? from[tid] : 0;
+    int src = -1;  // the lane (of this wave) whose write this read sees
+    uint64_t written = 0;
+    uint64_t wm = dev::ballot(valid && isw);
+    while (wm) {  // the columns written among the wave's 64 accesses
+      const uint32_t cc = (uint32_t)__builtin_amdgcn_readlane((int)col, __ffsll((unsigned long long)wm) - 1);
+      const uint64_t wc = dev::ballot(valid && isw && col == cc);
+      if (valid && col == cc) {
+        if (isw) {
+          if ((wc >> lane) >> 1 == 0) sum[w][cc] = wv;  // the wave's last write of cc
+        } else {
+          const uint64_t below = wc & dev::lanemask_lt();
+          if (below) src = 63 - __clzll((long long)below);
+        }
+      }
+      written |= 1ull << cc;
+      wm &= ~wc;
+    }
+    val[tid] = wv;
+    if (lane == 0) wmask[w] = written;
+    __syncthreads();
+    if (tid < c.cols) {
+      uint64_t cur = start;
+      for (int y = 0; y < CB_WAVES; ++y) {
+        cin[y][tid] = cur;
+        if ((wmask[y] >> tid) & 1ull) cur = sum[y][tid];
+      }
+      if (ch.z == 0) rc[tid] = cur;  // the queue's only chunk: the row's final cells
+    }
+    __syncthreads();
+    if (valid) {
+      if (!isw) c.reads[opid] = src >= 0 ? val[w * 64 + (uint32_t)src] : cin[w][col];
+      c.need[opid] = NEED_DONE;
+    }
+    done_ops += ch.y;
+    __syncthreads();  // val / sum / cin / wmask are rewritten by the next chunk
   }
-  if (tid == 0 && done_ops) atomicAdd((unsigned long long*)combined, (unsigned long long)done_ops);
+  if (tid == 0 && done_ops) atomicAdd(c.combined, (unsigned long long)done_ops);
 }
 
 // Open form (serving), one admitted batch at a time, accesses sorted by
@@ -1282,25 +1398,23 @@ hipError_t access_group_flags(const uint32_t* srow, const uint32_t* sop, uint64_
 uint64_t seg_tmp_words(uint64_t n) { return 4 * ((n + TT - 1) / TT); }
 template <class KT>
 static hipError_t seg_turns_impl(const KT* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
-                                 uint32_t* counters, uint64_t nrows, uint32_t comb_min, uint2* segs, uint32_t* seg_ctr,
-                                 uint32_t seg_cap, uint64_t* conflicts, hipStream_t s) {
+                                 uint32_t* counters, uint64_t nrows, const CombArgs& comb, uint64_t* conflicts,
+                                 hipStream_t s) {
   if (n == 0) return hipSuccess;
   const unsigned nb = (unsigned)((n + TT - 1) / TT);
   uint4* summ = reinterpret_cast<uint4*>(tmp);
   hipLaunchKernelGGL((k_seg_tiles<KT>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ);
-  hipLaunchKernelGGL((k_seg_turns<KT>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, need, counters, nrows, comb_min,
-                     segs, seg_ctr, seg_cap, (unsigned long long*)conflicts);
+  hipLaunchKernelGGL((k_seg_turns<KT>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, need, counters, nrows, comb,
+                     (unsigned long long*)conflicts);
   return hipGetLastError();
 }
 hipError_t seg_turns(const uint32_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
-                     uint32_t* counters, uint64_t nrows, uint32_t comb_min, uint2* segs, uint32_t* seg_ctr,
-                     uint32_t seg_cap, uint64_t* conflicts, hipStream_t s) {
-  return seg_turns_impl(key, val, n, rb, tmp, need, counters, nrows, comb_min, segs, seg_ctr, seg_cap, conflicts, s);
+                     uint32_t* counters, uint64_t nrows, const CombArgs& comb, uint64_t* conflicts, hipStream_t s) {
+  return seg_turns_impl(key, val, n, rb, tmp, need, counters, nrows, comb, conflicts, s);
 }
 hipError_t seg_turns64(const uint64_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
                        uint32_t* counters, uint64_t nrows, uint64_t* conflicts, hipStream_t s) {
-  return seg_turns_impl(key, val, n, rb, tmp, need, counters, nrows, 0u, (uint2*)nullptr, (uint32_t*)nullptr, 0u,
-                        conflicts, s);
+  return seg_turns_impl(key, val, n, rb, tmp, need, counters, nrows, CombArgs{}, conflicts, s);
 }
 hipError_t seg_ranks(const uint32_t* row, const uint32_t* val, uint64_t n, uint32_t* tmp, uint64_t nrows,
                      uint32_t* rank, uint32_t* max_rank, hipStream_t s) {
@@ -1311,19 +1425,17 @@ hipError_t seg_ranks(const uint32_t* row, const uint32_t* val, uint64_t n, uint3
   hipLaunchKernelGGL(k_seg_ranks, dim3(nb), dim3(BT), 0, s, row, val, n, summ, nrows, rank, max_rank);
   return hipGetLastError();
 }
-hipError_t gacco_combine(const uint2* segs, const uint32_t* seg_ctr, uint32_t seg_cap, const uint32_t* srow,
-                         const uint32_t* sop, const uint64_t* ops, const uint32_t* op_tx, const uint64_t* tx_off,
-                         uint64_t nops, uint64_t* cells, uint32_t cols, uint64_t seed, uint64_t* wvals, uint64_t* reads,
-                         uint32_t* need, uint64_t* combined, hipStream_t s) {
-  if (seg_cap == 0 || cols == 0 || cols > 64 || nops == 0) return hipSuccess;
-  // a capped grid: with no queue listed every block leaves at once
-  hipLaunchKernelGGL(k_gacco_wvals, dim3(reduce_blocks(nops)), dim3(BT), 0, s, op_tx, tx_off, nops, seed, seg_ctr,
-                     wvals);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const uint32_t grid = seg_cap < 512 ? seg_cap : 512;
-  hipLaunchKernelGGL(k_gacco_combine, dim3(grid), dim3(CB_BT), 0, s, segs, seg_ctr, seg_cap, srow, sop, ops, wvals,
-                     cells, cols, reads, need, combined);
+uint64_t comb_chunk_cap(uint64_t nops, uint32_t min) { return nops / min + nops / CB_BT + 1; }
+uint64_t comb_multi_cap(uint64_t nops) { return nops / CB_BT + 1; }
+uint64_t comb_sum_words(uint64_t nops, uint32_t cols) { return (2 * (nops / CB_BT) + 1) * (cols + 1ull); }
+hipError_t gacco_combine(const CombArgs& c, const uint32_t* srow, const uint32_t* sop, hipStream_t s) {
+  if (c.cols == 0 || c.cols > 64 || c.chunk_cap == 0) return hipSuccess;
+  // capped grids: with no queue listed every block leaves at once
+  const unsigned grid = c.chunk_cap < 2048 ? c.chunk_cap : 2048;
+  const unsigned mgrid = c.multi_cap < 256 ? c.multi_cap : 256;
+  hipLaunchKernelGGL(k_comb_sums, dim3(grid), dim3(CB_BT), 0, s, c, sop);
+  hipLaunchKernelGGL(k_comb_carry, dim3(mgrid), dim3(CC_WAVES * 64), 0, s, c, srow);
+  hipLaunchKernelGGL(k_comb_resolve, dim3(grid), dim3(CB_BT), 0, s, c, srow, sop);
   return hipGetLastError();
 }
 hipError_t gtx_exec_keys(const uint32_t* rows, const uint32_t* op_tx, const uint32_t* rank,

@@ -155,10 +155,10 @@ struct gcctb_ctx {
   bool hot_active = false; // the launch reads hot flags (2PL with the deferral)
   // 2PL: lock hot keys after the others (GCCTB_HOT_LAST=0 turns it off)
   bool hot_last = true;
-  // GaccO combiners: queue list (first position, length) and counters
-  // ([0] low half: queues listed; [1]: ops the combiners ran)
-  gcctb::DevBuf<uint64_t> comb_segs, comb_ctr, comb_wv;
-  uint64_t comb_cap = 0;
+  // GaccO combiners: chunk and queue lists, chunk summaries, and counters
+  // (launch::COMB_WORDS u32, then the ops the combiners ran)
+  gcctb::DevBuf<uint64_t> comb_lists, comb_sums, comb_ctr;
+  uint64_t comb_chunk_cap = 0, comb_multi_cap = 0;
   gcctb::DevBuf<uint64_t> conflicts;
   // watchdog diagnostics (GCCTB_DEBUG_DUMP=<file>)
   gcctb::DevBuf<uint64_t> dbg;
@@ -432,6 +432,26 @@ class GaccoHost : public SchemeHost {
     HIP_TRY(launch::row_base_add(srow, rstart, n, ctx.cfg.rows, ctx.rowbase.p, s));
   }
   bool OpenRowsProbed() const override { return true; }
+  launch::CombArgs comb_args() const {
+    launch::CombArgs c{};
+    c.min = ctx.comb_min;
+    c.chunk_cap = (uint32_t)ctx.comb_chunk_cap;
+    c.multi_cap = (uint32_t)ctx.comb_multi_cap;
+    c.chunks = reinterpret_cast<uint4*>(ctx.comb_lists.p);
+    c.multi = c.chunks + ctx.comb_chunk_cap;
+    c.sums = ctx.comb_sums.p;
+    c.ctr = reinterpret_cast<uint32_t*>(ctx.comb_ctr.p);
+    c.ops = ctx.ops.p;
+    c.op_tx = ctx.op_tx.p;
+    c.tx_off = ctx.tx_off.p;
+    c.cells = ctx.cells.p;
+    c.cols = ctx.cfg.cols;
+    c.seed = ctx.cfg.seed;
+    c.reads = ctx.reads.p;
+    c.need = ctx.need.p;
+    c.combined = reinterpret_cast<unsigned long long*>(ctx.comb_ctr.p + launch::COMB_WORDS / 2);
+    return c;
+  }
   // per-row access queues for ops [o0, o1) in (row, transaction id) order;
   // the rows also land in rows_out[o0, o1).  stream: the whole stream at
   // once, whose long row queues go to combiners (column mode).
@@ -444,17 +464,12 @@ class GaccoHost : public SchemeHost {
     // rows are below cfg.rows; a miss (IDX_MISS) has all row bits set and sorts last
     HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, bits_for(ctx.cfg.rows),
                                    ctx.sort_tmp.p, &srow, &sop, s));
-    const bool comb = stream && ctx.comb_min && ctx.comb_cap && ctx.cfg.cols <= 64 && !ctx.cfg.row_ops && !ctx.tpcc;
-    if (comb) HIP_TRY(launch::fill_u64(ctx.comb_ctr.p, 2, 0, s));
-    uint2* segs = reinterpret_cast<uint2*>(ctx.comb_segs.p);
-    uint32_t* nseg = reinterpret_cast<uint32_t*>(ctx.comb_ctr.p);
+    const bool comb = stream && ctx.comb_min && ctx.comb_chunk_cap && ctx.cfg.cols <= 64 && !ctx.cfg.row_ops && !ctx.tpcc;
+    const launch::CombArgs ca = comb ? comb_args() : launch::CombArgs{};
+    if (comb) HIP_TRY(launch::fill_u64(ctx.comb_ctr.p, ctx.comb_ctr.n, 0, s));
     HIP_TRY(launch::fill_u32(ctx.need.p + o0, n, NEED_FREE, s));
-    HIP_TRY(launch::seg_turns(srow, sop, n, 0, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows,
-                              comb ? ctx.comb_min : 0u, segs, nseg, (uint32_t)ctx.comb_cap, nullptr, s));
-    if (comb)
-      HIP_TRY(launch::gacco_combine(segs, nseg, (uint32_t)ctx.comb_cap, srow, sop, ctx.ops.p, ctx.op_tx.p,
-                                    ctx.tx_off.p, ctx.nops, ctx.cells.p, ctx.cfg.cols, ctx.cfg.seed, ctx.comb_wv.p,
-                                    ctx.reads.p, ctx.need.p, ctx.comb_ctr.p + 1, s));
+    HIP_TRY(launch::seg_turns(srow, sop, n, 0, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows, ca, nullptr, s));
+    if (comb) HIP_TRY(launch::gacco_combine(ca, srow, sop, s));
     if (stream) combined_ = comb;
   }
   void Launch(int b, uint64_t lo, uint64_t hi, bool persist) override {
@@ -467,7 +482,7 @@ class GaccoHost : public SchemeHost {
   // ops run by the combiners in the last persistent pass
   uint64_t Combined() const override {
     uint64_t v = 0;
-    if (combined_) HIP_TRY(hipMemcpy(&v, ctx.comb_ctr.p + 1, 8, hipMemcpyDeviceToHost));
+    if (combined_) HIP_TRY(hipMemcpy(&v, ctx.comb_ctr.p + launch::COMB_WORDS / 2, 8, hipMemcpyDeviceToHost));
     return v;
   }
   bool combined_ = false;
@@ -548,8 +563,8 @@ class GPUTxHost : public SchemeHost {
       uint32_t* skey;
       HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, row_bits + rank_bits,
                                      ctx.sort_tmp.p, &skey, &sop2, s));
-      HIP_TRY(launch::seg_turns(skey, sop2, n, rank_bits, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows, 0u,
-                                nullptr, nullptr, 0u, ctx.conflicts.p, s));
+      HIP_TRY(launch::seg_turns(skey, sop2, n, rank_bits, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows,
+                                launch::CombArgs{}, ctx.conflicts.p, s));
     } else {
       HIP_TRY(launch::gtx_exec_keys(ctx.rows_out.p, ctx.op_tx.p, ctx.rank.p, n, rank_bits, ctx.sk64a.p, s));
       uint64_t* skey;
@@ -985,12 +1000,12 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
       }
       c->sort_tmp.alloc(
           std::max({launch::radix_sort_tmp_words(n), launch::scan_tmp_words(n), launch::seg_tmp_words(n)}));
-      if (c->scheme == SCHEME_GACCO && c->comb_min) {
-        // at most nops / comb_min queues reach comb_min accesses
-        c->comb_cap = std::min<uint64_t>(nops / c->comb_min + 1, 0x7fffffffull);
-        c->comb_segs.alloc(c->comb_cap);
-        c->comb_ctr.alloc(2);
-        c->comb_wv.alloc(nops);  // every op's write value, for the combiners
+      if (c->scheme == SCHEME_GACCO && c->comb_min && c->cfg.cols <= 64) {
+        c->comb_chunk_cap = launch::comb_chunk_cap(nops, c->comb_min);
+        c->comb_multi_cap = launch::comb_multi_cap(nops);
+        c->comb_lists.alloc(2 * (c->comb_chunk_cap + c->comb_multi_cap));
+        c->comb_sums.alloc(launch::comb_sum_words(nops, c->cfg.cols));
+        c->comb_ctr.alloc(launch::COMB_WORDS / 2 + 1);
       }
       if (c->scheme == SCHEME_GPUTX) {
         c->sk64a.alloc(n);

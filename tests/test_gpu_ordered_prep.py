@@ -106,3 +106,29 @@ def test_slot_stash(scheme, wd, bs, window, ntx):
     exp_t, exp_r, ties = orc.replay(rows, 10, g.SEED, orc.seed_table(g.SEED, rows, 10), w.ops, w.tx_off, res["order"])
     isr = ~g.op_is_write(w.ops)
     assert ties == 0 and np.array_equal(res["table"], exp_t) and np.array_equal(res["reads"][isr], exp_r[isr])
+
+
+COMB_CHUNK = 256  # accesses per combiner chunk; the carry splits a queue's chunks over 16 waves
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length", [128, COMB_CHUNK, COMB_CHUNK + 1, 16 * COMB_CHUNK, 40 * COMB_CHUNK + 3])
+@pytest.mark.parametrize("cols,write_share", [(3, 0.5), (64, 0.02), (10, 0.0)])
+def test_combiner_chunks(length, cols, write_share):
+    """Two queues of the same length at chunk edges, beside short ones, run by
+    combiners: the serial run in transaction-id order."""
+    rng = np.random.default_rng(length * 100 + cols)
+    rows = 3 + length
+    keys = np.stack([np.full(length, 1), np.full(length, 2), 3 + rng.permutation(length)], axis=1)
+    ops = g.make_ops(keys.reshape(-1), rng.integers(0, cols, 3 * length), rng.random(3 * length) < write_share)
+    w = g.Ops(ops, np.arange(length + 1, dtype=np.uint64) * np.uint64(3))
+    print(f"[comb-chunks] length={length} cols={cols} writes={write_share}", flush=True)
+    with g.Context("gacco", rows=rows, cols=cols, warp_density=2, block_size=8, batch_size=1 << 20) as ctx:
+        ctx.seed_table()
+        ctx.load_ops(w)
+        st = ctx.run("persistent")
+        res = ctx.fetch()
+    assert st["committed"] == length and st["combined"] == 2 * length
+    t2, r2 = orc.replay_txid(rows, cols, g.SEED, orc.seed_table(g.SEED, rows, cols), w.ops, w.tx_off)
+    isr = ~g.op_is_write(w.ops)
+    assert np.array_equal(res["table"], t2) and np.array_equal(res["reads"][isr], r2[isr])
