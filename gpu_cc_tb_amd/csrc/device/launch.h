@@ -34,7 +34,7 @@ hipError_t seed_table(uint64_t* cells, uint64_t rows, uint32_t cols, uint64_t se
 // (every u32 IDX_EMPTY).  Keys must be unique and not IDX_EMPTY.
 hipError_t index_insert(const uint32_t* keys, const uint32_t* vals, uint64_t n, uint32_t* buckets,
                         uint32_t nbuckets, hipStream_t s);
-// rows_out[i] = row of ops[i]'s key; also into rows_copy when it is given;
+// rows_out[i] = row of ops[i]'s key (rows_out may be null); also into rows_copy when it is given;
 // ids_out[i] = what op_ids(ops, n, id_base) writes, when it is given; with
 // id_map, id_map[i] with the op's write flag in bit 31 instead
 hipError_t probe(const IndexView& ix, const uint64_t* ops, uint64_t n, uint32_t* rows_out,
@@ -54,13 +54,15 @@ hipError_t fill_u64(uint64_t* v, uint64_t n, uint64_t x, hipStream_t s);
 // Sorts bits [0, key_bits) of the keys.  Buffers: keys/vals in, alt buffers of
 // the same size; the sorted result ends in (*keys_out, *vals_out), which point
 // to one of the two buffer pairs.  tmp must hold radix_sort_tmp_words(n) u32.
+// Here and below, nd (when given) is a device word that holds the actual
+// element count, at most n.
 uint64_t radix_sort_tmp_words(uint64_t n);
 hipError_t radix_sort_u32(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint64_t n,
                           int key_bits, uint32_t* tmp, uint32_t** keys_out, uint32_t** vals_out,
-                          hipStream_t s);
+                          hipStream_t s, const uint32_t* nd = nullptr);
 hipError_t radix_sort_u64(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint64_t n,
                           int key_bits, uint32_t* tmp, uint64_t** keys_out, uint32_t** vals_out,
-                          hipStream_t s);
+                          hipStream_t s, const uint32_t* nd = nullptr);
 
 // --- scans (u32) --- tmp must hold scan_tmp_words(n) u32.
 uint64_t scan_tmp_words(uint64_t n);
@@ -106,15 +108,41 @@ uint64_t comb_chunk_cap(uint64_t nops, uint32_t min);
 uint64_t comb_multi_cap(uint64_t nops);
 uint64_t comb_sum_words(uint64_t nops, uint32_t cols);
 hipError_t seg_turns(const uint32_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
-                     uint32_t* counters, uint64_t nrows, const CombArgs& comb, uint64_t* conflicts, hipStream_t s);
+                     uint32_t* counters, uint64_t nrows, const CombArgs& comb, uint64_t* conflicts, hipStream_t s,
+                     const uint32_t* nd = nullptr);
 hipError_t seg_turns64(const uint64_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
-                       uint32_t* counters, uint64_t nrows, uint64_t* conflicts, hipStream_t s);
+                       uint32_t* counters, uint64_t nrows, uint64_t* conflicts, hipStream_t s,
+                       const uint32_t* nd = nullptr);
 // GPUTx one-pass rank (src/gputx.cu:5-27) from accesses sorted by (row, tx),
 // val[p] the access's transaction with its write flag in bit 31: rank[tx] =
 // max over tx's accesses of the access-group boundaries of their rows up to
-// them (the caller zeroes rank and max_rank); max_rank = max.
+// them (the caller zeroes rank and max_rank); max_rank = max.  tx_of (when
+// given) maps val[p] without its flag to the transaction.
 hipError_t seg_ranks(const uint32_t* row, const uint32_t* val, uint64_t n, uint32_t* tmp, uint64_t nrows,
-                     uint32_t* rank, uint32_t* max_rank, hipStream_t s);
+                     uint32_t* rank, uint32_t* max_rank, hipStream_t s, const uint32_t* tx_of = nullptr,
+                     const uint32_t* nd = nullptr);
+// The accesses that can meet another one: those of rows that some op of
+// ops[0, n) writes, in op order (rows: each op's row, null with a dense index:
+// the key).  crow / cval get their rows and op ids (id_base + i, write flag in
+// bit 31), *f.count their number, and need[i] = NEED_FREE for every op.  With
+// f.crow set, cval gets the access's own index (with the flag) instead, and
+// f.crow / f.cop / f.ctx its row, op id and transaction op_tx[i].  f.wmap
+// (ord_map_bytes(nrows) bytes) is zero before and after; f.bits holds
+// nrows / 32 words, f.flags ord_flag_words(n), tmp radix_sort_tmp_words(n).
+struct OrdFilter {
+  uint8_t* wmap;
+  uint32_t* bits;
+  uint64_t* flags;
+  uint32_t* count;
+  uint32_t* crow;
+  uint32_t* cop;
+  uint32_t* ctx;
+};
+uint64_t ord_flag_words(uint64_t n);
+uint64_t ord_map_bytes(uint64_t nrows);
+hipError_t ord_filter(const IndexView& ix, const uint64_t* ops, const uint32_t* rows, uint64_t n, uint64_t nrows,
+                      uint32_t id_base, const uint32_t* op_tx, const OrdFilter& f, uint32_t* tmp, uint32_t* need,
+                      uint32_t* crow, uint32_t* cval, hipStream_t s);
 // GaccO, persistent form: run each listed row queue in order on the row's
 // cells (cols <= 64), store its reads' results, mark its ops need = NEED_DONE
 // and add the ops run to *combined.  srow, sop: the sorted accesses.
@@ -126,12 +154,12 @@ hipError_t access_need_open(const uint32_t* srow, const uint32_t* sop, const uin
                             uint64_t n, uint64_t nrows, const uint32_t* base, uint32_t* need, hipStream_t s);
 hipError_t row_base_add(const uint32_t* srow, const uint32_t* rstart, uint64_t n, uint64_t nrows, uint32_t* base,
                         hipStream_t s);
-// composite key (row << rank_bits) | rank[op_tx[op]] for ops [0, n)
-hipError_t gtx_exec_keys(const uint32_t* rows, const uint32_t* op_tx, const uint32_t* rank,
-                         uint64_t n, int rank_bits, uint64_t* keys, hipStream_t s);
+// composite key (rows[i] << rank_bits) | rank[tx[i]] for i in [0, n)
+hipError_t gtx_exec_keys(const uint32_t* rows, const uint32_t* tx, const uint32_t* rank, uint64_t n, int rank_bits,
+                         uint64_t* keys, hipStream_t s, const uint32_t* nd = nullptr);
 // the same key cut to 32 bits, for row_bits + rank_bits <= 32
-hipError_t gtx_exec_keys32(const uint32_t* rows, const uint32_t* op_tx, const uint32_t* rank,
-                           uint64_t n, int rank_bits, uint32_t* keys, hipStream_t s);
+hipError_t gtx_exec_keys32(const uint32_t* rows, const uint32_t* tx, const uint32_t* rank, uint64_t n, int rank_bits,
+                           uint32_t* keys, hipStream_t s, const uint32_t* nd = nullptr);
 hipError_t rank_hist(const uint32_t* rank, uint64_t ntx, uint32_t nranks, uint32_t* hist, hipStream_t s);
 
 // --- memory-system ceilings (microbench.hip) ---

@@ -146,6 +146,11 @@ struct gcctb_ctx {
   // preprocessing scratch
   gcctb::DevBuf<uint32_t> sk0, sv0, sk1, sv1, flags, gstart, sort_tmp;
   gcctb::DevBuf<uint64_t> sk64a, sk64b;
+  // GaccO / GPUTx: written rows (a byte, then a bit each), the ops on them and
+  // their number; GPUTx: those ops' rows, ids and transactions in op order
+  gcctb::DevBuf<uint8_t> ord_map;
+  gcctb::DevBuf<uint32_t> ord_bits, ord_count, ord_row, ord_op, ord_tx;
+  gcctb::DevBuf<uint64_t> ord_flags;
   gcctb::DevBuf<uint32_t> rank, tx_map, max_rank;
   // hot-writer deferral: sampled counts and state, slot -> transaction map;
   // in use while defer_active
@@ -317,6 +322,35 @@ class SchemeHost {
     a.ev_commit = ctx.cfg.debug_events ? ctx.ev_commit.p : nullptr;
     return a;
   }
+  // GaccO / GPUTx preparation over n ops: whether only the accesses of written
+  // rows are sorted (launch::ord_filter).  Choosing them reads the ops three
+  // times and looks every row up in a bitmap, which pays while few rows are
+  // written (up to a third as many writes as rows: a quarter to a third of
+  // the accesses are left) and from 2^20 ops on, where the sort's passes and
+  // not its launches cost.  Preparation without / with it, GPUTx, 10,485,760
+  // rows, 16 ops: 1,048,576 transactions read ratio 0.9 1.24 / 0.73 ms, 0.75
+  // (0.4 writes per row) 1.38 / 1.12, 0.5 (0.8) 1.53 / 1.56; 65,536
+  // transactions 0.9 0.25 / 0.22; 16,384 0.18 / 0.20.  On 1,048,576 rows, 0.9
+  // (1.6 writes per row) 1.54 / 1.54 ms.  GaccO at 0.75: 0.61 / 0.57 ms, 0.5
+  // 0.67 / 0.77.
+  bool ord_filtered(uint64_t n) const {
+    if (n < (1ull << 20) || ctx.cfg.rows > 16 * n) return false;
+    const double writes = (double)(ctx.nops - ctx.nreads) * ((double)n / (double)ctx.nops);
+    return writes * 3 <= (double)ctx.cfg.rows;
+  }
+  launch::OrdFilter ord_buffers() const {
+    launch::OrdFilter f{};
+    f.wmap = ctx.ord_map.p;
+    f.bits = ctx.ord_bits.p;
+    f.flags = ctx.ord_flags.p;
+    f.count = ctx.ord_count.p;
+    if (ctx.scheme == SCHEME_GPUTX) {
+      f.crow = ctx.ord_row.p;
+      f.cop = ctx.ord_op.p;
+      f.ctx = ctx.ord_tx.p;
+    }
+    return f;
+  }
   // Kernel variants (whole-row mode, the event log): every scheme's plain
   // kernels of a variant come from one launcher.
   bool launch_rows(const ExecArgs& a, uint64_t n, bool persist) {
@@ -407,7 +441,7 @@ class GaccoHost : public SchemeHost {
   void PrepStream() override { prep_range(0, ctx.nops, true); }
   void PostStream() override {}
   void PrepLaunch(uint64_t o0, uint64_t o1) override { prep_range(o0, o1, false); }
-  bool ProbesRows() const override { return true; }
+  bool ProbesRows() const override { return !ctx.ix.dense; }
   // Open launch: every row's queue starts empty; each admitted batch's
   // accesses queue behind those of the batches admitted before it, in
   // transaction-id order (rowbase counts the queued accesses per row).
@@ -453,22 +487,33 @@ class GaccoHost : public SchemeHost {
     return c;
   }
   // per-row access queues for ops [o0, o1) in (row, transaction id) order;
-  // the rows also land in rows_out[o0, o1).  stream: the whole stream at
-  // once, whose long row queues go to combiners (column mode).
+  // over a hash index the rows also land in rows_out[o0, o1).  stream: the
+  // whole stream at once, whose long row queues go to combiners (column mode).
   void prep_range(uint64_t o0, uint64_t o1, bool stream) {
     const uint64_t n = o1 - o0;
     if (n == 0) return;
     hipStream_t s = ctx.stream;
-    HIP_TRY(launch::probe(ctx.ix, ctx.ops.p + o0, n, ctx.rows_out.p + o0, s, ctx.sk0.p, ctx.sv0.p, (uint32_t)o0));
+    const bool comb = stream && ctx.comb_min && ctx.comb_chunk_cap && ctx.cfg.cols <= 64 && !ctx.cfg.row_ops && !ctx.tpcc;
+    // a dense index: the row is the key, and the launch finds it itself
+    uint32_t* rows = ctx.ix.dense ? nullptr : ctx.rows_out.p + o0;
     uint32_t *srow, *sop;
+    const uint32_t* nd = nullptr;
+    if (!comb && ord_filtered(n)) {  // (a combiner also runs long queues of reads alone)
+      if (rows) HIP_TRY(launch::probe(ctx.ix, ctx.ops.p + o0, n, rows, s));
+      HIP_TRY(launch::ord_filter(ctx.ix, ctx.ops.p + o0, rows, n, ctx.cfg.rows, (uint32_t)o0, nullptr, ord_buffers(),
+                                 ctx.sort_tmp.p, ctx.need.p + o0, ctx.sk0.p, ctx.sv0.p, s));
+      nd = ctx.ord_count.p;
+    } else {
+      HIP_TRY(launch::probe(ctx.ix, ctx.ops.p + o0, n, rows, s, ctx.sk0.p, ctx.sv0.p, (uint32_t)o0));
+      HIP_TRY(launch::fill_u32(ctx.need.p + o0, n, NEED_FREE, s));
+    }
     // rows are below cfg.rows; a miss (IDX_MISS) has all row bits set and sorts last
     HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, bits_for(ctx.cfg.rows),
-                                   ctx.sort_tmp.p, &srow, &sop, s));
-    const bool comb = stream && ctx.comb_min && ctx.comb_chunk_cap && ctx.cfg.cols <= 64 && !ctx.cfg.row_ops && !ctx.tpcc;
+                                   ctx.sort_tmp.p, &srow, &sop, s, nd));
     const launch::CombArgs ca = comb ? comb_args() : launch::CombArgs{};
     if (comb) HIP_TRY(launch::fill_u64(ctx.comb_ctr.p, ctx.comb_ctr.n, 0, s));
-    HIP_TRY(launch::fill_u32(ctx.need.p + o0, n, NEED_FREE, s));
-    HIP_TRY(launch::seg_turns(srow, sop, n, 0, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows, ca, nullptr, s));
+    HIP_TRY(launch::seg_turns(srow, sop, n, 0, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows, ca, nullptr, s,
+                              nd));
     if (comb) HIP_TRY(launch::gacco_combine(ca, srow, sop, s));
     if (stream) combined_ = comb;
   }
@@ -527,17 +572,28 @@ class GPUTxHost : public SchemeHost {
     hipStream_t s = ctx.stream;
     // per-row access lists in (row, tx) order; the sorted values are the
     // accesses' transactions (with the write flag), so the rank pass needs
-    // no op -> transaction gather
-    HIP_TRY(launch::probe(ctx.ix, ctx.ops.p, n, ctx.rows_out.p, s, ctx.sk0.p, ctx.sv0.p, 0, ctx.op_tx.p));
+    // no op -> transaction gather (of the chosen accesses alone, their indexes)
+    const bool filt = ord_filtered(n);
+    uint32_t* rows = filt && ctx.ix.dense ? nullptr : ctx.rows_out.p;
+    const uint32_t *nd = nullptr, *tx_of = nullptr;
+    if (filt) {
+      if (rows) HIP_TRY(launch::probe(ctx.ix, ctx.ops.p, n, rows, s));
+      HIP_TRY(launch::ord_filter(ctx.ix, ctx.ops.p, rows, n, ctx.cfg.rows, 0, ctx.op_tx.p, ord_buffers(),
+                                 ctx.sort_tmp.p, ctx.need.p, ctx.sk0.p, ctx.sv0.p, s));
+      nd = ctx.ord_count.p;
+      tx_of = ctx.ord_tx.p;
+    } else {
+      HIP_TRY(launch::probe(ctx.ix, ctx.ops.p, n, rows, s, ctx.sk0.p, ctx.sv0.p, 0, ctx.op_tx.p));
+    }
     uint32_t *srow, *stx_ops;
     // rows are below cfg.rows; a miss (IDX_MISS) has all row bits set and sorts last
     const int row_bits = bits_for(ctx.cfg.rows);
     HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, row_bits, ctx.sort_tmp.p,
-                                   &srow, &stx_ops, s));
+                                   &srow, &stx_ops, s, nd));
     // one-pass local ranks and rank[tx] = max (src/gputx.cu:5-27)
     HIP_TRY(launch::fill_u32(ctx.rank.p, ntx, 0, s));
     HIP_TRY(launch::fill_u32(ctx.max_rank.p, 1, 0, s));
-    HIP_TRY(launch::seg_ranks(srow, stx_ops, n, ctx.sort_tmp.p, ctx.cfg.rows, ctx.rank.p, ctx.max_rank.p, s));
+    HIP_TRY(launch::seg_ranks(srow, stx_ops, n, ctx.sort_tmp.p, ctx.cfg.rows, ctx.rank.p, ctx.max_rank.p, s, tx_of, nd));
     uint32_t max_rank = 0;
     HIP_TRY(hipMemcpyAsync(&max_rank, ctx.max_rank.p, 4, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
@@ -555,30 +611,35 @@ class GPUTxHost : public SchemeHost {
     // when row and rank fit, else 64-bit
     if (!n) return;
     HIP_TRY(launch::fill_u64(ctx.conflicts.p, ctx.conflicts.n, 0, s));
-    HIP_TRY(launch::fill_u32(ctx.need.p, n, NEED_FREE, s));
-    HIP_TRY(launch::op_ids(ctx.ops.p, n, 0, ctx.sv0.p, s));
+    const uint32_t* krow = filt ? ctx.ord_row.p : ctx.rows_out.p;
+    const uint32_t* ktx = filt ? ctx.ord_tx.p : ctx.op_tx.p;
+    uint32_t* v0 = filt ? ctx.ord_op.p : ctx.sv0.p;  // op ids
+    if (!filt) {
+      HIP_TRY(launch::fill_u32(ctx.need.p, n, NEED_FREE, s));
+      HIP_TRY(launch::op_ids(ctx.ops.p, n, 0, v0, s));
+    }
     uint32_t* sop2;
     if (row_bits + rank_bits <= 32) {
-      HIP_TRY(launch::gtx_exec_keys32(ctx.rows_out.p, ctx.op_tx.p, ctx.rank.p, n, rank_bits, ctx.sk0.p, s));
+      HIP_TRY(launch::gtx_exec_keys32(krow, ktx, ctx.rank.p, n, rank_bits, ctx.sk0.p, s, nd));
       uint32_t* skey;
-      HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, row_bits + rank_bits,
-                                     ctx.sort_tmp.p, &skey, &sop2, s));
+      HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, v0, ctx.sk1.p, ctx.sv1.p, n, row_bits + rank_bits, ctx.sort_tmp.p,
+                                     &skey, &sop2, s, nd));
       HIP_TRY(launch::seg_turns(skey, sop2, n, rank_bits, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows,
-                                launch::CombArgs{}, ctx.conflicts.p, s));
+                                launch::CombArgs{}, ctx.conflicts.p, s, nd));
     } else {
-      HIP_TRY(launch::gtx_exec_keys(ctx.rows_out.p, ctx.op_tx.p, ctx.rank.p, n, rank_bits, ctx.sk64a.p, s));
+      HIP_TRY(launch::gtx_exec_keys(krow, ktx, ctx.rank.p, n, rank_bits, ctx.sk64a.p, s, nd));
       uint64_t* skey;
-      HIP_TRY(launch::radix_sort_u64(ctx.sk64a.p, ctx.sv0.p, ctx.sk64b.p, ctx.sv1.p, n, row_bits + rank_bits,
-                                     ctx.sort_tmp.p, &skey, &sop2, s));
+      HIP_TRY(launch::radix_sort_u64(ctx.sk64a.p, v0, ctx.sk64b.p, ctx.sv1.p, n, row_bits + rank_bits,
+                                     ctx.sort_tmp.p, &skey, &sop2, s, nd));
       HIP_TRY(launch::seg_turns64(skey, sop2, n, rank_bits, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows,
-                                  ctx.conflicts.p, s));
+                                  ctx.conflicts.p, s, nd));
     }
   }
   void Init(int, uint64_t) override {}
   // the persistent form runs every rank level in one launch: it needs no
   // per-rank counts (and no host round trip for them)
   void PrepStream() override { rank_all(); }
-  bool ProbesRows() const override { return true; }
+  bool ProbesRows() const override { return !ctx.ix.dense; }
   void PostStream() override {}
   void Launch(int, uint64_t lo, uint64_t hi, bool persist) override {
     ExecArgs a = args(0, lo, hi);
@@ -1000,6 +1061,13 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
       }
       c->sort_tmp.alloc(
           std::max({launch::radix_sort_tmp_words(n), launch::scan_tmp_words(n), launch::seg_tmp_words(n)}));
+      if (!c->ord_map.p) {
+        c->ord_map.alloc(launch::ord_map_bytes(c->cfg.rows));
+        HIP_TRY(hipMemsetAsync(c->ord_map.p, 0, c->ord_map.n, c->stream));
+        c->ord_bits.alloc((c->cfg.rows + 31) / 32);
+        c->ord_count.alloc(1);
+      }
+      c->ord_flags.alloc(launch::ord_flag_words(nops));
       if (c->scheme == SCHEME_GACCO && c->comb_min && c->cfg.cols <= 64) {
         c->comb_chunk_cap = launch::comb_chunk_cap(nops, c->comb_min);
         c->comb_multi_cap = launch::comb_multi_cap(nops);
@@ -1010,6 +1078,9 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
       if (c->scheme == SCHEME_GPUTX) {
         c->sk64a.alloc(n);
         c->sk64b.alloc(n);
+        c->ord_row.alloc(n);
+        c->ord_op.alloc(n);
+        c->ord_tx.alloc(n);
         c->rank.alloc(ntx);
         c->tx_map.alloc(ntx);
         c->max_rank.alloc(1);

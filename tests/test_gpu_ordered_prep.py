@@ -132,3 +132,51 @@ def test_combiner_chunks(length, cols, write_share):
     t2, r2 = orc.replay_txid(rows, cols, g.SEED, orc.seed_table(g.SEED, rows, cols), w.ops, w.tx_off)
     isr = ~g.op_is_write(w.ops)
     assert np.array_equal(res["table"], t2) and np.array_equal(res["reads"][isr], r2[isr])
+
+
+FILTER_MIN = 1 << 20  # ops from which only the accesses of written rows are sorted
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme,form", [("gputx", "persistent"), ("gputx", "plain"), ("gacco", "plain")])
+@pytest.mark.parametrize("read_ratio,missing", [(0.97, False), (0.97, True), (1.0, False)])
+def test_written_rows_filter(scheme, form, read_ratio, missing):
+    """Just past the size where only written rows' accesses are sorted, over a
+    dense index and over one that lacks keys, and with no write at all: the
+    serial replay, and for GPUTx the oracle's ranks."""
+    rows, ntx = 262147, FILTER_MIN // 16 + 3
+    w = g.generate(rows, ntx, theta=0.3, read_ratio=read_ratio)
+    print(f"[filter] scheme={scheme} form={form} reads={read_ratio} missing={missing}", flush=True)
+    with g.Context(scheme, rows=rows, warp_density=3, block_size=8, batch_size=1 << 20) as ctx:
+        ctx.seed_table()
+        if missing:
+            keys = np.arange(rows, dtype=np.uint32)
+            present = keys[keys % 9 != 4]
+            ctx.build_index(present, present)
+        ctx.load_ops(w)
+        st = ctx.run(form, check=False)
+        res = ctx.fetch()
+        ranks = ctx.fetch_ranks()[0] if scheme == "gputx" else None
+    hit = np.ones(w.nops, dtype=bool) if not missing else g.op_key(w.ops) % 9 != 4
+    assert st["committed"] == ntx and st["index_miss"] == int(np.count_nonzero(~hit))
+    # the ops that hit, as transactions of their own: what the run must equal
+    off = np.concatenate([[0], np.cumsum(hit)])[w.tx_off.astype(np.int64)].astype(np.uint64)
+    if missing:
+        # written values depend on the op's place in its transaction, so only reads of unwritten cells are compared
+        cell = g.op_key(w.ops).astype(np.int64) * 10 + g.op_col(w.ops)
+        isw = g.op_is_write(w.ops)
+        calm = hit & ~isw & ~np.isin(cell, np.unique(cell[isw & hit]))
+        init = orc.seed_table(g.SEED, rows, 10)
+        assert np.array_equal(res["reads"][calm], init[cell[calm]])
+        touched = np.zeros(rows * 10, dtype=bool)
+        touched[cell[isw & hit]] = True
+        assert np.array_equal(res["table"][~touched], init[~touched])
+        assert not np.any(res["table"][touched] == init[touched])
+    else:
+        init = orc.seed_table(g.SEED, rows, 10)
+        exp_t, exp_r, ties = orc.replay(rows, 10, g.SEED, init, w.ops, w.tx_off, res["order"])
+        isr = ~g.op_is_write(w.ops)
+        assert ties == 0 and np.array_equal(res["table"], exp_t) and np.array_equal(res["reads"][isr], exp_r[isr])
+    if ranks is not None:
+        part = g.Ops(w.ops[hit], off)
+        assert np.array_equal(ranks, orc.gputx_rank(rows, part.ops, part.tx_off)[0])
