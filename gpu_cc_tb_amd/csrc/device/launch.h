@@ -88,6 +88,7 @@ uint64_t seg_tmp_words(uint64_t n);
 // of several chunks: {first position, first summary, chunks, 0}.
 struct CombArgs {
   uint32_t min;          // shortest queue to combine (0: none)
+  uint32_t whole;        // 1: a queue is one chunk whatever its length
   uint32_t chunk_cap, multi_cap;
   uint4* chunks;
   uint4* multi;
@@ -96,6 +97,7 @@ struct CombArgs {
   const uint64_t* ops;
   const uint32_t* op_tx;
   const uint64_t* tx_off;
+  const uint32_t* op_param;  // TPC-C
   uint64_t* cells;
   uint32_t cols;
   uint64_t seed;
@@ -147,6 +149,8 @@ hipError_t ord_filter(const IndexView& ix, const uint64_t* ops, const uint32_t* 
 // cells (cols <= 64), store its reads' results, mark its ops need = NEED_DONE
 // and add the ops run to *combined.  srow, sop: the sorted accesses.
 hipError_t gacco_combine(const CombArgs& c, const uint32_t* srow, const uint32_t* sop, hipStream_t s);
+// TPC-C, GaccO: the same for queues of updates (c.whole), one wave per queue.
+hipError_t tpcc_combine(const CombArgs& c, const uint32_t* srow, const uint32_t* sop, hipStream_t s);
 // Open form, one admitted batch sorted by (row, op) with group starts gstart
 // and row starts rstart: need[op] = base[row] + gstart[p] - rstart[p]; then
 // row_base_add adds the batch's accesses of each row to base[row].

@@ -56,6 +56,13 @@ struct DevBuf {
   ~DevBuf() { release(); }
 };
 
+// TPC-C under GaccO: every queue of at least this many updates goes to a
+// combiner.  A turn costs the longest queue about 5 us, a combiner's wave a
+// few us for the whole queue.  New orders, 131,072 at 16 warehouses in batches
+// of 16,384: 1.04 / 1.04 / 1.07 ms from 2 / 3 / 4 updates on (from 16 on 1.28,
+// without combiners 4.80); payments, 262,144 at 128 warehouses: 0.59 / 0.64 /
+// 0.66 ms.
+constexpr uint32_t TPCC_COMBINE_MIN = 2;
 int bits_for(uint64_t maxval) {  // bits needed to represent values <= maxval
   int b = 0;
   while (b < 64 && (maxval >> b) != 0) ++b;
@@ -468,7 +475,8 @@ class GaccoHost : public SchemeHost {
   bool OpenRowsProbed() const override { return true; }
   launch::CombArgs comb_args() const {
     launch::CombArgs c{};
-    c.min = ctx.comb_min;
+    c.min = ctx.tpcc ? TPCC_COMBINE_MIN : ctx.comb_min;
+    c.whole = ctx.tpcc ? 1u : 0u;
     c.chunk_cap = (uint32_t)ctx.comb_chunk_cap;
     c.multi_cap = (uint32_t)ctx.comb_multi_cap;
     c.chunks = reinterpret_cast<uint4*>(ctx.comb_lists.p);
@@ -478,6 +486,7 @@ class GaccoHost : public SchemeHost {
     c.ops = ctx.ops.p;
     c.op_tx = ctx.op_tx.p;
     c.tx_off = ctx.tx_off.p;
+    c.op_param = ctx.op_param.p;
     c.cells = ctx.cells.p;
     c.cols = ctx.cfg.cols;
     c.seed = ctx.cfg.seed;
@@ -493,7 +502,9 @@ class GaccoHost : public SchemeHost {
     const uint64_t n = o1 - o0;
     if (n == 0) return;
     hipStream_t s = ctx.stream;
-    const bool comb = stream && ctx.comb_min && ctx.comb_chunk_cap && ctx.cfg.cols <= 64 && !ctx.cfg.row_ops && !ctx.tpcc;
+    // long queues go to combiners: the stream's in column mode (the plain
+    // form keeps the reference's turns), every batch's in TPC-C
+    const bool comb = ctx.comb_chunk_cap && !ctx.cfg.row_ops && (ctx.tpcc || (stream && ctx.cfg.cols <= 64));
     // a dense index: the row is the key, and the launch finds it itself
     uint32_t* rows = ctx.ix.dense ? nullptr : ctx.rows_out.p + o0;
     uint32_t *srow, *sop;
@@ -514,7 +525,7 @@ class GaccoHost : public SchemeHost {
     if (comb) HIP_TRY(launch::fill_u64(ctx.comb_ctr.p, ctx.comb_ctr.n, 0, s));
     HIP_TRY(launch::seg_turns(srow, sop, n, 0, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows, ca, nullptr, s,
                               nd));
-    if (comb) HIP_TRY(launch::gacco_combine(ca, srow, sop, s));
+    if (comb) HIP_TRY(ctx.tpcc ? launch::tpcc_combine(ca, srow, sop, s) : launch::gacco_combine(ca, srow, sop, s));
     if (stream) combined_ = comb;
   }
   void Launch(int b, uint64_t lo, uint64_t hi, bool persist) override {
@@ -1068,7 +1079,12 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
         c->ord_count.alloc(1);
       }
       c->ord_flags.alloc(launch::ord_flag_words(nops));
-      if (c->scheme == SCHEME_GACCO && c->comb_min && c->cfg.cols <= 64) {
+      if (c->scheme == SCHEME_GACCO && c->tpcc && c->comb_min) {
+        c->comb_chunk_cap = launch::comb_chunk_cap(nops, TPCC_COMBINE_MIN);
+        c->comb_multi_cap = 0;
+        c->comb_lists.alloc(2 * c->comb_chunk_cap);
+        c->comb_ctr.alloc(launch::COMB_WORDS / 2 + 1);
+      } else if (c->scheme == SCHEME_GACCO && c->comb_min && c->cfg.cols <= 64) {
         c->comb_chunk_cap = launch::comb_chunk_cap(nops, c->comb_min);
         c->comb_multi_cap = launch::comb_multi_cap(nops);
         c->comb_lists.alloc(2 * (c->comb_chunk_cap + c->comb_multi_cap));

@@ -81,8 +81,8 @@ typedef struct gcctb_stats {
   uint64_t deferred;       /* persistent form of the lock, timestamp and OCC schemes: transactions
                               admitted after all others because they write a hot key */
   uint64_t combined;       /* persistent form of gacco: ops run by hot-row combiners (a row whose
-                              queue holds at least 128 accesses is run in queue order by one
-                              workgroup before the launch) */
+                              queue holds at least 128 accesses is run in queue order on its
+                              own before the launch) */
 } gcctb_stats;
 
 /* Create a context: replaces constructing the scheme by name and its device
@@ -363,7 +363,9 @@ int gcctb_check_host(const gcctb_config* cfg, const uint64_t* init_table, const 
  * gcctb_tpcc_generate's ops and parameters, then gcctb_run_plain (or
  * gcctb_run_graph).  Every op updates its row under the scheme's exclusive
  * access and leaves its result (the next_o_id or stock quantity it read, or
- * the float it updated first) in the reads of gcctb_fetch. */
+ * the float it updated first) in the reads of gcctb_fetch.  Under gacco the
+ * updates of a row that several transactions of a batch share are applied in
+ * queue order before the launch (not counted in gcctb_stats.combined). */
 typedef struct gcctb_tpcc_workload {
   uint32_t warehouses;   /* W, 1..8192 */
   int32_t new_order;     /* 1: new_order transactions, 0: payment (benchmark_cpu/tpcc.cu's isno) */

@@ -180,3 +180,27 @@ def test_written_rows_filter(scheme, form, read_ratio, missing):
     if ranks is not None:
         part = g.Ops(w.ops[hit], off)
         assert np.array_equal(ranks, orc.gputx_rank(rows, part.ops, part.tx_off)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ntx", [1, 2, 63, 64, 65, 200])
+@pytest.mark.parametrize("new_order", [True, False])
+@pytest.mark.parametrize("form", ["plain", "graph"])
+def test_tpcc_queues(ntx, new_order, form):
+    """TPC-C queues around a wave's 64 updates (one warehouse), run twice with
+    the table carried on, the second time in batches: the oracle's replay."""
+    w = g.tpcc_generate(1, ntx, new_order=new_order, seed=ntx)
+    cells, _ = g.tpcc_seed_tables(1)
+    print(f"[tpcc-queues] ntx={ntx} new_order={new_order} form={form}", flush=True)
+    with g.Context("gacco", rows=g.tpcc_rows(1), cols=5, warp_density=4, block_size=4, batch_size=70,
+                   tpcc=True) as ctx:
+        ctx.load_table(cells)
+        ctx.load_ops(w)
+        ctx.load_params(w.params)
+        for _ in range(2):
+            ctx.run(form)
+            res = ctx.fetch()
+            assert g.tpcc_check(1, cells, res["table"], w, res["order"], res["reads"]) == 0
+            exp_t, exp_r = orc.tpcc_replay(g.tpcc_rows(1), cells, w.ops, w.params, w.tx_off, res["order"])[:2]
+            assert np.array_equal(res["table"], exp_t) and np.array_equal(res["reads"], exp_r)
+            cells = res["table"]
