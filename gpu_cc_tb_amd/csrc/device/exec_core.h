@@ -1791,7 +1791,9 @@ __global__ __launch_bounds__(MAXT) void txn_exec(ExecArgs a) {
   if constexpr (PERSIST) {
     run_persistent<S, G>(c, a);
   } else {
-    // plain form: one transaction per group
+    // plain form: one transaction per group; the host queues the batches
+    // without waiting for each, so one that reported an error stops the rest
+    if (a.stop_on_error && __builtin_amdgcn_readfirstlane((int)ld(&a.metrics->error_flags)) != 0) return;
     const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     c.t_round = now_ticks();
     load_tx(c, a, a.slot_lo + gtid / G, c.t_round);

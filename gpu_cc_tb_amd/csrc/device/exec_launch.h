@@ -2,6 +2,8 @@
 // instantiation per lanes-per-transaction G in {1, 2, 4, 8, 16, 32} and per
 // form (plain per-batch / persistent).
 #pragma once
+#include <atomic>
+
 #include "exec_core.h"
 #include "launch.h"
 
@@ -31,9 +33,15 @@ hipError_t launch_one(const ExecArgs& a, uint64_t nslots, int threads, hipStream
     int per_cu = 0, cus = 0, dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
+    // a constant of the kernel and the block size (0: not asked for yet)
+    static std::atomic<int> occupancy[MAXT / 32 + 1];
+    std::atomic<int>& known = occupancy[(threads + 31) / 32];
+    per_cu = known.load(std::memory_order_relaxed);
+    if (e == hipSuccess && per_cu == 0) {
       e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&txn_exec<S, G, P, MAXT>),
                                                        threads, 0);
+      if (e == hipSuccess) known.store(per_cu, std::memory_order_relaxed);
+    }
     if (e != hipSuccess) return e;
     uint64_t resident = (uint64_t)(per_cu > 0 ? per_cu : 1) * (uint64_t)(cus > 0 ? cus : 1);
     // The open form runs beside the admission copies and preparation kernels
@@ -58,6 +66,7 @@ hipError_t launch_exec_g(int G, const ExecArgs& args, uint64_t nslots, int threa
   if (threads <= 0 || threads > 1024) return hipErrorInvalidValue;
   ExecArgs a = args;
   a.persist = persist ? 1u : 0u;
+  a.stop_on_error = !persist && a.slot_lo > 0;
   if (persist) a.young_ticks = 0;  // a stream has no young phase
   // persistent launches of at most 256 threads per block take the
   // instantiation bounded by that block size (more registers, no spills);

@@ -43,7 +43,6 @@ hipError_t probe(const IndexView& ix, const uint64_t* ops, uint64_t n, uint32_t*
 
 // --- per-op helpers ---
 hipError_t op_tx(const uint64_t* tx_off, uint64_t ntx, uint32_t* op_tx, hipStream_t s);
-hipError_t iota_u32(uint32_t* v, uint64_t n, uint32_t base, hipStream_t s);
 // out[i] = (base + i) | OPID_WRITE if ops[base + i] writes: the values the
 // GaccO / GPUTx sorts carry, so later passes read the flag in order.
 hipError_t op_ids(const uint64_t* ops, uint64_t n, uint32_t base, uint32_t* out, hipStream_t s);
@@ -60,6 +59,10 @@ uint64_t radix_sort_tmp_words(uint64_t n);
 hipError_t radix_sort_u32(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint64_t n,
                           int key_bits, uint32_t* tmp, uint32_t** keys_out, uint32_t** vals_out,
                           hipStream_t s, const uint32_t* nd = nullptr);
+// the same with the positions 0 .. n-1 as values (key_bits > 0): one pass (up to 8
+// bits) only reads k0 and ends in (k1, v1)
+hipError_t radix_sort_ids(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint64_t n, int key_bits,
+                          uint32_t* tmp, uint32_t** keys_out, uint32_t** vals_out, hipStream_t s);
 hipError_t radix_sort_u64(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint64_t n,
                           int key_bits, uint32_t* tmp, uint64_t** keys_out, uint32_t** vals_out,
                           hipStream_t s, const uint32_t* nd = nullptr);
@@ -174,8 +177,8 @@ hipError_t microbench(int which, uint64_t n_words, uint64_t threads_total, uint6
 // map[slot] = the transaction the slot runs: the transactions that write no
 // hot key from slot 0 up, those that do from slot ntx - 1 down (a key is hot
 // when at least one transaction in `share` touches it, estimated from about
-// DEFER_SAMPLE sampled ops).  cnt holds DEFER_WORDS u32: DEFER_BUCKETS
-// sampled counts, then the state words (cnt + DEFER_BUCKETS)[DEFER_ANY] (a
+// DEFER_SAMPLE sampled ops).  cnt holds DEFER_WORDS u32, zero before
+// (run_begin): DEFER_BUCKETS sampled counts, then the state words (cnt + DEFER_BUCKETS)[DEFER_ANY] (a
 // key was hot) and [DEFER_NHOT] (the number deferred); map holds ntx u32.
 constexpr uint32_t DEFER_BUCKETS = 1u << DEFER_BUCKET_BITS;
 constexpr uint64_t DEFER_SAMPLE = 16384;
@@ -193,6 +196,18 @@ uint32_t defer_threshold(uint64_t ntx, uint64_t nops, uint32_t share);
 hipError_t reset_rows(const uint32_t* rows, uint64_t n, uint64_t nrows_table, uint64_t* cc,
                       uint32_t* vprev, hipStream_t s, bool latch = false);
 hipError_t batch_begin(uint64_t* ctrs, hipStream_t s);
+// Start of a run: clear the metrics slots (and the deferral's counts, when
+// given) and, with counters, do what batch_begin and persist_begin do.
+hipError_t run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, bool counters, hipStream_t s);
+// End of a run: what the host reports of it, written into host memory
+// (pinned, read after the stream is waited for).  conflicts, combined and
+// defer (the deferral's state words) may be null.
+struct RunResult {
+  Metrics metrics;  // sums over the slots (error_flags: or)
+  uint64_t conflicts, combined, deferred;
+};
+hipError_t run_end(const Metrics* metrics, const uint64_t* conflicts, const uint64_t* combined, const uint32_t* defer,
+                   RunResult* out, hipStream_t s);
 // admission state of a persistent launch (slot counter, gates, admission words)
 hipError_t persist_begin(uint64_t* ctrs, hipStream_t s);
 // *out = the device wall clock (100 MHz), written by a one-block kernel

@@ -208,11 +208,6 @@ __global__ void k_op_ids(const uint64_t* ops, uint64_t n, uint32_t base, uint32_
        i += (uint64_t)gridDim.x * blockDim.x)
     out[i] = (base + (uint32_t)i) | (op_is_write(ops[base + i]) ? OPID_WRITE : 0u);
 }
-__global__ void k_iota(uint32_t* v, uint64_t n, uint32_t base) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x)
-    v[i] = base + (uint32_t)i;
-}
 __global__ void k_fill32(uint32_t* v, uint64_t n, uint32_t x) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * blockDim.x)
@@ -350,7 +345,7 @@ __global__ __launch_bounds__(RS_BT) void k_rs_scatter(const KT* kin, const uint3
   for (int i = 0; i < RS_ITEMS; ++i) {
     const uint32_t e = wave * RS_WSPAN + i * 64 + lane;
     k[i] = e < cnt ? kin[base + e] : (KT)0;
-    v[i] = e < cnt ? vin[base + e] : 0u;
+    v[i] = e >= cnt ? 0u : vin ? vin[base + e] : (uint32_t)(base + e);  // no values: the positions
   }
   __syncthreads();
   // rank within (wave, digit): earlier items of the wave, then lower lanes
@@ -563,7 +558,7 @@ hipError_t scan_impl(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tm
 
 template <class KT, int ITEMS>
 hipError_t radix_impl(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, int key_bits,
-                      uint32_t* tmp, KT** kout, uint32_t** vout, const uint32_t* nd, hipStream_t s) {
+                      uint32_t* tmp, KT** kout, uint32_t** vout, const uint32_t* nd, hipStream_t s, bool ids = false) {
   KT* ka = k0;
   uint32_t* va = v0;
   KT* kb = k1;
@@ -580,7 +575,8 @@ hipError_t radix_impl(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, in
       hipLaunchKernelGGL((k_rs_hist<KT, ITEMS>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, n, shift, dmask, hist, stride, nd);
       hipLaunchKernelGGL(k_rs_rowscan, dim3(dmask + 1), dim3(RS_BT), 0, s, hist, stride, totals,
                          (uint32_t)(RS_BT * ITEMS), nd);
-      hipLaunchKernelGGL((k_rs_scatter<KT, ITEMS>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, va, kb, vb, n, shift, width,
+      hipLaunchKernelGGL((k_rs_scatter<KT, ITEMS>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka,
+                         ids && p == 0 ? (const uint32_t*)nullptr : va, kb, vb, n, shift, width,
                          hist, stride, totals, nd);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
@@ -1397,25 +1393,70 @@ __global__ void k_reset_rows(const uint32_t* rows, uint64_t n, uint64_t nrows_ta
     if (vprev) dev::st32(vprev + w, 0);
   }
 }
-__global__ void k_batch_begin(uint64_t* ctrs) {
-  if (threadIdx.x == 0) {
+// Start of a run: metrics (and the hot-key counts of a persistent run) to
+// zero, and, with `counters`, what k_batch_begin and k_persist_begin set.
+__device__ __forceinline__ void reset_batch(uint64_t* ctrs) {
+  const int i = threadIdx.x;
+  if (i == 0) {
     dev::st(ctrs + CTR_TICKET, 0);  // commit tickets
     dev::st(ctrs + CTR_POOL, 0);    // MVCC pool bump pointer
     dev::st(ctrs + CTR_T0, wall_clock64());
-    // timestamp allocators restart at 1 (timestamp.cuh:76-80)
-    for (int s = 0; s < TS_SHARDS; ++s) dev::st(ctrs + CTR_TS0 + 16 * s, 1);
   }
+  // timestamp allocators restart at 1 (timestamp.cuh:76-80)
+  if (i < TS_SHARDS) dev::st(ctrs + CTR_TS0 + 16 * i, 1);
 }
-
-// Admission state of one persistent launch: slot counter, gate copies and
-// (open form) admission words.
-__global__ void k_persist_begin(uint64_t* ctrs) {
+__device__ __forceinline__ void reset_admission(uint64_t* ctrs) {
   const int i = threadIdx.x;
   if (i == 0) dev::st(ctrs + CTR_SLOT, 0);
   if (i < GATE_SHARDS) {
     dev::st(ctrs + CTR_GATE0 + 16 * i + 1, 0);
     dev::st(ctrs + CTR_GATE0 + 16 * i + 2, 0);
     dev::st(ctrs + CTR_ADMIT0 + 16 * i, 0);  // the u32 admission word and its neighbour
+  }
+}
+__global__ void k_batch_begin(uint64_t* ctrs) { reset_batch(ctrs); }
+__global__ void k_persist_begin(uint64_t* ctrs) { reset_admission(ctrs); }
+__global__ void k_run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, int counters) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+  for (uint32_t k = i; k < (uint32_t)METRIC_SLOTS * METRICS_WORDS; k += step) metrics[k] = 0;
+  if (defer)
+    for (uint32_t k = i; k < (uint32_t)launch::DEFER_WORDS; k += step) defer[k] = 0;
+  if (counters && blockIdx.x == 0) {
+    reset_batch(ctrs);
+    reset_admission(ctrs);
+  }
+}
+// End of a run: the metrics slots' totals, GPUTx's conflicts, the ops run by
+// combiners and the deferral's state words, into host memory, so that the
+// host reads them after its one wait for the stream and no copy follows.
+__global__ __launch_bounds__(METRIC_SLOTS) void k_run_end(const Metrics* metrics, const uint64_t* conflicts,
+                                                          const uint64_t* combined, const uint32_t* defer,
+                                                          launch::RunResult* out) {
+  constexpr int F = 10;  // Metrics fields in use
+  __shared__ unsigned long long sum[F];
+  const uint32_t t = threadIdx.x;
+  if (t < F) sum[t] = 0;
+  __syncthreads();
+  const uint64_t* m = reinterpret_cast<const uint64_t*>(metrics + t);
+#pragma unroll
+  for (int f = 0; f < F; ++f) {
+    const uint64_t v = m[f];
+    if (!v) continue;
+    if (f == 9)
+      atomicOr(&sum[f], (unsigned long long)v);  // error_flags
+    else
+      atomicAdd(&sum[f], (unsigned long long)v);
+  }
+  __syncthreads();
+  uint64_t* o = reinterpret_cast<uint64_t*>(&out->metrics);
+  if (t < F) dev::st(o + t, sum[t]);
+  if (t == 0) {
+    uint64_t c = 0;
+    if (conflicts)
+      for (uint32_t i = 0; i < launch::CONFLICT_SLOTS; ++i) c += conflicts[16 * i];
+    dev::st(&out->conflicts, c);
+    dev::st(&out->combined, combined ? *combined : 0);
+    dev::st(&out->deferred, defer && defer[launch::DEFER_ANY] ? defer[launch::DEFER_NHOT] : 0);
   }
 }
 
@@ -1439,7 +1480,7 @@ __global__ void k_clock_sample(uint64_t* out) {
 // sampled access counts per bucket; the lanes of a wave that share a bucket
 // add together (one atomic per distinct bucket of the wave)
 __global__ __launch_bounds__(BT) void k_defer_count(const uint64_t* ops, uint64_t nsamp, uint64_t stride,
-                                                    uint32_t* cnt) {
+                                                    uint32_t* cnt, uint32_t thr, uint32_t* st) {
   for (uint64_t base = (uint64_t)blockIdx.x * BT; base < nsamp; base += (uint64_t)gridDim.x * BT) {
     const uint64_t i = base + threadIdx.x;
     const bool v = i < nsamp;
@@ -1449,16 +1490,13 @@ __global__ __launch_bounds__(BT) void k_defer_count(const uint64_t* ops, uint64_
       const int l = __ffsll((unsigned long long)act) - 1;
       const uint32_t lb = dev::shfl32(b, l);
       const uint64_t same = dev::ballot(b == lb) & act;
-      if ((int)dev::lane_id() == l) atomicAdd(cnt + lb, (uint32_t)__popcll(same));
+      if ((int)dev::lane_id() == l) {
+        const uint32_t add = (uint32_t)__popcll(same), old = atomicAdd(cnt + lb, add);
+        if (old < thr && old + add >= thr) st[launch::DEFER_ANY] = 1u;  // the add that makes the bucket hot
+      }
       act &= ~same;
     }
   }
-}
-
-// any bucket hot?  (st was cleared with the counts; every hit writes 1)
-__global__ __launch_bounds__(BT) void k_defer_any(const uint32_t* cnt, uint32_t thr, uint32_t* st) {
-  const uint32_t i = blockIdx.x * BT + threadIdx.x;
-  if (i < launch::DEFER_BUCKETS && cnt[i] >= thr) st[launch::DEFER_ANY] = 1u;
 }
 
 // map[slot] = transaction.  Nothing hot: the identity.  Otherwise a
@@ -1544,9 +1582,6 @@ hipError_t probe(const IndexView& ix, const uint64_t* ops, uint64_t n, uint32_t*
 hipError_t op_tx(const uint64_t* tx_off, uint64_t ntx, uint32_t* op_tx, hipStream_t s) {
   GC_LAUNCH(k_op_tx, ntx, tx_off, ntx, op_tx);
 }
-hipError_t iota_u32(uint32_t* v, uint64_t n, uint32_t base, hipStream_t s) {
-  GC_LAUNCH(k_iota, n, v, n, base);
-}
 hipError_t op_ids(const uint64_t* ops, uint64_t n, uint32_t base, uint32_t* out, hipStream_t s) {
   GC_LAUNCH(k_op_ids, n, ops, n, base, out);
 }
@@ -1564,15 +1599,11 @@ hipError_t defer_order(const uint64_t* tx_off, const uint64_t* ops, uint64_t ntx
   const uint64_t nsamp = nops / stride;
   const uint32_t thr = defer_threshold(ntx, nops, share);
   uint32_t* st = cnt + DEFER_BUCKETS;
-  hipLaunchKernelGGL(k_fill32, dim3(grid_stride_blocks(DEFER_WORDS)), dim3(BT), 0, s, cnt, (uint64_t)DEFER_WORDS, 0u);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
   if (nsamp) {
-    hipLaunchKernelGGL(k_defer_count, dim3(grid_stride_blocks(nsamp)), dim3(BT), 0, s, ops, nsamp, stride, cnt);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_defer_count, dim3(grid_stride_blocks(nsamp)), dim3(BT), 0, s, ops, nsamp, stride, cnt, thr, st);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k_defer_any, dim3(DEFER_BUCKETS / BT), dim3(BT), 0, s, cnt, thr, st);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(k_defer_order, dim3(reduce_blocks(ntx)), dim3(BT), 0, s, tx_off, ops, ntx, cnt, thr, st, map);
   return hipGetLastError();
 }
@@ -1587,6 +1618,16 @@ hipError_t radix_sort_u32(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1
                           int key_bits, uint32_t* tmp, uint32_t** keys_out, uint32_t** vals_out,
                           hipStream_t s, const uint32_t* nd) {
   return radix_sort<uint32_t>(k0, v0, k1, v1, n, key_bits, tmp, keys_out, vals_out, nd, s);
+}
+hipError_t radix_sort_ids(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint64_t n, int key_bits,
+                          uint32_t* tmp, uint32_t** keys_out, uint32_t** vals_out, hipStream_t s) {
+  if (n == 1) {
+    const hipError_t e = fill_u32(v0, 1, 0, s);
+    if (e != hipSuccess) return e;
+  }
+  return n <= RS_SHORT_MAX
+             ? radix_impl<uint32_t, RS_SHORT>(k0, v0, k1, v1, n, key_bits, tmp, keys_out, vals_out, nullptr, s, true)
+             : radix_impl<uint32_t, RS_LONG>(k0, v0, k1, v1, n, key_bits, tmp, keys_out, vals_out, nullptr, s, true);
 }
 hipError_t radix_sort_u64(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, uint64_t n,
                           int key_bits, uint32_t* tmp, uint64_t** keys_out, uint32_t** vals_out,
@@ -1711,6 +1752,15 @@ hipError_t row_base_add(const uint32_t* srow, const uint32_t* rstart, uint64_t n
                         hipStream_t s) {
   if (n == 0) return hipSuccess;
   GC_LAUNCH(k_row_base_add, n, srow, rstart, n, nrows, base);
+}
+hipError_t run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, bool counters, hipStream_t s) {
+  hipLaunchKernelGGL(k_run_begin, dim3(defer ? 64 : 16), dim3(BT), 0, s, metrics, defer, ctrs, counters ? 1 : 0);
+  return hipGetLastError();
+}
+hipError_t run_end(const Metrics* metrics, const uint64_t* conflicts, const uint64_t* combined, const uint32_t* defer,
+                   RunResult* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_run_end, dim3(1), dim3(METRIC_SLOTS), 0, s, metrics, conflicts, combined, defer, out);
+  return hipGetLastError();
 }
 hipError_t persist_begin(uint64_t* ctrs, hipStream_t s) {
   hipLaunchKernelGGL(k_persist_begin, dim3(1), dim3(64), 0, s, ctrs);

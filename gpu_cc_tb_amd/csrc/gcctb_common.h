@@ -323,6 +323,7 @@ struct ExecArgs {
   uint64_t persist_groups; // persistent form: at most this many transactions in flight (0 = device-filling)
   uint32_t open;           // persistent form: slots are admitted while the launch runs (CTR_ADMIT0)
   uint32_t persist;        // 1 in persistent launches (slots from CTR_SLOT, gates, urgent state)
+  uint32_t stop_on_error;  // plain launches after the first: do nothing once an earlier one reported an error
   uint32_t urgent_attempts; // persistent form: aborts that make a transaction urgent (0 = never)
   uint32_t backoff_exp;     // retry delay spans at most 2^backoff_exp units
   uint32_t young_ticks;     // plain form: until this long after CTR_T0 it spans at most 4 units (young_ticks())

@@ -91,6 +91,9 @@ int latch_scheme_from_name(const char* s) {
 
 class SchemeHost;
 
+constexpr uint64_t RANK_PINNED = 1024;   // per-rank counts copied through pinned memory
+constexpr size_t PLAIN_EVENTS = 256;     // plain form: batches queued before the host waits
+
 }  // namespace gcctb
 
 struct gcctb_ctx {
@@ -124,6 +127,11 @@ struct gcctb_ctx {
   // pinned host word: the error flags of the launches since the last metrics
   // clear, copied behind each launch so the host sees them at its sync
   uint64_t* h_err = nullptr;
+  gcctb::launch::RunResult* h_run = nullptr;  // pinned: what a run's last kernel reports
+  uint32_t* h_rank = nullptr;  // pinned: GPUTx's highest rank, then the first RANK_PINNED per-rank counts
+  double wall_khz = 0;         // rate of the device's wall clock
+  // per-batch events of the plain form, at most 2 * PLAIN_EVENTS
+  std::vector<hipEvent_t> pev;
   // table + index
   gcctb::DevBuf<uint64_t> cells;
   gcctb::DevBuf<uint32_t> buckets;  // hash index
@@ -158,7 +166,7 @@ struct gcctb_ctx {
   gcctb::DevBuf<uint8_t> ord_map;
   gcctb::DevBuf<uint32_t> ord_bits, ord_count, ord_row, ord_op, ord_tx;
   gcctb::DevBuf<uint64_t> ord_flags;
-  gcctb::DevBuf<uint32_t> rank, tx_map, max_rank;
+  gcctb::DevBuf<uint32_t> rank, tx_map, max_rank, rank_hist;
   // hot-writer deferral: sampled counts and state, slot -> transaction map;
   // in use while defer_active
   gcctb::DevBuf<uint32_t> defer_cnt, defer_map;
@@ -223,7 +231,8 @@ class SchemeHost {
   }
   // Persistent form: prepare the whole stream as one unit (no per-batch
   // resets: timestamps and tickets keep counting across batch boundaries).
-  virtual void PrepStream() { HIP_TRY(launch::batch_begin(ctx.ctrs.p, ctx.stream)); }
+  // run_begin has reset the counters and the admission state.
+  virtual void PrepStream() {}
   // Persistent form: restore the words every transaction of the stream touched.
   virtual void PostStream() { Post(0, 0, ctx.ntx); }
   // Serving form: prepare one launch over transactions whose ops are [o0, o1).
@@ -270,8 +279,8 @@ class SchemeHost {
   }
   // Device allocations of the scheme (GetMemSize, include/cc.cuh:39).
   virtual uint64_t GetMemSize() const { return ctx.cc.n * 8; }
-  // ops that row combiners ran in the last persistent pass (GaccO)
-  virtual uint64_t Combined() const { return 0; }
+  // device count of the ops that row combiners ran in the last persistent pass (GaccO; null: none)
+  virtual const uint64_t* Combined() const { return nullptr; }
   std::vector<uint64_t> batches;
 
  protected:
@@ -535,12 +544,7 @@ class GaccoHost : public SchemeHost {
   }
   void Post(int, uint64_t, uint64_t) override {}
   uint64_t GetMemSize() const override { return ctx.counters.n * 4 + ctx.need.n * 4; }
-  // ops run by the combiners in the last persistent pass
-  uint64_t Combined() const override {
-    uint64_t v = 0;
-    if (combined_) HIP_TRY(hipMemcpy(&v, ctx.comb_ctr.p + launch::COMB_WORDS / 2, 8, hipMemcpyDeviceToHost));
-    return v;
-  }
+  const uint64_t* Combined() const override { return combined_ ? ctx.comb_ctr.p + launch::COMB_WORDS / 2 : nullptr; }
   bool combined_ = false;
 };
 
@@ -563,12 +567,14 @@ class GPUTxHost : public SchemeHost {
     hipStream_t s = c.stream;
     c.h_rank_counts.assign(c.nranks, 0);
     if (c.nops && c.nranks) {
-      DevBuf<uint32_t> hist;
-      hist.alloc(c.nranks);
-      HIP_TRY(launch::fill_u32(hist.p, c.nranks, 0, s));
-      HIP_TRY(launch::rank_hist(c.rank.p, c.ntx, (uint32_t)c.nranks, hist.p, s));
-      HIP_TRY(hipMemcpyAsync(c.h_rank_counts.data(), hist.p, c.nranks * 4, hipMemcpyDeviceToHost, s));
+      c.rank_hist.alloc(c.nranks);
+      HIP_TRY(launch::fill_u32(c.rank_hist.p, c.nranks, 0, s));
+      HIP_TRY(launch::rank_hist(c.rank.p, c.ntx, (uint32_t)c.nranks, c.rank_hist.p, s));
+      const bool pinned = c.nranks <= RANK_PINNED;
+      HIP_TRY(hipMemcpyAsync(pinned ? c.h_rank + 1 : c.h_rank_counts.data(), c.rank_hist.p, c.nranks * 4,
+                             hipMemcpyDeviceToHost, s));
       HIP_TRY(hipStreamSynchronize(s));
+      if (pinned) std::memcpy(c.h_rank_counts.data(), c.h_rank + 1, c.nranks * 4);
     } else if (c.nranks) {
       // no ops at all: every transaction has rank 0
       c.h_rank_counts[0] = (uint32_t)c.ntx;
@@ -605,19 +611,22 @@ class GPUTxHost : public SchemeHost {
     HIP_TRY(launch::fill_u32(ctx.rank.p, ntx, 0, s));
     HIP_TRY(launch::fill_u32(ctx.max_rank.p, 1, 0, s));
     HIP_TRY(launch::seg_ranks(srow, stx_ops, n, ctx.sort_tmp.p, ctx.cfg.rows, ctx.rank.p, ctx.max_rank.p, s, tx_of, nd));
-    uint32_t max_rank = 0;
-    HIP_TRY(hipMemcpyAsync(&max_rank, ctx.max_rank.p, 4, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(ctx.h_rank, ctx.max_rank.p, 4, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     // no ops at all: every transaction has rank 0
-    ctx.nranks = n ? (uint64_t)max_rank + 1 : (ntx ? 1 : 0);
-    // transactions in (rank, tx) order: stable sort of ranks (include/gputx.cuh:281)
+    ctx.nranks = n ? (uint64_t)*ctx.h_rank + 1 : (ntx ? 1 : 0);
+    // transactions in (rank, tx) order: stable sort of ranks (include/gputx.cuh:281),
+    // whose values are the positions.  One pass (up to 256 ranks) leaves the
+    // keys alone and writes tx_map; more of them sort a copy of the ranks.
     const int rank_bits = std::max(1, bits_for(ctx.nranks ? ctx.nranks - 1 : 0));
-    HIP_TRY(hipMemcpyAsync(ctx.sk0.p, ctx.rank.p, ntx * 4, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(launch::iota_u32(ctx.sv0.p, ntx, 0, s));
-    uint32_t *srank, *stx;
-    HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, ntx, rank_bits, ctx.sort_tmp.p,
-                                   &srank, &stx, s));
-    HIP_TRY(hipMemcpyAsync(ctx.tx_map.p, stx, ntx * 4, hipMemcpyDeviceToDevice, s));
+    {
+      const bool one_pass = rank_bits <= 8;
+      uint32_t *srank, *stx;
+      if (!one_pass) HIP_TRY(hipMemcpyAsync(ctx.sk0.p, ctx.rank.p, ntx * 4, hipMemcpyDeviceToDevice, s));
+      HIP_TRY(launch::radix_sort_ids(one_pass ? ctx.rank.p : ctx.sk0.p, ctx.sv0.p, ctx.sk1.p,
+                                     one_pass ? ctx.tx_map.p : ctx.sv1.p, ntx, rank_bits, ctx.sort_tmp.p, &srank, &stx, s));
+      if (stx != ctx.tx_map.p) HIP_TRY(hipMemcpyAsync(ctx.tx_map.p, stx, ntx * 4, hipMemcpyDeviceToDevice, s));
+    }
     // execution order of every row: (row, rank, tx); 32-bit composite keys
     // when row and rank fit, else 64-bit
     if (!n) return;
@@ -826,6 +835,14 @@ int gcctb_create(const gcctb_config* cfg, gcctb_ctx** out) {
     for (auto& e : c->ev) HIP_TRY(hipEventCreate(&e));
     HIP_TRY(hipHostMalloc((void**)&c->h_err, sizeof(uint64_t), hipHostMallocDefault));
     *c->h_err = 0;
+    HIP_TRY(hipHostMalloc((void**)&c->h_run, sizeof(launch::RunResult), hipHostMallocDefault));
+    if (c->scheme == SCHEME_GPUTX)
+      HIP_TRY(hipHostMalloc((void**)&c->h_rank, (RANK_PINNED + 1) * sizeof(uint32_t), hipHostMallocDefault));
+    {
+      int rate = 0;
+      HIP_TRY(hipDeviceGetAttribute(&rate, hipDeviceAttributeWallClockRate, 0));
+      c->wall_khz = rate;
+    }
     switch (c->scheme) {
       case SCHEME_TPL_NW: c->host.reset(new TwoPLHost(*c, false)); break;
       case SCHEME_TPL_WD: c->host.reset(new TwoPLHost(*c, true)); break;
@@ -856,7 +873,10 @@ void gcctb_destroy(gcctb_ctx* c) {
   c->host.reset();
   for (auto& e : c->ev)
     if (e) (void)hipEventDestroy(e);
+  for (auto& e : c->pev) (void)hipEventDestroy(e);
   if (c->h_err) (void)hipHostFree(c->h_err);
+  if (c->h_run) (void)hipHostFree(c->h_run);
+  if (c->h_rank) (void)hipHostFree(c->h_rank);
   hipStream_t s = c->stream, s2 = c->stream2;
   if (s2) (void)hipStreamSynchronize(s2);
   delete c;  // DevBuf destructors free device memory
@@ -1177,19 +1197,15 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
   Metrics m{};
   try {
     hipStream_t s = c->stream;
-    HIP_TRY(hipMemsetAsync(c->metrics.p, 0, sizeof(Metrics) * METRIC_SLOTS, s));
     if (c->cfg.debug_events) {
       // a fresh log per run: no stamps, the stamp counter at zero
       if (c->nops) HIP_TRY(launch::fill_u64(c->ev_op.p, c->nops, 0, s));
       if (c->ntx) HIP_TRY(launch::fill_u64(c->ev_commit.p, c->ntx, 0, s));
       HIP_TRY(launch::fill_u64(c->ctrs.p + CTR_EVENT, 1, 0, s));
     }
-    HIP_TRY(hipStreamSynchronize(s));
-    *c->h_err = 0;
     float ms = 0;
     double pre = 0, proc = 0;
     uint64_t launches = 0;
-    HIP_TRY(hipEventRecord(c->ev[0], s));
     // hot-writer deferral (lock, timestamp and OCC schemes; the ordered
     // schemes wait on lower slots and keep the stream order)
     const uint32_t share = c->defer_share >= 0                                          ? (uint32_t)c->defer_share
@@ -1199,20 +1215,42 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
                        c->scheme != SCHEME_GPUTX;
     // 2PL with the deferral also locks hot keys last
     const bool hot = defer && c->hot_last && (c->scheme == SCHEME_TPL_NW || c->scheme == SCHEME_TPL_WD);
+    // plain form: batches whose events are not read yet, and the event that
+    // everything accounted for so far lies before
+    size_t queued = 0;
+    hipEvent_t before = c->ev[0];
+    auto settle = [&]() {  // the queued batches have ended
+      for (size_t k = 0; k < queued; ++k) {
+        HIP_TRY(hipEventElapsedTime(&ms, before, c->pev[2 * k]));
+        pre += ms;
+        HIP_TRY(hipEventElapsedTime(&ms, c->pev[2 * k], c->pev[2 * k + 1]));
+        proc += ms;
+        before = c->pev[2 * k + 1];
+      }
+      if (queued) {  // the next round reuses the pool: the last event is kept apart
+        std::swap(c->ev[1], c->pev[2 * queued - 1]);
+        before = c->ev[1];
+      }
+      queued = 0;
+    };
+    *c->h_err = 0;
+    HIP_TRY(hipEventRecord(c->ev[0], s));
+    HIP_TRY(launch::run_begin(reinterpret_cast<uint64_t*>(c->metrics.p), defer ? c->defer_cnt.p : nullptr, c->ctrs.p,
+                              form == FORM_PERSIST, s));
     if (form == FORM_PERSIST) {
       c->host->PrepStream();
       if (defer) {
         HIP_TRY(launch::defer_order(c->tx_off.p, c->ops.p, c->ntx, c->nops, share, c->defer_cnt.p, c->defer_map.p, s));
         c->defer_thr = launch::defer_threshold(c->ntx, c->nops, share);
       }
-      // Rows: GaccO's and GPUTx's preparation already has them; for the
-      // other schemes a probe pass finds every op's row first, or each group
-      // looks its rows up as it takes a transaction (WantsProbePass).
+      // Rows: over a hash index GaccO's and GPUTx's preparation already has
+      // them; for the other schemes a probe pass finds every op's row first,
+      // or each group looks its rows up as it takes a transaction
+      // (WantsProbePass).
       const bool pass = c->probe_pass >= 0 ? c->probe_pass != 0 : c->host->WantsProbePass();
       const bool probed = c->host->ProbesRows() || pass;
       if (!c->host->ProbesRows() && pass && c->nops)
         HIP_TRY(launch::probe(c->ix, c->ops.p, c->nops, c->rows_out.p, s));
-      HIP_TRY(launch::persist_begin(c->ctrs.p, s));
       HIP_TRY(hipEventRecord(c->ev[3], s));
       c->rows_probed = probed;
       c->defer_active = defer;
@@ -1223,15 +1261,6 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
       c->rows_probed = false;
       HIP_TRY(hipEventRecord(c->ev[4], s));
       c->host->PostStream();
-      enqueue_error_copy(*c);
-      HIP_TRY(hipEventRecord(c->ev[5], s));
-      HIP_TRY(hipEventSynchronize(c->ev[5]));
-      HIP_TRY(hipEventElapsedTime(&ms, c->ev[0], c->ev[3]));
-      pre += ms;
-      HIP_TRY(hipEventElapsedTime(&ms, c->ev[4], c->ev[5]));
-      pre += ms;
-      HIP_TRY(hipEventElapsedTime(&ms, c->ev[3], c->ev[4]));
-      proc += ms;
       launches = 1;
     } else if (form == FORM_GRAPH) {
       // Init0 may synchronize with the host (GPUTx ranks): it stays outside
@@ -1267,70 +1296,71 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
       for (uint64_t n : batches) launches += n ? 1 : 0;
       HIP_TRY(hipEventRecord(c->ev[3], s));
       HIP_TRY(hipGraphLaunch(c->graph_exec, s));
-      HIP_TRY(hipEventRecord(c->ev[4], s));
-      HIP_TRY(hipEventSynchronize(c->ev[4]));
+      HIP_TRY(hipEventRecord(c->ev[4], s));  // proc: kernels and per-batch preparation inside the graph
+    } else {
+      // Every batch is queued behind the one before (a launch does nothing
+      // once an earlier one reported an error), and the host waits at the end,
+      // or every PLAIN_EVENTS batches, instead of after each: a wait and the
+      // next batch's launches left the GPU idle for about 25 us a batch.
+      c->host->Init0();
+      uint64_t batch_st = 0;
+      const auto& batches = c->host->batches;
+      for (size_t i = 0; i < batches.size(); ++i) {
+        const uint64_t n = batches[i];
+        if (!n) continue;  // benchmark_cpu/ycsb.cu:266-267
+        while (c->pev.size() < 2 * (queued + 1)) {
+          hipEvent_t e = nullptr;
+          HIP_TRY(hipEventCreate(&e));
+          c->pev.push_back(e);
+        }
+        c->host->Init((int)i, batch_st);
+        HIP_TRY(hipEventRecord(c->pev[2 * queued], s));
+        c->host->Launch((int)i, batch_st, batch_st + n, false);
+        HIP_TRY(hipEventRecord(c->pev[2 * queued + 1], s));
+        c->host->Post((int)i, batch_st, n);
+        batch_st += n;
+        launches++;
+        if (++queued == PLAIN_EVENTS) {
+          enqueue_error_copy(*c);
+          HIP_TRY(hipStreamSynchronize(s));
+          settle();
+          if (*c->h_err) break;  // nothing after the first batch with an error ran
+        }
+      }
+    }
+    const bool stats_defer = defer && c->ntx;
+    HIP_TRY(launch::run_end(c->metrics.p, c->scheme == SCHEME_GPUTX && c->nops ? c->conflicts.p : nullptr,
+                            form == FORM_PERSIST ? c->host->Combined() : nullptr,
+                            stats_defer ? c->defer_cnt.p + launch::DEFER_BUCKETS : nullptr, c->h_run, s));
+    HIP_TRY(hipEventRecord(c->ev[6], s));
+    HIP_TRY(hipEventSynchronize(c->ev[6]));
+    m = c->h_run->metrics;
+    if (form == FORM_PLAIN) {
+      settle();
+      HIP_TRY(hipEventElapsedTime(&ms, before, c->ev[6]));
+      pre += ms;
+    } else {
       HIP_TRY(hipEventElapsedTime(&ms, c->ev[0], c->ev[3]));
       pre += ms;
-      HIP_TRY(hipEventElapsedTime(&ms, c->ev[3], c->ev[4]));
-      proc += ms;  // kernels and per-batch preparation inside the graph
-    } else {
-    c->host->Init0();
-    HIP_TRY(hipEventRecord(c->ev[1], s));
-    HIP_TRY(hipEventSynchronize(c->ev[1]));
-    HIP_TRY(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]));
-    pre += ms;
-    uint64_t batch_st = 0;
-    const auto& batches = c->host->batches;
-    for (size_t i = 0; i < batches.size(); ++i) {
-      const uint64_t n = batches[i];
-      if (!n) continue;  // benchmark_cpu/ycsb.cu:266-267
-      HIP_TRY(hipEventRecord(c->ev[2], s));
-      c->host->Init((int)i, batch_st);
-      HIP_TRY(hipEventRecord(c->ev[3], s));
-      c->host->Launch((int)i, batch_st, batch_st + n, false);
-      HIP_TRY(hipEventRecord(c->ev[4], s));
-      c->host->Post((int)i, batch_st, n);
-      enqueue_error_copy(*c);
-      HIP_TRY(hipEventRecord(c->ev[5], s));
-      HIP_TRY(hipEventSynchronize(c->ev[5]));
-      HIP_TRY(hipEventElapsedTime(&ms, c->ev[2], c->ev[3]));
-      pre += ms;
-      HIP_TRY(hipEventElapsedTime(&ms, c->ev[4], c->ev[5]));
+      HIP_TRY(hipEventElapsedTime(&ms, c->ev[4], c->ev[6]));
       pre += ms;
       HIP_TRY(hipEventElapsedTime(&ms, c->ev[3], c->ev[4]));
       proc += ms;
-      batch_st += n;
-      launches++;
-      if (*c->h_err) break;  // the first batch that reported an error ends the run
     }
-    }
-    HIP_TRY(hipEventRecord(c->ev[6], s));
-    HIP_TRY(hipEventSynchronize(c->ev[6]));
     HIP_TRY(hipEventElapsedTime(&ms, c->ev[0], c->ev[6]));
     st.tot_ms = ms;
     st.pre_ms = pre;
     st.proc_ms = proc;
     st.exec_kernel_ms = proc;
     st.batches = launches;
-    m = collect_metrics(c);
     if (m.error_flags) clear_cc_state(*c);
     if (c->scheme == SCHEME_GPUTX) {
       st.ranks = c->nranks;
-      if (c->nops) {
-        uint64_t slot[16 * launch::CONFLICT_SLOTS];
-        HIP_TRY(hipMemcpy(slot, c->conflicts.p, sizeof slot, hipMemcpyDeviceToHost));
-        for (uint32_t i = 0; i < launch::CONFLICT_SLOTS; ++i) st.same_rank_conflicts += slot[16 * i];
-      }
+      st.same_rank_conflicts = c->h_run->conflicts;
     }
-    if (form == FORM_PERSIST) st.combined = c->host->Combined();
-    if (defer && c->ntx) {
-      uint32_t dst[3] = {0, 0, 0};
-      HIP_TRY(hipMemcpy(dst, c->defer_cnt.p + launch::DEFER_BUCKETS, sizeof dst, hipMemcpyDeviceToHost));
-      st.deferred = dst[launch::DEFER_ANY] ? dst[launch::DEFER_NHOT] : 0;
-    }
-    int rate = 0;
-    HIP_TRY(hipDeviceGetAttribute(&rate, hipDeviceAttributeWallClockRate, 0));
-    st.tick_khz = rate;
+    st.combined = c->h_run->combined;
+    st.deferred = c->h_run->deferred;
+    st.tick_khz = c->wall_khz;
     if ((m.error_flags & ERR_WATCHDOG) && c->dbg.p) {
       std::vector<uint64_t> d(c->dbg.n);
       HIP_TRY(hipMemcpy(d.data(), c->dbg.p, d.size() * 8, hipMemcpyDeviceToHost));
