@@ -82,12 +82,40 @@ hipError_t scratch_ptr(uint64_t** out) {
   return hipSuccess;
 }
 
-// Row of every op when keys are row ids (Find(k) == k for the reference's
-// identity id column, benchmark_cpu/ycsb.cu:59): key < rows, else a miss.
-__global__ void k_identity_rows(const uint64_t* ops, uint64_t n, uint64_t rows, uint32_t* rows_out) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+// Start of a call: the row of every op (keys are row ids: Find(k) == k for the
+// reference's identity id column, benchmark_cpu/ycsb.cu:59; key < rows, else a
+// miss) and everything that must start at zero, in one launch: the words of
+// the rows that the ops name where those are few (`sparse`, the line that
+// launch::reset_rows draws), else all of them, and as many version nodes as
+// there can be writes.  A small call is launch latency alone: Silo with 40
+// transactions of 16 ops 10 launches and copies and 2 waits, 80 us; now 3
+// launches, 1 copy and 1 wait, 40 us.
+__global__ __launch_bounds__(256) void k_static_begin(const uint64_t* ops, uint64_t n, uint64_t rows, uint32_t shift,
+                                                      uint32_t* rows_out, uint64_t* cc, uint64_t cc_words,
+                                                      uint32_t* vprev, uint64_t* pool, uint64_t pool_words, int sparse,
+                                                      uint64_t* ctrs, uint64_t* metrics) {
+  const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t i = i0; i < n; i += step) {
     const uint32_t k = op_key(ops[i]);
-    rows_out[i] = (uint64_t)k < rows ? k : IDX_MISS;
+    const bool hit = (uint64_t)k < rows;
+    rows_out[i] = hit ? k : IDX_MISS;
+    if (sparse && hit) {
+      const uint32_t w = row_slot(k, shift);
+      cc[w] = 0;
+      if (vprev) vprev[w] = 0;
+    }
+  }
+  if (!sparse)
+    for (uint64_t i = i0; i < cc_words; i += step) {
+      cc[i] = 0;
+      if (vprev) vprev[i] = 0;
+    }
+  for (uint64_t i = i0; i < pool_words; i += step) pool[i] = 0;
+  for (uint64_t i = i0; i < (uint64_t)METRIC_SLOTS * METRICS_WORDS; i += step) metrics[i] = 0;
+  // the counters, as launch::batch_begin leaves them, come last
+  for (uint64_t i = i0; i < (uint64_t)CTR_WORDS; i += step) {
+    const bool ts = i >= (uint64_t)CTR_TS0 && i < (uint64_t)(CTR_TS0 + 16 * TS_SHARDS) && (i - CTR_TS0) % 16 == 0;
+    ctrs[i] = ts ? 1 : i == (uint64_t)CTR_T0 ? wall_clock64() : 0;
   }
 }
 
@@ -119,29 +147,6 @@ hipError_t launch_exec(int scheme, int G, const ExecArgs& a, uint64_t n, int thr
     case SCHEME_TICTOC: return launch::exec_tictoc(G, a, n, threads, false, s);
     default: return hipErrorInvalidValue;
   }
-}
-
-// Read the metrics slots (fixed host buffer on the stack) and sum them.
-Metrics sum_metrics(const uint64_t* dev_metrics, hipStream_t s) {
-  uint64_t slots[METRIC_SLOTS * METRICS_WORDS];
-  NA_TRY(hipMemcpyAsync(slots, dev_metrics, sizeof(slots), hipMemcpyDeviceToHost, s));
-  NA_TRY(hipStreamSynchronize(s));
-  Metrics m{};
-  for (int i = 0; i < METRIC_SLOTS; ++i) {
-    Metrics x;
-    std::memcpy(&x, slots + (uint64_t)i * METRICS_WORDS, sizeof(Metrics));
-    m.abort += x.abort;
-    m.ts_duration += x.ts_duration;
-    m.wait_duration += x.wait_duration;
-    m.abort_duration += x.abort_duration;
-    m.manager_duration += x.manager_duration;
-    m.tot_duration += x.tot_duration;
-    m.index_duration += x.index_duration;
-    m.committed += x.committed;
-    m.index_miss += x.index_miss;
-    m.error_flags |= x.error_flags;
-  }
-  return m;
 }
 
 }  // namespace
@@ -182,20 +187,17 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
     uint32_t* aborts = reinterpret_cast<uint32_t*>(base + OFF_ABORTS);
     uint64_t* ctrs = base + OFF_CTRS;
     uint64_t* metrics = base + OFF_METRICS;
-    // The array keeps the last call's contents: clear what must start at
-    // zero (fill kernels, which stream capture records as kernel nodes).
-    // per-row state sits at each row's slot (slot_words(rows) <= NA_MAX_ROWS)
+    // The array keeps the last call's contents: clear what must start at zero
+    // (per-row state sits at each row's slot; slot_words(rows) <= NA_MAX_ROWS).
     const uint64_t words = slot_words(r->rows);
-    NA_TRY(launch::fill_u64(cc, words, 0, s));
-    if (sch == SCHEME_MVCC) {
-      NA_TRY(launch::fill_u32(vprev, words, 0, s));
-      NA_TRY(launch::fill_u64(pool, 3 * NA_POOL_NODES, 0, s));
-    }
-    NA_TRY(launch::fill_u64(ctrs, CTR_WORDS, 0, s));
-    NA_TRY(launch::fill_u64(metrics, (uint64_t)METRIC_SLOTS * METRICS_WORDS, 0, s));
-    if (r->nops) {
-      const unsigned blocks = (unsigned)std::min<uint64_t>((r->nops + 255) / 256, 4096);
-      hipLaunchKernelGGL(k_identity_rows, dim3(blocks), dim3(256), 0, s, r->ops, r->nops, r->rows, rows);
+    const bool mvcc = sch == SCHEME_MVCC;
+    const bool sparse = r->nops * 8 < r->rows;
+    const uint64_t pool_words = mvcc ? 3 * std::min<uint64_t>(NA_POOL_NODES, r->nops) : 0;
+    {
+      const uint64_t most = std::max({r->nops, sparse ? 0 : words, pool_words, (uint64_t)METRIC_SLOTS * METRICS_WORDS});
+      const unsigned blocks = (unsigned)std::min<uint64_t>((most + 255) / 256, 4096);
+      hipLaunchKernelGGL(k_static_begin, dim3(blocks), dim3(256), 0, s, r->ops, r->nops, r->rows, slot_shift(r->rows), rows,
+                         cc, words, mvcc ? vprev : nullptr, pool, pool_words, sparse ? 1 : 0, ctrs, metrics);
       NA_TRY(hipGetLastError());
     }
     ExecArgs a{};
@@ -234,10 +236,12 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
     const int G = 1 << r->warp_density;
     const int threads = r->block_size * 32;
     // Per batch: reset the counters, one launch, restore the touched words
-    // (benchmark_cpu/ycsb.cu:262-285), stop on the first batch with an error.
-    // The host learns the row offsets of a batch from nothing but the op
-    // count, so the restore clears the rows of every op (<= rows / 8 ops:
-    // those rows; more: the whole arrays).
+    // (benchmark_cpu/ycsb.cu:262-285).  The batches are queued one behind the
+    // other (a launch does nothing once an earlier one reported an error) and
+    // the host waits once.  The host learns the row offsets of a batch from
+    // nothing but the op count, so the restore clears the rows of every op
+    // (<= rows / 8 ops: those rows; more: the whole arrays); after the last
+    // batch nothing reads the words before the next call clears them.
     uint64_t b = 0;
     for (uint64_t st0 = 0; st0 < r->ntx; st0 += r->batch_size, ++b) {
       const uint64_t n = std::min<uint64_t>(r->batch_size, r->ntx - st0);
@@ -245,23 +249,21 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
       a.slot_lo = st0;
       a.slot_hi = st0 + n;
       a.young_ticks = young_ticks(n);
-      NA_TRY(launch::batch_begin(ctrs, s));
+      if (b) {
+        if (sch != SCHEME_TPL_NW && sch != SCHEME_TPL_WD)
+          NA_TRY(launch::reset_rows(rows, r->nops, r->rows, cc, mvcc ? vprev : nullptr, s));
+        NA_TRY(launch::batch_begin(ctrs, s));
+      }
       NA_TRY(launch_exec(sch, G, a, n, threads, s));
-      if (sch != SCHEME_TPL_NW && sch != SCHEME_TPL_WD)
-        NA_TRY(launch::reset_rows(rows, r->nops, r->rows, cc, sch == SCHEME_MVCC ? vprev : nullptr, s));
-      uint64_t flags = 0;
-      NA_TRY(hipMemcpyAsync(&flags, &reinterpret_cast<Metrics*>(metrics)->error_flags, 8, hipMemcpyDeviceToHost, s));
-      NA_TRY(hipStreamSynchronize(s));
       ++launches;
-      if (flags) break;
     }
-    m = sum_metrics(metrics, s);
-    if (m.error_flags) {
-      // a stopped launch can leave locks or marks behind: clear them all
-      NA_TRY(launch::fill_u64(cc, words, 0, s));
-      if (sch == SCHEME_MVCC) NA_TRY(launch::fill_u32(vprev, words, 0, s));
-      NA_TRY(hipStreamSynchronize(s));
-    }
+    // the totals into the first slots, then to the host
+    launch::RunResult res;
+    NA_TRY(launch::run_end(reinterpret_cast<Metrics*>(metrics), nullptr, nullptr, nullptr,
+                           reinterpret_cast<launch::RunResult*>(metrics), s));
+    NA_TRY(hipMemcpyAsync(&res, metrics, sizeof res, hipMemcpyDeviceToHost, s));
+    NA_TRY(hipStreamSynchronize(s));
+    m = res.metrics;
   } catch (const NaFail& f) {
     return set_error(GCCTB_EDEVICE, std::string("HIP error: ") + hipGetErrorString(f.err) + " in " + f.where);
   }

@@ -93,6 +93,12 @@ class SchemeHost;
 
 constexpr uint64_t RANK_PINNED = 1024;   // per-rank counts copied through pinned memory
 constexpr size_t PLAIN_EVENTS = 256;     // plain form: batches queued before the host waits
+// the context's pinned host memory, one allocation
+struct PinnedWords {
+  uint64_t err;
+  launch::RunResult run;
+  uint32_t rank[RANK_PINNED + 1];
+};
 
 }  // namespace gcctb
 
@@ -126,6 +132,7 @@ struct gcctb_ctx {
   hipEvent_t ev[8] = {};
   // pinned host word: the error flags of the launches since the last metrics
   // clear, copied behind each launch so the host sees them at its sync
+  gcctb::PinnedWords* pinned = nullptr;
   uint64_t* h_err = nullptr;
   gcctb::launch::RunResult* h_run = nullptr;  // pinned: what a run's last kernel reports
   uint32_t* h_rank = nullptr;  // pinned: GPUTx's highest rank, then the first RANK_PINNED per-rank counts
@@ -833,11 +840,11 @@ int gcctb_create(const gcctb_config* cfg, gcctb_ctx** out) {
     HIP_TRY(hipSetDevice(0));
     HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     for (auto& e : c->ev) HIP_TRY(hipEventCreate(&e));
-    HIP_TRY(hipHostMalloc((void**)&c->h_err, sizeof(uint64_t), hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void**)&c->pinned, sizeof(gcctb::PinnedWords), hipHostMallocDefault));
+    c->h_err = &c->pinned->err;
     *c->h_err = 0;
-    HIP_TRY(hipHostMalloc((void**)&c->h_run, sizeof(launch::RunResult), hipHostMallocDefault));
-    if (c->scheme == SCHEME_GPUTX)
-      HIP_TRY(hipHostMalloc((void**)&c->h_rank, (RANK_PINNED + 1) * sizeof(uint32_t), hipHostMallocDefault));
+    c->h_run = &c->pinned->run;
+    c->h_rank = c->pinned->rank;
     {
       int rate = 0;
       HIP_TRY(hipDeviceGetAttribute(&rate, hipDeviceAttributeWallClockRate, 0));
@@ -874,9 +881,7 @@ void gcctb_destroy(gcctb_ctx* c) {
   for (auto& e : c->ev)
     if (e) (void)hipEventDestroy(e);
   for (auto& e : c->pev) (void)hipEventDestroy(e);
-  if (c->h_err) (void)hipHostFree(c->h_err);
-  if (c->h_run) (void)hipHostFree(c->h_run);
-  if (c->h_rank) (void)hipHostFree(c->h_rank);
+  if (c->pinned) (void)hipHostFree(c->pinned);
   hipStream_t s = c->stream, s2 = c->stream2;
   if (s2) (void)hipStreamSynchronize(s2);
   delete c;  // DevBuf destructors free device memory
@@ -1092,13 +1097,15 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
       }
       c->sort_tmp.alloc(
           std::max({launch::radix_sort_tmp_words(n), launch::scan_tmp_words(n), launch::seg_tmp_words(n)}));
-      if (!c->ord_map.p) {
+      // (ord_filtered may ask for them: from 2^20 ops, a row per 16 ops at least)
+      const bool filter = nops >= (1ull << 20) && c->cfg.rows <= 16 * nops;
+      if (filter && !c->ord_map.p) {
         c->ord_map.alloc(launch::ord_map_bytes(c->cfg.rows));
         HIP_TRY(hipMemsetAsync(c->ord_map.p, 0, c->ord_map.n, c->stream));
         c->ord_bits.alloc((c->cfg.rows + 31) / 32);
         c->ord_count.alloc(1);
       }
-      c->ord_flags.alloc(launch::ord_flag_words(nops));
+      if (filter) c->ord_flags.alloc(launch::ord_flag_words(nops));
       if (c->scheme == SCHEME_GACCO && c->tpcc && c->comb_min) {
         c->comb_chunk_cap = launch::comb_chunk_cap(nops, TPCC_COMBINE_MIN);
         c->comb_multi_cap = 0;
@@ -1114,9 +1121,11 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
       if (c->scheme == SCHEME_GPUTX) {
         c->sk64a.alloc(n);
         c->sk64b.alloc(n);
-        c->ord_row.alloc(n);
-        c->ord_op.alloc(n);
-        c->ord_tx.alloc(n);
+        if (filter) {
+          c->ord_row.alloc(n);
+          c->ord_op.alloc(n);
+          c->ord_tx.alloc(n);
+        }
         c->rank.alloc(ntx);
         c->tx_map.alloc(ntx);
         c->max_rank.alloc(1);

@@ -137,8 +137,8 @@ int gcctb_check_ops(const uint64_t* ops, const uint64_t* tx_off, uint64_t ntx, u
 
 /* Run every loaded transaction with the reference's launch structure: Init0
  * splits into batches, then per batch Init (reset / preprocess) + one kernel
- * launch + synchronization (benchmark_cpu/ycsb.cu:249-291, include/cc.cuh:29-36,
- * benchmark/ycsb.cu:21-111).  The table keeps the result; run again to
+ * launch, one batch after the other (benchmark_cpu/ycsb.cu:249-291, include/cc.cuh:29-36,
+ * benchmark/ycsb.cu:21-111).  The host queues the batches and waits at the end.  The table keeps the result; run again to
  * continue on it.  A batch whose kernel reports an error (GCCTB_EKERNEL, e.g.
  * the per-wave watchdog, GCCTB_WATCHDOG_S seconds) ends the run; every CC
  * word is then cleared, so no lock or mark of an unfinished transaction
@@ -201,7 +201,7 @@ int gcctb_serve(gcctb_ctx* ctx, const gcctb_serve_config* cfg, const uint64_t* b
  * reference: it is for callers that cannot allocate device memory (code under
  * stream capture, tight serving loops, harnesses that forbid hipMalloc).  It
  * runs the gcctb_run_plain kernels (per batch: counter reset, one launch,
- * restore of the touched words, host synchronization) for tpl_nw, tpl_wd, to,
+ * restore of the touched words; one host synchronization at the end) for tpl_nw, tpl_wd, to,
  * mvcc, silo and tictoc over device buffers the caller owns; keys are row ids
  * (key < rows, the reference's identity id column; other keys are index
  * misses).  Every other device word (CC words, MVCC chain heads and version
