@@ -105,6 +105,8 @@ struct TxCtx {
   bool done = true;
   uint64_t ts = 0;         // attempt timestamp (T/O, MVCC) or commit timestamp
   uint64_t t_start = 0, t_attempt = 0, t_resume = 0, t_round = 0;
+  uint32_t unit = 0;       // ticks per unit of the current retry delay
+  uint32_t cut_at = 0;     // `attempts` when a rest was first cut (0: never)
   uint64_t m_ts = 0, m_wait = 0, m_abort = 0, m_idx = 0, m_tot = 0, m_commit = 0, m_att = 0, m_miss = 0;
   uint32_t row[K];
   uint32_t meta[K];
@@ -307,6 +309,7 @@ __device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, ui
   if (c.backoff < 2 || !a.young_ticks || t - ld(a.ctrs + CTR_T0) >= a.young_ticks) c.backoff++;
   const uint32_t span = 1u << (c.backoff < a.backoff_exp ? c.backoff : a.backoff_exp);
   c.t_resume = t + (h % span) * unit;
+  c.unit = (uint32_t)unit;
   c.ph = PH_START;
 }
 
@@ -374,6 +377,7 @@ __device__ __forceinline__ void raise_ts_floor(const ExecArgs& a, uint64_t seen)
 template <bool WAIT_DIE>
 struct TwoPL {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
+  static constexpr uint32_t kTailShare = 2;
   static constexpr bool kBulkRefill = true;
   static constexpr bool kSlotStash = false;
   // lock_shared (twopl.cuh:233-267), continuing from an observed word `cur`
@@ -614,6 +618,7 @@ __device__ __forceinline__ void ts_head_reads(const TxCtx<G>& c, const ExecArgs&
 
 struct TimestampOrdering {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
+  static constexpr uint32_t kTailShare = 4;
   static constexpr bool kBulkRefill = true;
   static constexpr bool kSlotStash = false;
   static __device__ StepResult write_mark(uint64_t* w, uint64_t ts, uint64_t& prev, uint64_t& seen) {
@@ -738,6 +743,7 @@ constexpr uint64_t MVCC_COL_STRIDE = 3;
 __device__ __forceinline__ uint64_t mvcc_stride(const ExecArgs& a) { return kRowOps ? 2 + (uint64_t)a.cols : MVCC_COL_STRIDE; }
 struct Mvcc {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
+  static constexpr uint32_t kTailShare = 4;
   static constexpr bool kBulkRefill = true;
   static constexpr bool kSlotStash = false;
   static __device__ StepResult read(const ExecArgs& a, uint32_t row, uint32_t col, uint64_t ts,
@@ -1017,6 +1023,7 @@ __device__ __forceinline__ void occ_lock(const TxCtx<G>& c, const ExecArgs& a, u
 // ===========================================================================
 struct Silo {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
+  static constexpr uint32_t kTailShare = 4;
   static constexpr bool kBulkRefill = true;
   static constexpr bool kSlotStash = false;
   // Read: the word, then the cell (silo.cuh:223-259 loads the word a second
@@ -1161,6 +1168,7 @@ struct Silo {
 // ===========================================================================
 struct Tictoc {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
+  static constexpr uint32_t kTailShare = 4;
   static constexpr bool kBulkRefill = true;
   static constexpr bool kSlotStash = false;
   template <int G>
@@ -1424,6 +1432,7 @@ __device__ __forceinline__ void load_tx(TxCtx<G>& c, const ExecArgs& a, uint64_t
   c.ph = PH_START;
   c.attempts = 0;
   c.backoff = 0;
+  c.cut_at = 0;
   c.t_resume = 0;
   c.t_start = now;
   c.nops = 0;
@@ -1577,6 +1586,8 @@ __device__ void watchdog_stop(const TxCtx<G>& c, const ExecArgs& a) {
 // watchdog period.
 // ---------------------------------------------------------------------------
 constexpr uint64_t GATE_TICKS = 5000;    // a refilling wave re-reads its gate copy at most every 50 us
+constexpr uint64_t TAIL_TICKS = 1000;    // a wave that rests for longer looks at the launch's end this often (10 us)
+constexpr uint32_t TAIL_EXP = 1;         // the delay exponent that the stream's end leaves
 constexpr uint64_t PARK_TICKS = 20000;   // a wave with no live group: every 200 us
 constexpr uint64_t ADMIT_TICKS = 1000;   // a wave whose groups wait for an admission: every 10 us
 constexpr uint64_t STALL_TICKS = 100000; // held-back waves sample the slot counter every 1 ms
@@ -1638,8 +1649,74 @@ __device__ __forceinline__ uint64_t stash_take(SlotStash& s, uint64_t* ctr, bool
   return r < had ? lo + r : hi + (r - had);
 }
 
+// The end of a launch.  A retry delay is drawn for the crowd that the attempt
+// failed in.  Once no transactions follow (in the plain form from the start,
+// in the persistent form when the stream is handed out), that crowd thins out
+// and the delays drawn in it are what the launch waits for: up to 1,024 units
+// of up to 50 us.  Each wave therefore reports its groups that are through
+// (when it rests and when it ends, one add to its block's gate line), and a
+// wave that rests for longer than TAIL_TICKS looks up, once per TAIL_TICKS,
+// how many groups are left and cuts its rest to (left / share + 4) units,
+// twice that after every 16 further aborts, so that transactions that go on
+// colliding end up with the delays they draw.  In the persistent form the
+// first such look also takes the exponent back to TAIL_EXP: from there on it
+// grows with the crowd that is left.  The share is 4, and 2 for 2PL, whose
+// failed attempts hold locks that make others fail.
+//
+// Persistent kernel ms before -> after, tuned shapes: 131,072 tx x 16 ops,
+// 2,097,152 rows, theta 0.9, read ratio 0.9: TicToc 43 -> 29, Silo 42 -> 31,
+// 2PL 37 -> 34, T/O 59 -> 28, MVCC 75 -> 39; 262,144 tx, theta 0.6: TicToc 8
+// -> 2.1, Silo 18 -> 2.5, 2PL 9 -> 3.7, T/O 23 -> 3.8, MVCC 24 -> 4.6; 400,000
+// tx, 1,048,576 rows, theta 0.1: Silo 1.3 -> .6, 2PL 3.4 -> 1.1, MVCC 3.4 ->
+// .95.  Plain form, the same streams in batches: theta 0.9: TicToc 124 -> 53,
+// Silo 54 -> 37, 2PL 55 -> 51, T/O 88 -> 39, MVCC 117 -> 47; theta 0.6: T/O 38
+// -> 3.6, MVCC 50 -> 3.9.  With a share of 8 plain 2PL loses a sixth at theta
+// 0.99; cut to left / 64 units it drowns in retries (126 -> 2,000 ms).
+struct Tail {
+  uint32_t told = 0;   // groups of this wave that it has reported
+  bool ended = false;  // persistent form: saw the stream handed out
+  uint64_t next = 0;   // next look
+};
+template <int G>
+__device__ __forceinline__ void tail_report(const ExecArgs& a, Tail& t, bool through) {
+  const uint32_t n = (uint32_t)__popcll(ballot(through && (lane_id() & (G - 1)) == 0));
+  if (n != t.told && lane_id() == 0)
+    fetch_add(a.ctrs + CTR_GATE0 + 16 * (blockIdx.x & (GATE_SHARDS - 1)) + 3, (uint64_t)(n - t.told));
+  t.told = n;
+}
+// A wave all of whose live groups rest (the whole wave calls it).
+template <int G>
+__device__ __forceinline__ void tail_rest(TxCtx<G>& c, const ExecArgs& a, Tail& t, bool through, uint32_t share,
+                                          uint64_t now) {
+  if (now < t.next || ballot(!c.done && c.ph == PH_START && c.t_resume > now + TAIL_TICKS) == 0) return;
+  t.next = now + TAIL_TICKS;
+  tail_report<G>(a, t, through);
+  if (a.persist && ld(a.ctrs + CTR_GATE0 + 16 * (blockIdx.x & (GATE_SHARDS - 1)) + 2) == 0) return;
+  // the smallest wave (a block of 32 threads) has a lane for every gate line
+  static_assert(GATE_SHARDS <= 32 && (GATE_SHARDS & (GATE_SHARDS - 1)) == 0, "lanes 0..GATE_SHARDS-1 sum the lines");
+  uint64_t n = lane_id() < (uint32_t)GATE_SHARDS ? ld(a.ctrs + CTR_GATE0 + 16 * lane_id() + 3) : 0;
+#pragma unroll
+  for (int m = 1; m < GATE_SHARDS; m <<= 1) n += shfl_xor64(n, m);
+  n = shfl64(n, 0);
+  const uint64_t groups = (uint64_t)(blockDim.x / G) * gridDim.x;
+  const uint64_t others = n + 1 < groups ? groups - n - 1 : 0;
+  const uint32_t since = c.cut_at ? (c.attempts - c.cut_at) / 16 : 0;
+  uint64_t most = others ? (others / share + 4) * c.unit << (since < 10 ? since : 10) : 0;
+  if (a.persist && !t.ended) {
+    t.ended = true;
+    c.backoff = c.backoff < TAIL_EXP ? c.backoff : TAIL_EXP;
+    const uint64_t first = (uint64_t)c.unit << TAIL_EXP;
+    most = most < first ? most : first;
+  }
+  if (!c.done && c.ph == PH_START && c.t_resume > now + most) {
+    c.t_resume = now + (most ? (c.t_resume - now) % most : 0);
+    if (!c.cut_at) c.cut_at = c.attempts;
+  }
+}
+
 template <class S, int G>
 __device__ void run_persistent(TxCtx<G>& c, const ExecArgs& a) {
+  Tail tail_state;
   __shared__ SlotStash stash;
   if constexpr (S::kSlotStash) {
     if (threadIdx.x == 0) {
@@ -1768,9 +1845,10 @@ __device__ void run_persistent(TxCtx<G>& c, const ExecArgs& a) {
     }
     if (ballot(!c.done) == 0)
       __builtin_amdgcn_s_sleep(64);  // no group of the wave is live (held back, waiting or finished)
-    else if (ballot(!c.done && !((c.ph == PH_START || S::kRestInOps) && c.t_round < c.t_resume)) == 0)
+    else if (ballot(!c.done && !((c.ph == PH_START || S::kRestInOps) && c.t_round < c.t_resume)) == 0) {
       __builtin_amdgcn_s_sleep(4);  // every live group is resting
-    else
+      if constexpr (!S::kRestInOps) tail_rest<G>(c, a, tail_state, finished, S::kTailShare, now);
+    } else
       scheme_round<S, G>(c, a);
     c.t_round = now = now_ticks();
     const bool stuck = !c.done && a.watchdog_ticks && now - c.t_start > a.watchdog_ticks;
@@ -1779,6 +1857,7 @@ __device__ void run_persistent(TxCtx<G>& c, const ExecArgs& a) {
       break;
     }
   }
+  if constexpr (!S::kRestInOps) tail_report<G>(a, tail_state, true);
 }
 
 // MAXT: the largest block the instantiation is launched with.  A block of
@@ -1797,13 +1876,15 @@ __global__ __launch_bounds__(MAXT) void txn_exec(ExecArgs a) {
     const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     c.t_round = now_ticks();
     load_tx(c, a, a.slot_lo + gtid / G, c.t_round);
+    Tail tail_state;
 #pragma unroll 1
     while (true) {
       if (ballot(!c.done) == 0) break;
       // every live group of the wave is resting: sleep instead of spinning
-      if (ballot(!c.done && !((c.ph == PH_START || S::kRestInOps) && c.t_round < c.t_resume)) == 0)
+      if (ballot(!c.done && !((c.ph == PH_START || S::kRestInOps) && c.t_round < c.t_resume)) == 0) {
         __builtin_amdgcn_s_sleep(4);
-      else
+        if constexpr (!S::kRestInOps) tail_rest<G>(c, a, tail_state, c.done, S::kTailShare, c.t_round);
+      } else
         scheme_round<S, G>(c, a);
       c.t_round = now_ticks();
       // Watchdog on the oldest live transaction of the wave; the wall clock is
@@ -1814,6 +1895,7 @@ __global__ __launch_bounds__(MAXT) void txn_exec(ExecArgs a) {
         break;
       }
     }
+    if constexpr (!S::kRestInOps) tail_report<G>(a, tail_state, true);
   }
   // metrics: sums over the transactions the group ran, reduced over the wave
   const bool leader = (lane_id() & (G - 1)) == 0;

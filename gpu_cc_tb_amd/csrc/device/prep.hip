@@ -1404,6 +1404,7 @@ __device__ __forceinline__ void reset_batch(uint64_t* ctrs) {
   }
   // timestamp allocators restart at 1 (timestamp.cuh:76-80)
   if (i < TS_SHARDS) dev::st(ctrs + CTR_TS0 + 16 * i, 1);
+  if (i < GATE_SHARDS) dev::st(ctrs + CTR_GATE0 + 16 * i + 3, 0);  // groups that are through
 }
 __device__ __forceinline__ void reset_admission(uint64_t* ctrs) {
   const int i = threadIdx.x;
@@ -1411,6 +1412,7 @@ __device__ __forceinline__ void reset_admission(uint64_t* ctrs) {
   if (i < GATE_SHARDS) {
     dev::st(ctrs + CTR_GATE0 + 16 * i + 1, 0);
     dev::st(ctrs + CTR_GATE0 + 16 * i + 2, 0);
+    dev::st(ctrs + CTR_GATE0 + 16 * i + 3, 0);
     dev::st(ctrs + CTR_ADMIT0 + 16 * i, 0);  // the u32 admission word and its neighbour
   }
 }

@@ -195,7 +195,8 @@ constexpr int TS_SHARD_BITS = 4;
 // GATE_SHARDS copies of the gate a wave reads before taking slots (one copy
 // per block index mod GATE_SHARDS, each on its own line, so the polls of
 // thousands of waves spread out): [1] transactions in urgent state, [2]
-// stream handed out.  The open form (serving) adds GATE_SHARDS copies of the
+// stream handed out, [3] groups of the copy's blocks that take no more
+// transactions (also in the plain form).  The open form (serving) adds GATE_SHARDS copies of the
 // admission word that the host writes while the launch runs: a u32 at the
 // start of each copy's line (a host copy writes an aligned 32-bit word in one
 // piece, a 64-bit word possibly in two); slots below its low 31 bits are
