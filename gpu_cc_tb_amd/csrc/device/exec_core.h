@@ -269,14 +269,16 @@ __device__ __forceinline__ void ev_commit(const TxCtx<G>& c, const ExecArgs& a) 
 // wait, and 1024 such units would idle a transaction for seconds.
 //
 // A young plain launch (until 300 us + 4 ns per transaction after its
-// counters were reset) spans at most 4 units and does not raise e: the
-// conflicts of a low-contention batch are over within that time, and delays
-// that had already grown to 8 and 16 units of the first, crowded attempt were
-// half of such a launch (65,536 transactions of 16 ops on 1,048,576 rows,
-// theta 0.1, read ratio 0.9, 8 lanes each: 2PL 800 -> 350 us, T/O 290 -> 215,
-// MVCC 420 -> 350, Silo 520 -> 330, TicToc 510 -> 375; 6,007 transactions of 4
-// to 32 ops on 131,071 rows, read ratio 0.5: 390-910 -> 140-290 us).  A
-// contended launch runs for tens of ms, so the aborts of its first 300 us do
+// counters were reset) spans at most 4 units of at most 4 us and does not
+// raise e: the conflicts of a low-contention batch are over within that time,
+// and delays of 8 and 16 units, or of units as long as the first, crowded
+// attempt (50 us and more), were half of such a launch.  65,536 transactions
+// of 16 ops on 1,048,576 rows, theta 0.1, read ratio 0.9, 8 lanes each, us
+// with growing delays, with 4 units, with 4 units of at most 4 us: 2PL 800,
+// 435, 383; T/O 290, 300, 197; MVCC 420, 430, 330; Silo 520, 463, 383; TicToc
+// 510, 445, 367.  Units of at most 2 us: 1-4% less there, but 2PL 232 -> 296
+// on 6,007 transactions of 4 to 32 ops on 131,071 rows, read ratio 0.5.
+// A contended launch runs for tens of ms, so the aborts of its first 300 us do
 // not count (theta 0.99, read ratio 0.5 and 0.9: within 2% either way).  By
 // the age of the transaction instead, the waves that start late would each
 // bring a burst of retries of their own: 2PL 1.5x slower at theta 0.99.
@@ -294,6 +296,7 @@ __device__ __forceinline__ void urgent_add(const ExecArgs& a, uint64_t delta) {
 }
 
 constexpr uint64_t BACKOFF_UNIT_MAX = 5000;  // 50 us of the 100 MHz wall clock
+constexpr uint64_t YOUNG_UNIT_MAX = 400;     // 4 us, while a plain launch is young
 
 template <int G>
 __device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, uint64_t now) {
@@ -306,7 +309,9 @@ __device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, ui
   uint64_t unit = dur > a.backoff_ticks ? dur : a.backoff_ticks;
   if (unit > BACKOFF_UNIT_MAX) unit = BACKOFF_UNIT_MAX;
   const uint64_t h = hash3(a.seed ^ TAG_BACKOFF, c.tx, c.attempts);
-  if (c.backoff < 2 || !a.young_ticks || t - ld(a.ctrs + CTR_T0) >= a.young_ticks) c.backoff++;
+  const bool young = a.young_ticks && t - ld(a.ctrs + CTR_T0) < a.young_ticks;
+  if (c.backoff < 2 || !young) c.backoff++;
+  if (young && unit > YOUNG_UNIT_MAX) unit = YOUNG_UNIT_MAX;
   const uint32_t span = 1u << (c.backoff < a.backoff_exp ? c.backoff : a.backoff_exp);
   c.t_resume = t + (h % span) * unit;
   c.unit = (uint32_t)unit;
