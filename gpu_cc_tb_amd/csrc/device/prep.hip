@@ -2,6 +2,7 @@
 // index construction and probing, a stable LSD radix sort, scans, and the
 // GaccO / GPUTx access-order passes that replace the reference's Thrust calls
 // (include/gacco.cuh:307-336, include/gputx.cuh:252-281).
+#include <cstddef>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "dev_util.h"
@@ -1431,34 +1432,49 @@ __global__ void k_run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, 
 // End of a run: the metrics slots' totals, GPUTx's conflicts, the ops run by
 // combiners and the deferral's state words, into host memory, so that the
 // host reads them after its one wait for the stream and no copy follows.
-__global__ __launch_bounds__(METRIC_SLOTS) void k_run_end(const Metrics* metrics, const uint64_t* conflicts,
-                                                          const uint64_t* combined, const uint32_t* defer,
-                                                          launch::RunResult* out) {
-  constexpr int F = 10;  // Metrics fields in use
-  __shared__ unsigned long long sum[F];
-  const uint32_t t = threadIdx.x;
-  if (t < F) sum[t] = 0;
-  __syncthreads();
-  const uint64_t* m = reinterpret_cast<const uint64_t*>(metrics + t);
+// One block, since every run waits for it; bound by one load latency: thread t
+// sums field t mod 16 of every 16th slot, all its loads (whole lines per 16
+// threads) issued at once, and 16 threads add 16 sums each out of LDS.  An LDS
+// atomic per slot and field took 15-22 us.
+constexpr int RUN_FIELDS = 10;  // Metrics fields in use; the last is error_flags
+static_assert(offsetof(Metrics, error_flags) == 8 * (RUN_FIELDS - 1) && METRICS_WORDS == 16, "the fields k_run_end sums");
+__global__ __launch_bounds__(256) void k_run_end(const Metrics* metrics, const uint64_t* conflicts,
+                                                 const uint64_t* combined, const uint32_t* defer,
+                                                 launch::RunResult* out) {
+  constexpr int STEP = 256 / METRICS_WORDS;  // slots that the block reads at once
+  constexpr int N = METRIC_SLOTS / STEP;
+  static_assert(METRIC_SLOTS % STEP == 0 && launch::CONFLICT_SLOTS == METRICS_WORDS, "no remainder");
+  __shared__ uint64_t part[STEP + 1][METRICS_WORDS];
+  const uint32_t f = threadIdx.x % METRICS_WORDS, g = threadIdx.x / METRICS_WORDS;
+  const bool flags = f == RUN_FIELDS - 1;
+  const uint64_t* m = reinterpret_cast<const uint64_t*>(metrics) + threadIdx.x;
+  uint64_t v[N];
 #pragma unroll
-  for (int f = 0; f < F; ++f) {
-    const uint64_t v = m[f];
-    if (!v) continue;
-    if (f == 9)
-      atomicOr(&sum[f], (unsigned long long)v);  // error_flags
-    else
-      atomicAdd(&sum[f], (unsigned long long)v);
-  }
+  for (int i = 0; i < N; ++i) v[i] = m[(size_t)i * 256];
+  const uint64_t confl = g == 0 && conflicts ? conflicts[16 * f] : 0;
+  const uint64_t comb = threadIdx.x == 0 && combined ? *combined : 0;
+  const uint32_t any = threadIdx.x == 0 && defer ? defer[launch::DEFER_ANY] : 0;
+  const uint32_t nhot = threadIdx.x == 0 && defer ? defer[launch::DEFER_NHOT] : 0;
+  uint64_t x = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) x = flags ? x | v[i] : x + v[i];
+  part[g][f] = x;
+  if (g == 0) part[STEP][f] = confl;
   __syncthreads();
   uint64_t* o = reinterpret_cast<uint64_t*>(&out->metrics);
-  if (t < F) dev::st(o + t, sum[t]);
-  if (t == 0) {
+  if (threadIdx.x < RUN_FIELDS) {
+    uint64_t y = 0;
+#pragma unroll
+    for (int i = 0; i < STEP; ++i) y = flags ? y | part[i][f] : y + part[i][f];
+    dev::st(o + f, y);
+  }
+  if (threadIdx.x == 0) {
     uint64_t c = 0;
-    if (conflicts)
-      for (uint32_t i = 0; i < launch::CONFLICT_SLOTS; ++i) c += conflicts[16 * i];
+#pragma unroll
+    for (int i = 0; i < (int)launch::CONFLICT_SLOTS; ++i) c += part[STEP][i];
     dev::st(&out->conflicts, c);
-    dev::st(&out->combined, combined ? *combined : 0);
-    dev::st(&out->deferred, defer && defer[launch::DEFER_ANY] ? defer[launch::DEFER_NHOT] : 0);
+    dev::st(&out->combined, comb);
+    dev::st(&out->deferred, any ? nhot : 0);
   }
 }
 
@@ -1761,7 +1777,7 @@ hipError_t run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, bool co
 }
 hipError_t run_end(const Metrics* metrics, const uint64_t* conflicts, const uint64_t* combined, const uint32_t* defer,
                    RunResult* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_run_end, dim3(1), dim3(METRIC_SLOTS), 0, s, metrics, conflicts, combined, defer, out);
+  hipLaunchKernelGGL(k_run_end, dim3(1), dim3(256), 0, s, metrics, conflicts, combined, defer, out);
   return hipGetLastError();
 }
 hipError_t persist_begin(uint64_t* ctrs, hipStream_t s) {
