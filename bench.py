@@ -17,7 +17,7 @@ commit, one restore of the touched CC words.
 The timed region holds exactly --steps steps; inputs are already resident in
 HBM.  `value` is whole-job committed Tx/s of the batched form (8 x 1,048,576 x
 steps transactions / time).  The plain form (the reference's per batch
-reset + launch + synchronize) is timed the same way and reported beside it.
+reset + launch, one wait at the end) is timed the same way and reported beside it.
 
 Batched-vs-plain legs (one pass of each form per scheme, preparation inside
 the timed region, at full size):

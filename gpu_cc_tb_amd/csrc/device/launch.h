@@ -36,10 +36,12 @@ hipError_t index_insert(const uint32_t* keys, const uint32_t* vals, uint64_t n, 
                         uint32_t nbuckets, hipStream_t s);
 // rows_out[i] = row of ops[i]'s key (rows_out may be null); also into rows_copy when it is given;
 // ids_out[i] = what op_ids(ops, n, id_base) writes, when it is given; with
-// id_map, id_map[i] with the op's write flag in bit 31 instead
+// id_map, id_map[i] with the op's write flag in bit 31 instead; need[i] =
+// NEED_FREE when given; nzero words (at most 256) at `zero` are cleared
 hipError_t probe(const IndexView& ix, const uint64_t* ops, uint64_t n, uint32_t* rows_out,
                  hipStream_t s, uint32_t* rows_copy = nullptr, uint32_t* ids_out = nullptr,
-                 uint32_t id_base = 0, const uint32_t* id_map = nullptr);
+                 uint32_t id_base = 0, const uint32_t* id_map = nullptr, uint32_t* need = nullptr,
+                 uint64_t* zero = nullptr, uint32_t nzero = 0);
 
 // --- per-op helpers ---
 hipError_t op_tx(const uint64_t* tx_off, uint64_t ntx, uint32_t* op_tx, hipStream_t s);

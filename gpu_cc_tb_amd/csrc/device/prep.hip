@@ -1,9 +1,10 @@
-// Preprocessing and maintenance kernels for gfx950: table seeding, sorted-array
-// index construction and probing, a stable LSD radix sort, scans, and the
+// Preprocessing and maintenance kernels for gfx950: table seeding, hash-index
+// construction and probing, a stable LSD radix sort, scans, and the
 // GaccO / GPUTx access-order passes that replace the reference's Thrust calls
 // (include/gacco.cuh:307-336, include/gputx.cuh:252-281).
 #include <cstddef>
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <stdint.h>
 #include "dev_util.h"
 #include "launch.h"
@@ -137,9 +138,14 @@ __device__ __forceinline__ bool quad_bucket_match(const uint4& w, uint32_t key, 
 // the same number) maps each key to itself and reads no bucket.
 // ids_out[i] (optional): the op's id (id_base + i), or id_map[i] when given,
 // with the op's write flag in bit 31
+// need[i] (optional) = NEED_FREE, and nzero words at `zero` are cleared: the
+// ordered schemes' preparation starts here, and each fill of its own cost a
+// launch per batch (16,384 TPC-C orders: 6 us and two launches of 17;
+// 16.8 M ops: 81 -> 65 us).
 __global__ __launch_bounds__(256) void k_probe(IndexView ix, const uint64_t* ops, uint64_t n, uint32_t* rows_out,
                                                uint32_t* rows_copy, uint32_t* ids_out, uint32_t id_base,
-                                               const uint32_t* id_map) {
+                                               const uint32_t* id_map, uint32_t* need, uint64_t* zero, uint32_t nzero) {
+  if (blockIdx.x == 0 && threadIdx.x < nzero) zero[threadIdx.x] = 0;
   if (ix.dense) {  // direct addressing: no bucket to read
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
       const uint64_t op = ops[i];
@@ -147,6 +153,7 @@ __global__ __launch_bounds__(256) void k_probe(IndexView ix, const uint64_t* ops
       if (rows_out) rows_out[i] = r;
       if (rows_copy) rows_copy[i] = r;
       if (ids_out) ids_out[i] = (id_map ? id_map[i] : id_base + (uint32_t)i) | (op_is_write(op) ? OPID_WRITE : 0u);
+      if (need) need[i] = NEED_FREE;
     }
     return;
   }
@@ -191,6 +198,7 @@ __global__ __launch_bounds__(256) void k_probe(IndexView ix, const uint64_t* ops
       if (rows_copy) rows_copy[mine] = r;
       if (ids_out)
         ids_out[mine] = (id_map ? id_map[mine] : id_base + (uint32_t)mine) | (op_is_write(myop) ? OPID_WRITE : 0u);
+      if (need) need[mine] = NEED_FREE;
     }
   }
 }
@@ -743,7 +751,7 @@ __global__ __launch_bounds__(BT) void k_ord_compact(IndexView ix, const uint64_t
 // (EV_ROW), or a new access group of its row (EV_GROUP: it or the access
 // before it writes), or continues a run of reads (0).
 //
-// Two passes over tiles of TT elements, 8 consecutive ones per thread:
+// Two passes over tiles of TT elements, TT_ITEMS consecutive ones per thread:
 // k_seg_tiles leaves each tile's last row start, last group start and the
 // group starts after its last row start; then a tile's carry-in is found by
 // reading the summaries before it backwards, 64 at a time (one step unless a
@@ -755,12 +763,19 @@ __global__ __launch_bounds__(BT) void k_ord_compact(IndexView ix, const uint64_t
 // Bound: the scattered need stores, which only accesses that meet another one
 // still make (the others keep NEED_FREE from a streaming fill).
 // ---------------------------------------------------------------------------
-constexpr int TT_ITEMS = 8;
-constexpr int TT = BT * TT_ITEMS;
+// Up to TT_SHORT_MAX accesses a thread takes TT_FEW for the turns, not
+// TT_MANY: tiles of 2,048 left most of the chip idle at the sizes of a batch
+// (180,224 accesses of 16,384 TPC-C orders, 88 tiles: 15.6 -> 12.3 us; the
+// chosen accesses of 65,536 GPUTx transactions: 13.1 -> 8.5).  The ranks keep
+// TT_MANY (9.0 us against 12.2: more blocks end in an atomic on one word).
+constexpr int TT_MANY = 8, TT_FEW = 2;
+constexpr uint64_t TT_SHORT_MAX = 1ull << 20;
+inline bool tt_few(uint64_t n) { return n <= TT_SHORT_MAX; }
 constexpr uint32_t EV_ROW = 1u, EV_GROUP = 2u;
 
-template <class KT>
+template <class KT, int TT_ITEMS>
 struct SegTile {
+  static constexpr int TT = BT * TT_ITEMS;
   KT k[TT_ITEMS];
   uint32_t v[TT_ITEMS];
   KT pk;         // the access before the thread's first
@@ -772,12 +787,13 @@ struct SegTile {
     p0 = (uint64_t)blockIdx.x * TT + (uint64_t)threadIdx.x * TT_ITEMS;
     cnt = p0 >= n ? 0u : n - p0 < (uint64_t)TT_ITEMS ? (uint32_t)(n - p0) : (uint32_t)TT_ITEMS;
     if (cnt == (uint32_t)TT_ITEMS) {
-      constexpr int Q = (int)sizeof(KT) * TT_ITEMS / 16;
-      uint4 q[Q], w[2];
+      typedef uint32_t Wide __attribute__((ext_vector_type(TT_ITEMS < 4 ? TT_ITEMS : 4)));
+      constexpr int W = (int)sizeof(Wide) / 4, Q = (int)sizeof(KT) / 4 * TT_ITEMS / W, V = TT_ITEMS / W;
+      Wide q[Q], w[V];
 #pragma unroll
-      for (int i = 0; i < Q; ++i) q[i] = reinterpret_cast<const uint4*>(key + p0)[i];
+      for (int i = 0; i < Q; ++i) q[i] = reinterpret_cast<const Wide*>(key + p0)[i];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) w[i] = reinterpret_cast<const uint4*>(val + p0)[i];
+      for (int i = 0; i < V; ++i) w[i] = reinterpret_cast<const Wide*>(val + p0)[i];
       __builtin_memcpy(k, q, sizeof k);
       __builtin_memcpy(v, w, sizeof v);
     } else {
@@ -842,8 +858,8 @@ __device__ __forceinline__ SegScan seg_block_scan(const SegScan& mine, SegScan* 
   return seg_join(before, e);
 }
 // what the thread's own accesses add to the scan
-template <class KT>
-__device__ __forceinline__ SegScan seg_own(const SegTile<KT>& t, int rb) {
+template <class KT, int TT_ITEMS>
+__device__ __forceinline__ SegScan seg_own(const SegTile<KT, TT_ITEMS>& t, int rb) {
   SegScan s{0, 0, 0};
 #pragma unroll
   for (int i = 0; i < TT_ITEMS; ++i) {
@@ -887,12 +903,13 @@ __device__ __forceinline__ SegScan seg_carry(const uint4* summ) {
   return in;
 }
 
-template <class KT>
+template <class KT, int TT_ITEMS>
 __global__ __launch_bounds__(BT) void k_seg_tiles(const KT* key, const uint32_t* val, uint64_t n, int rb, uint4* summ,
                                                   const uint32_t* nd) {
+  constexpr int TT = BT * TT_ITEMS;
   if (nd) n = *nd;
   if ((uint64_t)blockIdx.x * TT >= n) return;
-  SegTile<KT> t;
+  SegTile<KT, TT_ITEMS> t;
   t.load(key, val, n);
   SegScan total;
   seg_block_scan(seg_own(t, rb), &total);
@@ -931,15 +948,16 @@ __device__ __forceinline__ uint32_t block_file(uint32_t n, uint32_t* ctr) {  // 
 }
 constexpr uint32_t CB_BT = 256;  // accesses per combiner chunk, one per thread
 
-template <class KT>
+template <class KT, int TT_ITEMS>
 __global__ __launch_bounds__(BT) void k_seg_turns(const KT* key, const uint32_t* val, uint64_t n, int rb,
                                                   const uint4* summ, uint32_t* need, uint32_t* counters,
                                                   uint64_t nrows, launch::CombArgs comb,
                                                   unsigned long long* conflicts, const uint32_t* nd) {
+  constexpr int TT = BT * TT_ITEMS;
   if (nd) n = *nd;
   if ((uint64_t)blockIdx.x * TT >= n) return;
   __shared__ uint32_t wnext[BT / 64];
-  SegTile<KT> t;
+  SegTile<KT, TT_ITEMS> t;
   t.load(key, val, n);
   const uint32_t lane = dev::lane_id(), wave = threadIdx.x / 64;
   SegScan total, at = seg_block_scan(seg_own(t, rb), &total);
@@ -1061,9 +1079,10 @@ __global__ __launch_bounds__(BT) void k_seg_turns(const KT* key, const uint32_t*
 __global__ __launch_bounds__(BT) void k_seg_ranks(const uint32_t* key, const uint32_t* val, uint64_t n,
                                                   const uint4* summ, uint64_t nrows, uint32_t* rank,
                                                   uint32_t* max_rank, const uint32_t* tx_of, const uint32_t* nd) {
+  constexpr int TT_ITEMS = TT_MANY, TT = BT * TT_ITEMS;
   if (nd) n = *nd;
   if ((uint64_t)blockIdx.x * TT >= n) return;
-  SegTile<uint32_t> t;
+  SegTile<uint32_t, TT_ITEMS> t;
   t.load(key, val, n);
   SegScan total, at = seg_block_scan(seg_own(t, 0), &total);
   at = seg_join(seg_carry(summ), at);
@@ -1594,8 +1613,10 @@ hipError_t index_insert(const uint32_t* keys, const uint32_t* vals, uint64_t n, 
   GC_LAUNCH(k_index_insert, n, keys, vals, n, buckets, nbuckets);
 }
 hipError_t probe(const IndexView& ix, const uint64_t* ops, uint64_t n, uint32_t* rows_out,
-                 hipStream_t s, uint32_t* rows_copy, uint32_t* ids_out, uint32_t id_base, const uint32_t* id_map) {
-  GC_LAUNCH(k_probe, n, ix, ops, n, rows_out, rows_copy, ids_out, id_base, id_map);
+                 hipStream_t s, uint32_t* rows_copy, uint32_t* ids_out, uint32_t id_base, const uint32_t* id_map,
+                 uint32_t* need, uint64_t* zero, uint32_t nzero) {
+  if (nzero > 256) return hipErrorInvalidValue;  // one word per thread of a block
+  GC_LAUNCH(k_probe, n, ix, ops, n, rows_out, rows_copy, ids_out, id_base, id_map, need, zero, nzero);
 }
 hipError_t op_tx(const uint64_t* tx_off, uint64_t ntx, uint32_t* op_tx, hipStream_t s) {
   GC_LAUNCH(k_op_tx, ntx, tx_off, ntx, op_tx);
@@ -1659,17 +1680,29 @@ hipError_t access_group_flags(const uint32_t* srow, const uint32_t* sop, uint64_
                               hipStream_t s, uint32_t* rowstart) {
   GC_LAUNCH(k_access_group_flags, n, srow, sop, n, flags, rowstart);
 }
-uint64_t seg_tmp_words(uint64_t n) { return 4 * ((n + TT - 1) / TT); }
+static unsigned seg_blocks(uint64_t n) {
+  const uint64_t tile = BT * (tt_few(n) ? TT_FEW : TT_MANY);
+  return (unsigned)((n + tile - 1) / tile);
+}
+// a smaller n may take the shorter tiles
+uint64_t seg_tmp_words(uint64_t n) { return 4 * std::max<uint64_t>(seg_blocks(n), seg_blocks(std::min(n, TT_SHORT_MAX))); }
 template <class KT>
 static hipError_t seg_turns_impl(const KT* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
                                  uint32_t* counters, uint64_t nrows, const CombArgs& comb, uint64_t* conflicts,
                                  const uint32_t* nd, hipStream_t s) {
   if (n == 0) return hipSuccess;
-  const unsigned nb = (unsigned)((n + TT - 1) / TT);
+  const unsigned nb = seg_blocks(n);
   uint4* summ = reinterpret_cast<uint4*>(tmp);
-  hipLaunchKernelGGL((k_seg_tiles<KT>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, nd);
-  hipLaunchKernelGGL((k_seg_turns<KT>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, need, counters, nrows, comb,
-                     (unsigned long long*)conflicts, nd);
+  auto* confl = reinterpret_cast<unsigned long long*>(conflicts);
+  if (tt_few(n)) {
+    hipLaunchKernelGGL((k_seg_tiles<KT, TT_FEW>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, nd);
+    hipLaunchKernelGGL((k_seg_turns<KT, TT_FEW>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, need, counters, nrows,
+                       comb, confl, nd);
+  } else {
+    hipLaunchKernelGGL((k_seg_tiles<KT, TT_MANY>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, nd);
+    hipLaunchKernelGGL((k_seg_turns<KT, TT_MANY>), dim3(nb), dim3(BT), 0, s, key, val, n, rb, summ, need, counters, nrows,
+                       comb, confl, nd);
+  }
   return hipGetLastError();
 }
 hipError_t seg_turns(const uint32_t* key, const uint32_t* val, uint64_t n, int rb, uint32_t* tmp, uint32_t* need,
@@ -1685,11 +1718,10 @@ hipError_t seg_turns64(const uint64_t* key, const uint32_t* val, uint64_t n, int
 hipError_t seg_ranks(const uint32_t* row, const uint32_t* val, uint64_t n, uint32_t* tmp, uint64_t nrows,
                      uint32_t* rank, uint32_t* max_rank, hipStream_t s, const uint32_t* tx_of, const uint32_t* nd) {
   if (n == 0) return hipSuccess;
-  const unsigned nb = (unsigned)((n + TT - 1) / TT);
+  const unsigned nb = (unsigned)((n + BT * TT_MANY - 1) / (BT * TT_MANY));
   uint4* summ = reinterpret_cast<uint4*>(tmp);
-  hipLaunchKernelGGL((k_seg_tiles<uint32_t>), dim3(nb), dim3(BT), 0, s, row, val, n, 0, summ, nd);
-  hipLaunchKernelGGL(k_seg_ranks, dim3(nb), dim3(BT), 0, s, row, val, n, summ, nrows, rank, max_rank,
-                     tx_of, nd);
+  hipLaunchKernelGGL((k_seg_tiles<uint32_t, TT_MANY>), dim3(nb), dim3(BT), 0, s, row, val, n, 0, summ, nd);
+  hipLaunchKernelGGL(k_seg_ranks, dim3(nb), dim3(BT), 0, s, row, val, n, summ, nrows, rank, max_rank, tx_of, nd);
   return hipGetLastError();
 }
 uint64_t comb_chunk_cap(uint64_t nops, uint32_t min) { return nops / min + nops / CB_BT + 1; }

@@ -531,14 +531,13 @@ class GaccoHost : public SchemeHost {
                                  ctx.sort_tmp.p, ctx.need.p + o0, ctx.sk0.p, ctx.sv0.p, s));
       nd = ctx.ord_count.p;
     } else {
-      HIP_TRY(launch::probe(ctx.ix, ctx.ops.p + o0, n, rows, s, ctx.sk0.p, ctx.sv0.p, (uint32_t)o0));
-      HIP_TRY(launch::fill_u32(ctx.need.p + o0, n, NEED_FREE, s));
+      HIP_TRY(launch::probe(ctx.ix, ctx.ops.p + o0, n, rows, s, ctx.sk0.p, ctx.sv0.p, (uint32_t)o0, nullptr,
+                            ctx.need.p + o0, ctx.comb_ctr.p, comb ? (uint32_t)ctx.comb_ctr.n : 0));
     }
     // rows are below cfg.rows; a miss (IDX_MISS) has all row bits set and sorts last
     HIP_TRY(launch::radix_sort_u32(ctx.sk0.p, ctx.sv0.p, ctx.sk1.p, ctx.sv1.p, n, bits_for(ctx.cfg.rows),
                                    ctx.sort_tmp.p, &srow, &sop, s, nd));
     const launch::CombArgs ca = comb ? comb_args() : launch::CombArgs{};
-    if (comb) HIP_TRY(launch::fill_u64(ctx.comb_ctr.p, ctx.comb_ctr.n, 0, s));
     HIP_TRY(launch::seg_turns(srow, sop, n, 0, ctx.sort_tmp.p, ctx.need.p, ctx.counters.p, ctx.cfg.rows, ca, nullptr, s,
                               nd));
     if (comb) HIP_TRY(ctx.tpcc ? launch::tpcc_combine(ca, srow, sop, s) : launch::gacco_combine(ca, srow, sop, s));
@@ -607,7 +606,7 @@ class GPUTxHost : public SchemeHost {
       nd = ctx.ord_count.p;
       tx_of = ctx.ord_tx.p;
     } else {
-      HIP_TRY(launch::probe(ctx.ix, ctx.ops.p, n, rows, s, ctx.sk0.p, ctx.sv0.p, 0, ctx.op_tx.p));
+      HIP_TRY(launch::probe(ctx.ix, ctx.ops.p, n, rows, s, ctx.sk0.p, ctx.sv0.p, 0, ctx.op_tx.p, ctx.need.p));
     }
     uint32_t *srow, *stx_ops;
     // rows are below cfg.rows; a miss (IDX_MISS) has all row bits set and sorts last
@@ -641,10 +640,7 @@ class GPUTxHost : public SchemeHost {
     const uint32_t* krow = filt ? ctx.ord_row.p : ctx.rows_out.p;
     const uint32_t* ktx = filt ? ctx.ord_tx.p : ctx.op_tx.p;
     uint32_t* v0 = filt ? ctx.ord_op.p : ctx.sv0.p;  // op ids
-    if (!filt) {
-      HIP_TRY(launch::fill_u32(ctx.need.p, n, NEED_FREE, s));
-      HIP_TRY(launch::op_ids(ctx.ops.p, n, 0, v0, s));
-    }
+    if (!filt) HIP_TRY(launch::op_ids(ctx.ops.p, n, 0, v0, s));
     uint32_t* sop2;
     if (row_bits + rank_bits <= 32) {
       HIP_TRY(launch::gtx_exec_keys32(krow, ktx, ctx.rank.p, n, rank_bits, ctx.sk0.p, s, nd));
@@ -1189,10 +1185,12 @@ static std::string error_text(uint64_t flags) {
 }
 
 // One pass over every loaded transaction.
-//   plain:      the reference's structure -- per batch Init, one launch, Post,
-//               host synchronization (benchmark_cpu/ycsb.cu:262-285)
+//   plain:      the reference's structure -- per batch Init, one launch, Post
+//               (benchmark_cpu/ycsb.cu:262-285); the batches are queued and
+//               the host waits once, at the end (a launch does nothing once
+//               an earlier one reported an error)
 //   graph:      the same per-batch kernels captured once into a hipGraph and
-//               replayed, with no host round trip between batches
+//               replayed
 //   persistent: one preparation of the whole stream and one persistent launch
 static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
   if (!c) return set_error(GCCTB_EINVAL, "null context");

@@ -38,12 +38,16 @@ def _one_row_stream(ntx, writes, rows, seed):
 
 
 TURN_TILE = 2048  # accesses per tile of the turn kernels; carries look back 64 tiles a step
+TURN_SHORT = 512  # up to SHORT_MAX accesses
 TURN_CASES = {
     # name: (ntx, transactions that write row 0)
     "no_writes": (TURN_TILE, []),
     "tile_edges": (2 * TURN_TILE + 1, [TURN_TILE - 1, TURN_TILE, 2 * TURN_TILE]),
     "first_and_last": (TURN_TILE + 7, [0, TURN_TILE + 6]),
     "past_64_tiles": (66 * TURN_TILE + 5, [0, 3, 66 * TURN_TILE + 1]),
+    "short_tile_edges": (2 * TURN_SHORT + 1, [TURN_SHORT - 1, TURN_SHORT, 2 * TURN_SHORT]),
+    "longest_short": (SHORT_MAX // 2, [0, 3, SHORT_MAX // 2 - 1]),
+    "shortest_long": (SHORT_MAX // 2 + 1, [0, 3, TURN_TILE, SHORT_MAX // 2]),
 }
 
 
