@@ -103,6 +103,7 @@ struct TxCtx {
   uint32_t backoff = 0;    // exponent of the retry delay
   bool live = false;
   bool done = true;
+  bool deep = false;       // ordered schemes: an op was deep_turns or more turns from its own (this or, once done, the last transaction)
   uint64_t ts = 0;         // attempt timestamp (T/O, MVCC) or commit timestamp
   uint64_t t_start = 0, t_attempt = 0, t_resume = 0, t_round = 0;
   uint32_t unit = 0;       // ticks per unit of the current retry delay
@@ -1400,6 +1401,7 @@ struct Ordered {
       // POLL_REST_MAX) instead of polling every round; deep waiters on a hot
       // row then stop flooding the memory system the row's chain depends on.
       const uint64_t turns = group_min64<G>(gap);
+      c.deep |= turns >= a.deep_turns;
       if (turns > 1) {
         const uint64_t rest = (turns - 1) * (uint64_t)a.poll_ticks;
         c.t_resume = now + (rest < POLL_REST_MAX ? rest : POLL_REST_MAX);
@@ -1438,6 +1440,7 @@ __device__ __forceinline__ void load_tx(TxCtx<G>& c, const ExecArgs& a, uint64_t
   c.attempts = 0;
   c.backoff = 0;
   c.cut_at = 0;
+  c.deep = false;
   c.t_resume = 0;
   c.t_start = now;
   c.nops = 0;
@@ -1615,13 +1618,28 @@ __device__ __forceinline__ void scheme_round(TxCtx<G>& c, const ExecArgs& a) {
 
 // Slots a block has drawn and not started, [next, end), under a lock that a
 // wave holds for one draw at most (its holder never waits for another wave).
+//
+// Where rows have long queues, a slot that lies in a stash holds up every
+// transaction queued behind it, in all blocks.  A wave that finds a
+// transaction deep_turns or more turns from its own (now, or in the one just
+// finished) therefore makes its block's next STASH_SINGLE draws take no more
+// slots than they start.  GPUTx, 1,048,576 transactions of 16 ops, kernel ms
+// drawing singly / in chunks / by this rule, (4, 8, 4,096): theta 0.99, read
+// ratio 0.9: 208 / 375 / 211; theta 0.8: 48 / 66 / 49; theta 0.6: 7.1 / 5.8 /
+// 6.0; theta 0.1: 3.2 / 1.6 / 1.6.  deep_turns is 8, and 128 where
+// combiners have run GaccO's queues of that length: its launch with 8 drew
+// singly over queues that are not worth it (262,144 transactions of 4 to 32
+// ops, theta 0.99, read ratio 0.5: 1,845 -> 2,580 us a pass).
+constexpr uint32_t STASH_SINGLE = 32;
 struct SlotStash {
   uint32_t lock;
+  uint32_t single;  // draws to come that take no more than they need
   uint64_t next, end;
 };
 // A slot for every lane with `take` (the wave's first such lane draws for
 // all; every lane of the wave calls it).
-__device__ __forceinline__ uint64_t stash_take(SlotStash& s, uint64_t* ctr, bool take, uint32_t chunk, uint64_t tail) {
+__device__ __forceinline__ uint64_t stash_take(SlotStash& s, uint64_t* ctr, bool take, uint32_t chunk, uint64_t tail,
+                                               bool deep) {
   const uint64_t m = ballot(take);
   const int first = __ffsll((unsigned long long)m) - 1;
   const uint32_t want = (uint32_t)__popcll(m);
@@ -1640,7 +1658,9 @@ __device__ __forceinline__ uint64_t stash_take(SlotStash& s, uint64_t* ctr, bool
     s.next = lo + had;
     if (had < want) {
       const uint32_t rest = want - had;
-      const uint32_t n = s.end < tail && chunk > rest ? chunk : rest;
+      const uint32_t single = deep ? STASH_SINGLE : s.single;
+      s.single = single ? single - 1 : 0;
+      const uint32_t n = single == 0 && s.end < tail && chunk > rest ? chunk : rest;
       hi = fetch_add(ctr, n);
       s.next = hi + rest;
       s.end = hi + n;
@@ -1726,6 +1746,7 @@ __device__ void run_persistent(TxCtx<G>& c, const ExecArgs& a) {
   if constexpr (S::kSlotStash) {
     if (threadIdx.x == 0) {
       stash.lock = 0;
+      stash.single = 0;
       stash.next = stash.end = 0;
     }
     __syncthreads();
@@ -1790,7 +1811,7 @@ __device__ void run_persistent(TxCtx<G>& c, const ExecArgs& a) {
       if (!stashing && handed_out && need && held == NO_SLOT) finished = true;
       const bool take = need && !finished && urgent == 0 && held == NO_SLOT;
       if (ballot(take) != 0) {
-        uint64_t got = stashing ? stash_take(stash, slot_ctr, take && leader, chunk, tail)
+        uint64_t got = stashing ? stash_take(stash, slot_ctr, take && leader, chunk, tail, ballot(c.deep) != 0)
                                 : wave_fetch_inc(slot_ctr, take && leader);
         got = group_bcast64<G>(got);
         if (take) {

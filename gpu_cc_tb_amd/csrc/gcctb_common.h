@@ -329,6 +329,7 @@ struct ExecArgs {
   uint32_t backoff_exp;     // retry delay spans at most 2^backoff_exp units
   uint32_t young_ticks;     // plain form: until this long after CTR_T0 it spans at most 4 units (young_ticks())
   uint32_t poll_ticks;      // ordered schemes: expected ticks per handoff on a row (rest pacing)
+  uint32_t deep_turns;      // ordered schemes, persistent form: a wait of this many turns counts as long
   uint64_t* tcommit;       // optional, per tx: wall-clock tick of its commit (serving form)
   uint64_t* ev_op;         // event-log kernels: per op, the stamp of its access (0 = none)
   uint64_t* ev_commit;     // event-log kernels: per tx, the stamp of its commit (0 = none)

@@ -338,6 +338,7 @@ class SchemeHost {
     a.backoff_exp = ctx.backoff_exp;
     a.young_ticks = young_ticks(slot_hi - slot_lo);
     a.poll_ticks = ctx.poll_ticks;
+    a.deep_turns = 8;
     a.dbg = ctx.dbg.p;
     a.persist_groups = ctx.cfg.persist_window;
     a.open = ctx.open_launch ? 1u : 0u;
@@ -544,7 +545,8 @@ class GaccoHost : public SchemeHost {
     if (stream) combined_ = comb;
   }
   void Launch(int b, uint64_t lo, uint64_t hi, bool persist) override {
-    const ExecArgs a = args(b, lo, hi);
+    ExecArgs a = args(b, lo, hi);
+    if (persist && combined_) a.deep_turns = std::max(a.deep_turns, ctx.comb_min);
     if (launch_rows(a, hi - lo, persist)) return;
     HIP_TRY(launch::exec_ordered(ctx.G, a, hi - lo, ctx.threads, persist, ctx.stream));
   }
