@@ -232,26 +232,39 @@ __global__ void k_fill64(uint64_t* v, uint64_t n, uint64_t x) {
 // Stable LSD radix sort, three launches per pass: per-tile digit histograms,
 // the scan of each digit's row of the [digit][tile] matrix (one block per
 // digit), then the scatter, whose blocks scan the 256 digit totals
-// themselves.  The key bits are split evenly over ceil(bits / 8) passes
-// (20 bits: 7 + 7 + 6), which shortens the per-item ballot loop and
-// lengthens each digit's run.  A tile is 256 x RS_ITEMS elements; wave w of the
-// block holds tile elements [w*RS_WSPAN, (w+1)*RS_WSPAN), lane-minor, so
-// (wave, item, lane) order is input order.  The scatter ranks every element
-// within its digit (ballots inside a wave, a per-wave LDS counter across its
-// items, a prefix over waves), sorts the tile in LDS, and writes it out digit
-// run by digit run, so consecutive lanes store to consecutive addresses.
+// themselves (two launches for short inputs, RS_OWN_COUNTS).  The key bits are
+// split evenly over ceil(bits / 8) passes (20 bits: 7 + 7 + 6), which shortens
+// the per-item ballot loop and lengthens each digit's run.  A tile is 256 x
+// RS_ITEMS elements; wave w of the block holds tile elements [w*RS_WSPAN,
+// (w+1)*RS_WSPAN), lane-minor, so (wave, item, lane) order is input order.  The
+// scatter ranks every element within its digit (ballots inside a wave, a
+// per-wave LDS counter across its items, a prefix over waves), sorts the tile in
+// LDS, and writes it out digit run by digit run, so consecutive lanes store to
+// consecutive addresses.
 // Bound: the stores of the digit runs (a pass over 2^24 u32 pairs moves 335
 // MB in about 120 us, 2.8 TB/s) and, below 2^20 pairs, launch latency (about
 // 4 us each).  Sort of u32 pairs by 24 bits against 5 launches a pass on
 // 4,096-element tiles: 2^24 pairs 370 -> 368 us, 2^20 90 -> 73 us, 180,000 80 ->
-// 39 us.
+// 39 us (with the scan's launch).
 // ---------------------------------------------------------------------------
 constexpr int RS_BT = 256;
 constexpr int RS_WAVES = RS_BT / 64;
+// Short inputs do without the scan's launch: the scatter's blocks read the
+// whole matrix, laid out [tile][digit] then, with RS_OWN_LOADS 16-byte loads
+// per thread, all in flight at once.  That costs them 1 to 4 us, growing with
+// the matrix, against the launch's 4.  Sort of u32 pairs with / without the
+// scan's launch, 24 loads: 16,384 pairs by 21 bits 34.5 -> 30.3 us, 65,536
+// 34.9 -> 31.5, 131,072 35.9 -> 33.0, 180,000 (22,528 counts) 37.4 -> 33.8; by
+// 24 bits 65,536 (16,384 counts) 36.8 -> 31.9.  In two rounds of 16 loads the
+// gain ends there: 131,072 by 24 bits (32,768 counts) 38.0 -> 37.6, 262,144 by
+// 21 bits (32,768) 38.3 -> 38.6, 262,144 by 24 bits (65,536) 43.5 -> 47.8.
+constexpr int RS_OWN_LOADS = 24;
+constexpr uint64_t RS_OWN_COUNTS = (uint64_t)RS_OWN_LOADS * 4 * RS_BT;
+constexpr int RS_OWN_WIDTH = 5;  // digits of fewer bits would leave long sums to few threads
 
 template <class KT, int RS_ITEMS>
 __global__ __launch_bounds__(RS_BT) void k_rs_hist(const KT* keys, uint64_t n, int shift, uint32_t dmask,
-                                                   uint32_t* hist, uint32_t nb, const uint32_t* nd) {
+                                                   uint32_t* hist, uint32_t nb, const uint32_t* nd, int by_tile) {
   __shared__ uint32_t h[256];
   constexpr int RS_TILE = RS_BT * RS_ITEMS;
   if (nd) n = *nd;
@@ -269,7 +282,9 @@ __global__ __launch_bounds__(RS_BT) void k_rs_hist(const KT* keys, uint64_t n, i
   for (int i = 0; i < RS_ITEMS; ++i)
     if (d[i] < 256u) atomicAdd(&h[d[i]], 1u);
   __syncthreads();
-  if (threadIdx.x <= dmask) {
+  if (by_tile) {  // [tile][digit], read by the scatter itself
+    if (threadIdx.x <= dmask) hist[(uint64_t)blockIdx.x * (dmask + 1) + threadIdx.x] = h[threadIdx.x];
+  } else if (threadIdx.x <= dmask) {
     hist[(uint64_t)threadIdx.x * nb + blockIdx.x] = h[threadIdx.x];
     if (base + RS_TILE >= n)  // the last tile also clears up to the next whole 16-byte load
       for (uint32_t b = blockIdx.x + 1; b & 3u; ++b) hist[(uint64_t)threadIdx.x * nb + b] = 0;
@@ -327,8 +342,9 @@ __global__ __launch_bounds__(RS_BT) void k_rs_rowscan(uint32_t* offs, uint32_t n
 
 // offs[d * nb + b]: where tile b's first element of digit d goes within the
 // digit, totals[d] the elements of digit d; the digit is the `width` bits of
-// the key from `shift` up
-template <class KT, int RS_ITEMS>
+// the key from `shift` up.  OWN_SCAN: offs is the unscanned [tile][digit]
+// matrix (16-byte rows) and totals is unused; the block adds the columns up.
+template <class KT, int RS_ITEMS, bool OWN_SCAN>
 __global__ __launch_bounds__(RS_BT) void k_rs_scatter(const KT* kin, const uint32_t* vin, KT* kout,
                                                       uint32_t* vout, uint64_t n, int shift, int width,
                                                       const uint32_t* offs, uint32_t nb, const uint32_t* totals,
@@ -348,6 +364,25 @@ __global__ __launch_bounds__(RS_BT) void k_rs_scatter(const KT* kin, const uint3
   const uint32_t cnt = n - base < (uint64_t)RS_TILE ? (uint32_t)(n - base) : (uint32_t)RS_TILE;
 #pragma unroll
   for (int w = 0; w < RS_WAVES; ++w) wcnt[w][t] = 0;
+  // counts of four digits in the tiles before this one, and in all of them
+  uint4 before = make_uint4(0, 0, 0, 0), every = before;
+  if constexpr (OWN_SCAN) {
+    const uint4* m = reinterpret_cast<const uint4*>(offs);
+    const int qbits = width - 2;  // a row is 2^qbits loads; the thread's column is the same in every row it reads
+    const uint32_t cells = (uint32_t)((n + RS_TILE - 1) / RS_TILE) << qbits;
+    uint4 c[RS_OWN_LOADS];
+#pragma unroll
+    for (int i = 0; i < RS_OWN_LOADS; ++i) {
+      const uint32_t j = i * RS_BT + t;
+      c[i] = j < cells ? m[j] : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < RS_OWN_LOADS; ++i) {
+      const uint32_t f = (i * RS_BT + t) >> qbits < blockIdx.x ? ~0u : 0u;
+      before.x += c[i].x & f, before.y += c[i].y & f, before.z += c[i].z & f, before.w += c[i].w & f;
+      every.x += c[i].x, every.y += c[i].y, every.z += c[i].z, every.w += c[i].w;
+    }
+  }
   KT k[RS_ITEMS];
   uint32_t v[RS_ITEMS];
 #pragma unroll
@@ -390,8 +425,21 @@ __global__ __launch_bounds__(RS_BT) void k_rs_scatter(const KT* kin, const uint3
     wcnt[w][t] = tot;
     tot += c;
   }
-  const uint32_t all = t <= dmask ? totals[t] : 0u;
-  const uint32_t in_digit = t <= dmask ? offs[(uint64_t)t * nb + blockIdx.x] : 0u;
+  uint32_t all = 0, in_digit = 0;
+  if constexpr (OWN_SCAN) {
+    __shared__ uint4 part[2][RS_BT];
+    part[0][t] = before;
+    part[1][t] = every;
+    __syncthreads();
+    if (t <= dmask)  // column t / 4 was added up by every 2^(width-2)-th thread
+      for (uint32_t j = t; j < 4 * RS_BT; j += dmask + 1) {
+        in_digit += reinterpret_cast<const uint32_t*>(part[0])[j];
+        all += reinterpret_cast<const uint32_t*>(part[1])[j];
+      }
+  } else if (t <= dmask) {
+    all = totals[t];
+    in_digit = offs[(uint64_t)t * nb + blockIdx.x];
+  }
   uint32_t x = tot, y = all;
 #pragma unroll
   for (int dd = 1; dd < 64; dd <<= 1) {
@@ -565,6 +613,13 @@ hipError_t scan_impl(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tm
   return hipGetLastError();
 }
 
+// Items per thread (a tile is 256 x items).  Up to 2^20 elements a 4,096-element
+// tile leaves at most one block per CU, whose 16 items per wave then rank one
+// after another with nothing to hide their latency; above, the longer tile's
+// longer digit runs win.  24-bit sort, 16 / 4 items: 180,000 pairs 64 / 39 us,
+// 2^20 73 / 71 us, 2^21 84 / 107 us, 2^24 363 / 741 us.
+constexpr int RS_LONG = 16, RS_SHORT = 4;
+constexpr uint64_t RS_SHORT_MAX = 1ull << 20;
 template <class KT, int ITEMS>
 hipError_t radix_impl(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, int key_bits,
                       uint32_t* tmp, KT** kout, uint32_t** vout, const uint32_t* nd, hipStream_t s, bool ids = false) {
@@ -581,12 +636,19 @@ hipError_t radix_impl(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, in
     for (int p = 0, shift = 0; p < passes; ++p) {
       const int width = (key_bits - shift + passes - p - 1) / (passes - p);  // what is left, evenly
       const uint32_t dmask = (1u << width) - 1u;
-      hipLaunchKernelGGL((k_rs_hist<KT, ITEMS>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, n, shift, dmask, hist, stride, nd);
-      hipLaunchKernelGGL(k_rs_rowscan, dim3(dmask + 1), dim3(RS_BT), 0, s, hist, stride, totals,
-                         (uint32_t)(RS_BT * ITEMS), nd);
-      hipLaunchKernelGGL((k_rs_scatter<KT, ITEMS>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka,
-                         ids && p == 0 ? (const uint32_t*)nullptr : va, kb, vb, n, shift, width,
-                         hist, stride, totals, nd);
+      const uint32_t* vin = ids && p == 0 ? nullptr : va;
+      const bool own = ITEMS == RS_SHORT && nb << width <= RS_OWN_COUNTS && width >= RS_OWN_WIDTH;
+      hipLaunchKernelGGL((k_rs_hist<KT, ITEMS>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, n, shift, dmask, hist, stride, nd,
+                         own ? 1 : 0);
+      if (own) {
+        hipLaunchKernelGGL((k_rs_scatter<KT, RS_SHORT, true>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, vin, kb, vb, n,
+                           shift, width, hist, stride, totals, nd);
+      } else {
+        hipLaunchKernelGGL(k_rs_rowscan, dim3(dmask + 1), dim3(RS_BT), 0, s, hist, stride, totals,
+                           (uint32_t)(RS_BT * ITEMS), nd);
+        hipLaunchKernelGGL((k_rs_scatter<KT, ITEMS, false>), dim3((unsigned)nb), dim3(RS_BT), 0, s, ka, vin, kb, vb, n,
+                           shift, width, hist, stride, totals, nd);
+      }
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
       shift += width;
@@ -603,13 +665,6 @@ hipError_t radix_impl(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, in
   return hipGetLastError();
 }
 
-// Items per thread (a tile is 256 x items).  Up to 2^20 elements a 4,096-element
-// tile leaves at most one block per CU, whose 16 items per wave then rank one
-// after another with nothing to hide their latency; above, the longer tile's
-// longer digit runs win.  24-bit sort, 16 / 4 items: 180,000 pairs 64 / 39 us,
-// 2^20 73 / 71 us, 2^21 84 / 107 us, 2^24 363 / 741 us.
-constexpr int RS_LONG = 16, RS_SHORT = 4;
-constexpr uint64_t RS_SHORT_MAX = 1ull << 20;
 template <class KT>
 hipError_t radix_sort(KT* k0, uint32_t* v0, KT* k1, uint32_t* v1, uint64_t n, int key_bits, uint32_t* tmp, KT** kout,
                       uint32_t** vout, const uint32_t* nd, hipStream_t s) {

@@ -23,6 +23,24 @@ def test_sort_tile_sizes(n, dtype, bits):
     assert np.array_equal(v, order.astype(np.uint32)) and np.array_equal(k, keys[order])
 
 
+OWN_SCAN_COUNTS = 24 * 4 * 256  # counts (tiles x digits) that a scatter block adds up itself
+
+
+@pytest.mark.parametrize("n", [2, 1024, 5121] + [OWN_SCAN_COUNTS // d * 1024 + e for d in (256, 128, 32) for e in (0, 1)])
+@pytest.mark.parametrize("dtype,bits", [(np.uint32, 4), (np.uint32, 5), (np.uint32, 21), (np.uint32, 32), (np.uint64, 41)])
+def test_sort_without_scan_launch(n, dtype, bits):
+    """One tile, a few, and as many as digits of 8, 7 and 5 bits allow and one
+    more; digits of 4 to 8 bits: the stable sort."""
+    rng = np.random.default_rng(n * 64 + bits)
+    keys = rng.integers(0, np.iinfo(dtype).max, n, dtype=dtype, endpoint=True)
+    keys[: n // 3] = keys[0]  # one digit with a long run
+    vals = np.arange(n, dtype=np.uint32)
+    print(f"[sort-own-scan] n={n} bits={bits}", flush=True)
+    k, v, _ = g.sort_pairs(keys, vals, key_bits=bits)
+    order = np.argsort(keys & dtype((1 << bits) - 1), kind="stable")
+    assert np.array_equal(v, order.astype(np.uint32)) and np.array_equal(k, keys[order])
+
+
 def _one_row_stream(ntx, writes, rows, seed):
     """ntx transactions of 2 ops: row 0, read or (at the given transactions)
     written, and a row of their own, so one queue runs through the sorted
