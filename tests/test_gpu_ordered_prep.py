@@ -26,6 +26,7 @@ def test_sort_tile_sizes(n, dtype, bits):
 OWN_SCAN_COUNTS = 24 * 4 * 256  # counts (tiles x digits) that a scatter block adds up itself
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [2, 1024, 5121] + [OWN_SCAN_COUNTS // d * 1024 + e for d in (256, 128, 32) for e in (0, 1)])
 @pytest.mark.parametrize("dtype,bits", [(np.uint32, 4), (np.uint32, 5), (np.uint32, 21), (np.uint32, 32), (np.uint64, 41)])
 def test_sort_without_scan_launch(n, dtype, bits):
