@@ -1097,13 +1097,13 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
           std::max({launch::radix_sort_tmp_words(n), launch::scan_tmp_words(n), launch::seg_tmp_words(n)}));
       // (ord_filtered may ask for them: from 2^20 ops, a row per 16 ops at least)
       const bool filter = nops >= (1ull << 20) && c->cfg.rows <= 16 * nops;
-      if (filter && !c->ord_map.p) {
+      if (filter) {
         c->ord_map.alloc(launch::ord_map_bytes(c->cfg.rows));
         HIP_TRY(hipMemsetAsync(c->ord_map.p, 0, c->ord_map.n, c->stream));
         c->ord_bits.alloc((c->cfg.rows + 31) / 32);
         c->ord_count.alloc(1);
+        c->ord_flags.alloc(launch::ord_flag_words(nops));
       }
-      if (filter) c->ord_flags.alloc(launch::ord_flag_words(nops));
       if (c->scheme == SCHEME_GACCO && c->tpcc && c->comb_min) {
         c->comb_chunk_cap = launch::comb_chunk_cap(nops, TPCC_COMBINE_MIN);
         c->comb_multi_cap = 0;

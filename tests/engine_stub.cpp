@@ -1,0 +1,151 @@
+// The host engine on the CPU: gpu_cc_tb_amd/csrc/host/engine.cpp linked with
+// these stand-ins for the HIP runtime and the kernel launchers (launchers that
+// no scenario reaches stay undefined).  Device memory is host memory, work is
+// done when it is queued, and an allocation or a launch can be made to fail.
+// Each scenario prints "ok" or what it found.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "../gpu_cc_tb_amd/csrc/device/launch.h"
+#include "../include/gcctb.h"
+
+namespace {
+std::map<void*, size_t> live;  // allocation -> bytes
+size_t fail_bytes = 0;         // the next hipMalloc of this size fails
+int blocks(size_t bytes) {
+  int n = 0;
+  for (const auto& b : live) n += b.second == bytes;
+  return n;
+}
+std::string found;
+void expect(bool ok, const char* what) {
+  if (!ok && found.empty()) found = what;
+}
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+  if (n == fail_bytes) {
+    fail_bytes = 0;
+    return hipErrorOutOfMemory;
+  }
+  *p = std::calloc(1, n);
+  live[*p] = n;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  live.erase(p);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  *p = std::calloc(1, n);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
+  std::memset(d, v, n);
+  return hipSuccess;
+}
+hipError_t hipGetDeviceCount(int* n) {
+  *n = 1;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
+  *v = 100000;
+  return hipSuccess;
+}
+const char* hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = nullptr;
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) {
+  *e = nullptr;
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+}
+
+namespace gcctb {
+namespace launch {
+hipError_t op_tx(const uint64_t*, uint64_t, uint32_t*, hipStream_t) { return hipSuccess; }
+uint64_t scan_tmp_words(uint64_t n) { return n + 64; }
+uint64_t radix_sort_tmp_words(uint64_t n) { return n + 1024; }
+uint64_t seg_tmp_words(uint64_t n) { return n + 64; }
+uint64_t comb_chunk_cap(uint64_t n, uint32_t min) { return n / min + 1; }
+uint64_t comb_multi_cap(uint64_t n) { return n / 256 + 1; }
+uint64_t comb_sum_words(uint64_t n, uint32_t cols) { return n / 128 * (cols + 1) + 16; }
+uint64_t ord_flag_words(uint64_t n) { return n / 64 + 64; }
+uint64_t ord_map_bytes(uint64_t rows) { return (rows + 31) / 32 * 32; }
+hipError_t seed_table(uint64_t*, uint64_t, uint32_t, uint64_t, hipStream_t) { return hipSuccess; }
+}  // namespace launch
+}  // namespace gcctb
+
+namespace {
+using namespace gcctb;
+
+gcctb_ctx* make(const char* scheme, uint64_t rows) {
+  gcctb_config cfg{};
+  cfg.cc_scheme = scheme;
+  cfg.rows = rows;
+  cfg.cols = 1;
+  cfg.warp_density = 3;
+  cfg.block_size = 8;
+  cfg.batch_size = 1 << 16;
+  gcctb_ctx* c = nullptr;
+  expect(gcctb_create(&cfg, &c) == GCCTB_OK, "create");
+  expect(gcctb_seed_table(c) == GCCTB_OK, "seed");
+  return c;
+}
+
+// ntx transactions of one read each
+int load(gcctb_ctx* c, uint64_t ntx) {
+  std::vector<uint64_t> ops(ntx), off(ntx + 1);
+  for (uint64_t i = 0; i < ntx; ++i) ops[i] = make_op((uint32_t)(i % 1000), 0, false);
+  for (uint64_t i = 0; i <= ntx; ++i) off[i] = i;
+  return gcctb_load_ops(c, ops.data(), off.data(), ntx);
+}
+
+// A load whose allocation of the written-row bits, of their count or of the
+// row map fails, then the same load again: it returns OK with all of them.
+void load_after_failed_alloc(const char* scheme, int which) {
+  const uint64_t rows = 3000017, ntx = 1 << 20;  // sizes that no other buffer has
+  const size_t bits = (rows + 31) / 32 * 4, map = (rows + 31) / 32 * 32, count = 4;
+  gcctb_ctx* c = make(scheme, rows);
+  fail_bytes = which == 0 ? map : which == 1 ? bits : count;
+  expect(load(c, ntx) == GCCTB_EDEVICE, "the failed allocation is reported");
+  expect(load(c, ntx) == GCCTB_OK, "the second load fits");
+  expect(blocks(map) == 1, "the row map is there");
+  expect(blocks(bits) == 1, "the bits are there");
+  expect(blocks(count) == (!std::strcmp(scheme, "gputx") ? 2 : 1), "the count is there");  // (GPUTx: and the highest rank)
+  gcctb_destroy(c);
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+  if (argc < 2) return 2;
+  const std::string what = argv[1];
+  const char* scheme = argc > 2 ? argv[2] : "";
+  if (what == "alloc") load_after_failed_alloc(scheme, std::atoi(argv[3]));
+  std::printf("%s\n", found.empty() ? "ok" : found.c_str());
+  return found.empty() ? 0 : 1;
+}
