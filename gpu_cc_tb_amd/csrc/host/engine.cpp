@@ -147,7 +147,7 @@ struct gcctb_ctx {
   bool table_ready = false;
   // transactions
   uint64_t ntx = 0, nops = 0, nreads = 0;
-  std::vector<uint64_t> h_tx_off;
+  std::vector<uint64_t> h_tx_off{0};
   gcctb::DevBuf<uint64_t> ops, tx_off;
   gcctb::DevBuf<uint32_t> op_tx;
   // CC state
@@ -595,6 +595,8 @@ class GPUTxHost : public SchemeHost {
     ctx.rank_counts_ready = false;
     const uint64_t n = ctx.nops, ntx = ctx.ntx;
     hipStream_t s = ctx.stream;
+    ctx.nranks = 0;
+    if (!ntx) return;
     // per-row access lists in (row, tx) order; the sorted values are the
     // accesses' transactions (with the write flag), so the rank pass needs
     // no op -> transaction gather (of the chosen accesses alone, their indexes)
@@ -622,7 +624,7 @@ class GPUTxHost : public SchemeHost {
     HIP_TRY(hipMemcpyAsync(ctx.h_rank, ctx.max_rank.p, 4, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     // no ops at all: every transaction has rank 0
-    ctx.nranks = n ? (uint64_t)*ctx.h_rank + 1 : (ntx ? 1 : 0);
+    ctx.nranks = n ? (uint64_t)*ctx.h_rank + 1 : 1;
     // transactions in (rank, tx) order: stable sort of ranks (include/gputx.cuh:281),
     // whose values are the positions.  One pass (up to 256 ranks) leaves the
     // keys alone and writes tx_map; more of them sort a copy of the ranks.
@@ -1038,13 +1040,13 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
   // form keeps every version of the stream; a plain batch needs at most that)
   if (c->scheme == SCHEME_MVCC) cap = nops - nreads;
   try {
-    c->ntx = ntx;
-    c->nops = nops;
-    c->nreads = nreads;
+    // until every buffer is there the context holds no transactions: a run
+    // after a load that failed does nothing
+    c->ntx = c->nops = c->nreads = 0;
+    c->h_tx_off.assign(1, 0);
     c->params_loaded = 0;  // TPC-C parameters belong to the ops loaded before
     c->inputs_gen++;
     c->custom_batches.clear();
-    c->h_tx_off.assign(tx_off, tx_off + ntx + 1);
     c->ops.alloc(nops);
     c->tx_off.alloc(ntx + 1);
     c->op_tx.alloc(nops);
@@ -1134,6 +1136,10 @@ int gcctb_load_ops(gcctb_ctx* c, const uint64_t* ops, const uint64_t* tx_off, ui
   } catch (const HipFailure& f) {
     return hip_fail(f);
   }
+  c->h_tx_off.assign(tx_off, tx_off + ntx + 1);
+  c->ntx = ntx;
+  c->nops = nops;
+  c->nreads = nreads;
   return GCCTB_OK;
 }
 

@@ -24,6 +24,7 @@ int blocks(size_t bytes) {
   for (const auto& b : live) n += b.second == bytes;
   return n;
 }
+int launched = 0;              // execution launches over some transactions
 std::string found;
 void expect(bool ok, const char* what) {
   if (!ok && found.empty()) found = what;
@@ -83,6 +84,12 @@ hipError_t hipEventCreate(hipEvent_t* e) {
   return hipSuccess;
 }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = 1;
+  return hipSuccess;
+}
 }
 
 namespace gcctb {
@@ -97,6 +104,41 @@ uint64_t comb_sum_words(uint64_t n, uint32_t cols) { return n / 128 * (cols + 1)
 uint64_t ord_flag_words(uint64_t n) { return n / 64 + 64; }
 uint64_t ord_map_bytes(uint64_t rows) { return (rows + 31) / 32 * 32; }
 hipError_t seed_table(uint64_t*, uint64_t, uint32_t, uint64_t, hipStream_t) { return hipSuccess; }
+hipError_t fill_u32(uint32_t* v, uint64_t n, uint32_t x, hipStream_t) {
+  for (uint64_t i = 0; i < n; ++i) v[i] = x;
+  return hipSuccess;
+}
+hipError_t batch_begin(uint64_t*, hipStream_t) { return hipSuccess; }
+hipError_t reset_rows(const uint32_t*, uint64_t n, uint64_t, uint64_t*, uint32_t*, hipStream_t, bool) {
+  expect(n == 0, "rows are reset");
+  return hipSuccess;
+}
+hipError_t run_begin(uint64_t* m, uint32_t*, uint64_t*, bool, hipStream_t) {
+  std::memset(m, 0, METRIC_SLOTS * METRICS_WORDS * 8);
+  return hipSuccess;
+}
+hipError_t run_end(const Metrics* m, const uint64_t*, const uint64_t*, const uint32_t*, RunResult* out, hipStream_t) {
+  *out = RunResult{};
+  out->metrics = m[0];
+  return hipSuccess;
+}
+uint32_t defer_threshold(uint64_t, uint64_t, uint32_t) { return 2; }
+hipError_t defer_order(const uint64_t*, const uint64_t*, uint64_t n, uint64_t, uint32_t, uint32_t*, uint32_t*, hipStream_t) {
+  expect(n == 0, "transactions are deferred");
+  return hipSuccess;
+}
+// an execution launch commits its transactions
+hipError_t exec(const ExecArgs& a, uint64_t n) {
+  launched += n != 0;
+  a.metrics->committed += n;
+  return hipSuccess;
+}
+hipError_t exec_tpl(bool, int, const ExecArgs& a, uint64_t n, int, bool, hipStream_t) { return exec(a, n); }
+hipError_t exec_to(int, const ExecArgs& a, uint64_t n, int, bool, hipStream_t) { return exec(a, n); }
+hipError_t exec_mvcc(int, const ExecArgs& a, uint64_t n, int, bool, hipStream_t) { return exec(a, n); }
+hipError_t exec_silo(int, const ExecArgs& a, uint64_t n, int, bool, hipStream_t) { return exec(a, n); }
+hipError_t exec_tictoc(int, const ExecArgs& a, uint64_t n, int, bool, hipStream_t) { return exec(a, n); }
+hipError_t exec_ordered(int, const ExecArgs& a, uint64_t n, int, bool, hipStream_t) { return exec(a, n); }
 }  // namespace launch
 }  // namespace gcctb
 
@@ -139,6 +181,24 @@ void load_after_failed_alloc(const char* scheme, int which) {
   expect(blocks(count) == (!std::strcmp(scheme, "gputx") ? 2 : 1), "the count is there");  // (GPUTx: and the highest rank)
   gcctb_destroy(c);
 }
+
+// A run after a load that failed (the context's first, or one after a smaller
+// load) has no transactions.
+void run_after_failed_load(const char* scheme, bool first) {
+  const uint64_t ntx = 5003;
+  for (const bool persist : {false, true}) {
+    gcctb_ctx* c = make(scheme, 1000);
+    if (!first) expect(load(c, 100) == GCCTB_OK, "the smaller load");
+    fail_bytes = 4 * ntx;
+    expect(load(c, ntx) == GCCTB_EDEVICE, "the failed allocation is reported");
+    launched = 0;
+    gcctb_stats st{};
+    expect((persist ? gcctb_run_persistent(c, &st) : gcctb_run_plain(c, &st)) == GCCTB_OK, "the run");
+    expect(st.txs == 0 && st.committed == 0 && st.total_ops == 0 && st.batches == (persist ? 1 : 0), "an empty run");
+    expect(launched == 0, "nothing is launched");
+    gcctb_destroy(c);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -146,6 +206,7 @@ int main(int argc, char** argv) {
   const std::string what = argv[1];
   const char* scheme = argc > 2 ? argv[2] : "";
   if (what == "alloc") load_after_failed_alloc(scheme, std::atoi(argv[3]));
+  if (what == "run") run_after_failed_load(scheme, !std::strcmp(argv[3], "first"));
   std::printf("%s\n", found.empty() ? "ok" : found.c_str());
   return found.empty() ? 0 : 1;
 }

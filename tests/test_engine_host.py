@@ -30,3 +30,11 @@ def test_load_after_failed_allocation(engine, scheme, which):
     """The buffers of the written-row filter are all there after a load that
     returns OK, also when one of them could not be had in the load before."""
     engine("alloc", scheme, ["map", "bits", "count"].index(which))
+
+
+@pytest.mark.parametrize("when", ["first", "later"])
+@pytest.mark.parametrize("scheme", ["tpl_nw", "to", "mvcc", "tictoc", "gacco", "gputx"])
+def test_run_after_failed_load(engine, scheme, when):
+    """A run after a load that failed finds no transactions, not the new
+    counts on buffers that are missing or too small."""
+    engine("run", scheme, when)
