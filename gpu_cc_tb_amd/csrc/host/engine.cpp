@@ -1395,6 +1395,7 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
       }
     }
   } catch (const HipFailure& f) {
+    (void)hipStreamSynchronize(c->stream);  // batches queued before the failure may still run
     c->rows_probed = false;
     c->defer_active = false;
     c->hot_active = false;

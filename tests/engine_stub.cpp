@@ -25,6 +25,8 @@ int blocks(size_t bytes) {
   return n;
 }
 int launched = 0;              // execution launches over some transactions
+int fail_launch = 0;           // this one fails
+bool waited = true;            // the host has waited since the last launch
 std::string found;
 void expect(bool ok, const char* what) {
   if (!ok && found.empty()) found = what;
@@ -78,14 +80,17 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) {
+  waited = true;
+  return hipSuccess;
+}
 hipError_t hipEventCreate(hipEvent_t* e) {
   *e = nullptr;
   return hipSuccess;
 }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipStreamSynchronize(nullptr); }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
   *ms = 1;
   return hipSuccess;
@@ -110,7 +115,7 @@ hipError_t fill_u32(uint32_t* v, uint64_t n, uint32_t x, hipStream_t) {
 }
 hipError_t batch_begin(uint64_t*, hipStream_t) { return hipSuccess; }
 hipError_t reset_rows(const uint32_t*, uint64_t n, uint64_t, uint64_t*, uint32_t*, hipStream_t, bool) {
-  expect(n == 0, "rows are reset");
+  expect(n == 0 || launched, "rows are reset");
   return hipSuccess;
 }
 hipError_t run_begin(uint64_t* m, uint32_t*, uint64_t*, bool, hipStream_t) {
@@ -130,6 +135,8 @@ hipError_t defer_order(const uint64_t*, const uint64_t*, uint64_t n, uint64_t, u
 // an execution launch commits its transactions
 hipError_t exec(const ExecArgs& a, uint64_t n) {
   launched += n != 0;
+  if (fail_launch && launched == fail_launch) return hipErrorLaunchFailure;
+  waited = false;
   a.metrics->committed += n;
   return hipSuccess;
 }
@@ -199,6 +206,23 @@ void run_after_failed_load(const char* scheme, bool first) {
     gcctb_destroy(c);
   }
 }
+
+// A launch that cannot be queued ends the run: the error is reported once the
+// batches queued before it have ended, and the next run is whole.
+void failed_launch(const char* scheme) {
+  gcctb_ctx* c = make(scheme, 1000);
+  const uint64_t sizes[4] = {10, 20, 30, 40};
+  expect(load(c, 100) == GCCTB_OK, "load");
+  expect(gcctb_set_batches(c, sizes, 4) == GCCTB_OK, "batches");
+  fail_launch = 3;
+  expect(gcctb_run_plain(c, nullptr) == GCCTB_EDEVICE, "the failed launch is reported");
+  expect(launched == 3, "the batches after it are not queued");
+  expect(waited, "the queued batches have ended");
+  fail_launch = launched = 0;
+  gcctb_stats st{};
+  expect(gcctb_run_plain(c, &st) == GCCTB_OK && st.committed == 100 && st.batches == 4, "the next run");
+  gcctb_destroy(c);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -207,6 +231,7 @@ int main(int argc, char** argv) {
   const char* scheme = argc > 2 ? argv[2] : "";
   if (what == "alloc") load_after_failed_alloc(scheme, std::atoi(argv[3]));
   if (what == "run") run_after_failed_load(scheme, !std::strcmp(argv[3], "first"));
+  if (what == "launch") failed_launch(scheme);
   std::printf("%s\n", found.empty() ? "ok" : found.c_str());
   return found.empty() ? 0 : 1;
 }

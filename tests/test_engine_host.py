@@ -38,3 +38,9 @@ def test_run_after_failed_load(engine, scheme, when):
     """A run after a load that failed finds no transactions, not the new
     counts on buffers that are missing or too small."""
     engine("run", scheme, when)
+
+
+@pytest.mark.parametrize("scheme", ["tpl_nw", "to"])
+def test_run_waits_for_queued_batches(engine, scheme):
+    """A plain run whose launch fails returns with no batch still running."""
+    engine("launch", scheme)
