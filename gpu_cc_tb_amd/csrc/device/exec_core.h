@@ -255,6 +255,15 @@ __device__ __forceinline__ void ev_commit(const TxCtx<G>& c, const ExecArgs& a) 
   }
 }
 
+// Report an error.  In the plain form the batches behind this launch are queued
+// already: they do nothing once its number is there (txn_exec).  Its own waves
+// go on, those that start later too: every transaction of the batch runs, and
+// under the ordered schemes has its turn, as far as the error lets it.
+__device__ __forceinline__ void report_error(const ExecArgs& a, uint64_t flag) {
+  atomicOr((unsigned long long*)&a.metrics->error_flags, flag);
+  if (a.launch_no) st(&a.metrics->failed, a.launch_no);
+}
+
 // Abort bookkeeping, identical on every lane of the group (the wall clock is a
 // scalar read, so every lane of the wave sees the same value).
 //
@@ -653,7 +662,7 @@ struct TimestampOrdering {
       c.ts = group_bcast64<G>(ts);
       c.m_ts += now_ticks() - now;
       if (c.ts > tsw::TS_MAX) {
-        if ((lane_id() & (G - 1)) == 0) atomicOr((unsigned long long*)&a.metrics->error_flags, ERR_TS_OVERFLOW);
+        if ((lane_id() & (G - 1)) == 0) report_error(a, ERR_TS_OVERFLOW);
         finish_tx(c, a, now, c.ts, 0);
         return;
       }
@@ -802,7 +811,7 @@ struct Mvcc {
         p = (uint32_t)link;
       }
       if (broken) {
-        atomicOr((unsigned long long*)&a.metrics->error_flags, ERR_CHAIN_BROKEN);
+        report_error(a, ERR_CHAIN_BROKEN);
         val = 0;
         return R_OK;
       }
@@ -823,7 +832,7 @@ struct Mvcc {
       c.ts = group_bcast64<G>(ts);
       c.m_ts += now_ticks() - now;
       if (c.ts > tsw::TS_MAX) {
-        if ((lane_id() & (G - 1)) == 0) atomicOr((unsigned long long*)&a.metrics->error_flags, ERR_TS_OVERFLOW);
+        if ((lane_id() & (G - 1)) == 0) report_error(a, ERR_TS_OVERFLOW);
         finish_tx(c, a, now, c.ts, 0);
       } else {
         begin_attempt(c, now);
@@ -915,7 +924,7 @@ struct Mvcc {
     uint64_t node = wave_fetch_add(a.ctrs + CTR_POOL, nw);
     if (!commit) return;
     if (node + nw > a.pool_cap) {
-      atomicOr((unsigned long long*)&a.metrics->error_flags, ERR_POOL_OVERFLOW);
+      report_error(a, ERR_POOL_OVERFLOW);
     }
     // Install, in three steps for all of the lane's writes at once (this
     // attempt holds the uncommitted mark of every row it installs on):
@@ -1528,7 +1537,7 @@ __device__ __forceinline__ void load_tx(TxCtx<G>& c, const ExecArgs& a, uint64_t
     }
   }
   if (c.live) {
-    if (c.nops > (uint32_t)(K * G)) atomicOr((unsigned long long*)&a.metrics->error_flags, ERR_TXLEN);
+    if (c.nops > (uint32_t)(K * G)) report_error(a, ERR_TXLEN);
     c.m_idx += now_ticks() - now;
   }
 }
@@ -1538,7 +1547,7 @@ __device__ __forceinline__ void load_tx(TxCtx<G>& c, const ExecArgs& a, uint64_t
 template <int G>
 __device__ void watchdog_stop(const TxCtx<G>& c, const ExecArgs& a) {
   constexpr int K = TxCtx<G>::K;
-  if (lane_id() == 0) atomicOr((unsigned long long*)&a.metrics->error_flags, ERR_WATCHDOG);
+  if (lane_id() == 0) report_error(a, ERR_WATCHDOG);
   if (a.dbg && !c.done) {
     // per op: flags/row, the CC word through the coherent load and through an
     // atomic read, and phase/attempts
@@ -1896,9 +1905,12 @@ __global__ __launch_bounds__(MAXT) void txn_exec(ExecArgs a) {
   if constexpr (PERSIST) {
     run_persistent<S, G>(c, a);
   } else {
-    // plain form: one transaction per group; the host queues the batches
-    // without waiting for each, so one that reported an error stops the rest
-    if (a.stop_on_error && __builtin_amdgcn_readfirstlane((int)ld(&a.metrics->error_flags)) != 0) return;
+    // plain form: one transaction per group; nothing once a launch before this
+    // one reported an error (the host queues the batches without a wait each)
+    if (a.launch_no > 1) {
+      const uint32_t failed = (uint32_t)__builtin_amdgcn_readfirstlane((int)ld(&a.metrics->failed));
+      if (failed != 0 && failed != a.launch_no) return;
+    }
     const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     c.t_round = now_ticks();
     load_tx(c, a, a.slot_lo + gtid / G, c.t_round);

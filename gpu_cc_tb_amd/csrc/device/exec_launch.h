@@ -66,8 +66,7 @@ hipError_t launch_exec_g(int G, const ExecArgs& args, uint64_t nslots, int threa
   if (threads <= 0 || threads > 1024) return hipErrorInvalidValue;
   ExecArgs a = args;
   a.persist = persist ? 1u : 0u;
-  a.stop_on_error = !persist && a.slot_lo > 0;
-  if (persist) a.young_ticks = 0;  // a stream has no young phase
+  if (persist) a.launch_no = a.young_ticks = 0;  // one launch; a stream has no young phase
   // persistent launches of at most 256 threads per block take the
   // instantiation bounded by that block size (more registers, no spills);
   // whole-row mode, the event log and the latch schemes have the plain

@@ -246,6 +246,7 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
     for (uint64_t st0 = 0; st0 < r->ntx; st0 += r->batch_size, ++b) {
       const uint64_t n = std::min<uint64_t>(r->batch_size, r->ntx - st0);
       a.batch_id = (uint32_t)b;
+      a.launch_no = (uint32_t)b + 1;
       a.slot_lo = st0;
       a.slot_hi = st0 + n;
       a.young_ticks = young_ticks(n);

@@ -178,7 +178,8 @@ struct Metrics {
   uint64_t committed;
   uint64_t index_miss;
   uint64_t error_flags;
-  uint64_t pad[6];
+  uint64_t failed;  // slot 0, plain form: the launch_no of the launch that reported an error (0: none)
+  uint64_t pad[5];
 };
 constexpr int METRICS_WORDS = 16;
 // Device counters (u64 indices into ExecArgs::ctrs, each on its own 128-byte
@@ -324,7 +325,7 @@ struct ExecArgs {
   uint64_t persist_groups; // persistent form: at most this many transactions in flight (0 = device-filling)
   uint32_t open;           // persistent form: slots are admitted while the launch runs (CTR_ADMIT0)
   uint32_t persist;        // 1 in persistent launches (slots from CTR_SLOT, gates, urgent state)
-  uint32_t stop_on_error;  // plain launches after the first: do nothing once an earlier one reported an error
+  uint32_t launch_no;      // plain form: 1 for the run's first launch, 2 for the second, ... (0 in the other forms)
   uint32_t urgent_attempts; // persistent form: aborts that make a transaction urgent (0 = never)
   uint32_t backoff_exp;     // retry delay spans at most 2^backoff_exp units
   uint32_t young_ticks;     // plain form: until this long after CTR_T0 it spans at most 4 units (young_ticks())

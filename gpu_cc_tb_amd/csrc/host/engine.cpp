@@ -191,6 +191,7 @@ struct gcctb_ctx {
   gcctb::DevBuf<uint64_t> dbg;
   std::string dbg_path;
   uint64_t nranks = 0;
+  uint32_t launch_no = 0;    // plain and graph forms: the launch that is being queued, from 1
   uint64_t last_committed = 0;
   bool rows_probed = false;  // rows_out holds every op's row (persistent form)
   gcctb::DevBuf<uint64_t> tcommit;  // serving form: per-tx commit tick
@@ -331,6 +332,7 @@ class SchemeHost {
     a.metrics = ctx.metrics.p;
     a.seed = ctx.cfg.seed;
     a.batch_id = (uint32_t)batch_id;
+    a.launch_no = ctx.launch_no;
     a.backoff_ticks = ctx.cfg.backoff_ticks;
     a.tx_rank = nullptr;
     a.watchdog_ticks = ctx.watchdog_ticks;
@@ -1294,9 +1296,11 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
         hipGraph_t g = nullptr;
         HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         uint64_t batch_st = 0;
+        c->launch_no = 0;
         for (size_t i = 0; i < batches.size(); ++i) {
           const uint64_t n = batches[i];
           if (!n) continue;
+          c->launch_no++;
           c->host->Init((int)i, batch_st);
           c->host->Launch((int)i, batch_st, batch_st + n, false);
           c->host->Post((int)i, batch_st, n);
@@ -1328,6 +1332,7 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
           HIP_TRY(hipEventCreate(&e));
           c->pev.push_back(e);
         }
+        c->launch_no = (uint32_t)launches + 1;
         c->host->Init((int)i, batch_st);
         HIP_TRY(hipEventRecord(c->pev[2 * queued], s));
         c->host->Launch((int)i, batch_st, batch_st + n, false);
