@@ -1325,12 +1325,50 @@ struct Tictoc {
 // On the low-contention workload (1,048,576 transactions of 16 ops on
 // 10,485,760 rows, theta 0.1, read ratio 0.9) 88% of the ops do neither, and
 // a random load and a random atomic per op were what bounded the launch
-// (the atomics alone 0.7 ms at 23.9 G/s).  Every op's cell load is issued
-// before the first result is stored: a lane's 8 slots cost one memory latency
-// instead of 8.  That launch at 2 lanes per transaction: GaccO 1,077 -> 692 us,
-// GPUTx 1,130 -> 751 us.
+// (the atomics alone 0.7 ms at 23.9 G/s).  That launch at 2 lanes per
+// transaction: GaccO 1,077 -> 692 us, GPUTx 1,130 -> 751 us.
+//
+// Under skew a launch is the hottest row's chain of handoffs of about 1 us, and
+// a handoff is a round of the wave that holds the turn.  So:
+//  - The ready ops' cell accesses come first, then one wait for all of them,
+//    then the increments that pass the turns on, and the reads' results are
+//    stored after that.  A result that is stored before waits for its load,
+//    and for every store before it, while the turn is held.
+//  - A slot's tests have no branches, and a lane mask per slot says which are
+//    ready.  One-lane groups have 32 slots, whose state lies in scratch: there
+//    a branch saves a waiting or finished slot's reloads, and the ready ones
+//    are a bit each.
+//  - The accesses go 8 slots at a time: 32 in flight cost the registers that
+//    the other slots' state needs.
+// 30,000 transactions of 16 ops, theta 0.99, read ratio 0.5, plain form, ms at
+// 1 / 2 / 4 / 8 / 16 / 32 lanes each: 125 / 39.7 / 22.4 / 19.4 / 19.3 / 17.5 with
+// every op polling and counting and each result stored at its load; 169 / 53.6 /
+// 29.8 / 22.7 / 21.3 / 17.6 with the loads of all slots in front and the results
+// stored before the increments; 67.7 / 37.2 / 23.9 / 19.5 / 18.1 / 16.7 now.
+// 4 slots at a time: 30.3 at 4 lanes, the others within 4%.
 // ===========================================================================
+// The slots of a round whose turn has come.
+template <int K>
+struct ReadySlots {
+  bool r[K];  // a lane mask each
+  __device__ __forceinline__ void set(int k, bool x) { r[k] = x; }
+  __device__ __forceinline__ bool has(int k) const { return r[k]; }
+  __device__ __forceinline__ bool any(int b, int n) const {
+    bool x = false;
+#pragma unroll
+    for (int i = 0; i < n; ++i) x |= r[b + i];
+    return x;
+  }
+};
+template <>
+struct ReadySlots<32> {
+  uint32_t r = 0;
+  __device__ __forceinline__ void set(int k, bool x) { r |= x ? 1u << k : 0u; }
+  __device__ __forceinline__ bool has(int k) const { return (r >> k) & 1u; }
+  __device__ __forceinline__ bool any(int b, int n) const { return ((r >> b) & (uint32_t)((1ull << n) - 1)) != 0; }
+};
 struct Ordered {
+  static constexpr int CHUNK = 8;
   template <int G>
   static __device__ void round(TxCtx<G>& c, const ExecArgs& a) {
     constexpr int K = TxCtx<G>::K;
@@ -1347,56 +1385,77 @@ struct Ordered {
     if (now < c.t_resume) return;  // resting: no op can have its turn yet
     // Poll the row counter of every op that waits for one at once
     // (independent loads, one memory latency for all slots), then run the ops
-    // whose turn has come: one acquire before their cell accesses, one release
-    // before the counter increments that pass the turn on.
+    // whose turn has come.
     uint32_t seen[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const uint32_t m = c.meta[k], need = (uint32_t)c.st[k] & ~NEED_LAST;
-      seen[k] = ((m & M_VALID) && !(m & M_DONE) && need) ? ld32(turn_counter(a, c.row[k])) : 0u;
-    }
-    bool pending = false, any = false, pass = false;
-    bool ready[K];
+    ReadySlots<K> ready;
+    bool pending = false;
     uint32_t gap = 0xffffffffu;  // fewest turns any still-waiting op is away from its own
+    if constexpr (K > 16) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const uint32_t m = c.meta[k], need = (uint32_t)c.st[k] & ~NEED_LAST;
-      const bool waiting = (m & M_VALID) && !(m & M_DONE);
-      ready[k] = waiting && seen[k] >= need;
-      pending |= waiting && !ready[k];
-      any |= ready[k];
-      pass |= ready[k] && !((uint32_t)c.st[k] & NEED_LAST);
-      if (waiting && !ready[k]) {
-        const uint32_t d = need - seen[k];
+      for (int k = 0; k < K; ++k) {
+        const uint32_t m = c.meta[k], need = (uint32_t)c.st[k] & ~NEED_LAST;
+        seen[k] = ((m & M_VALID) && !(m & M_DONE) && need) ? ld32(turn_counter(a, c.row[k])) : 0u;
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const uint32_t m = c.meta[k], need = (uint32_t)c.st[k] & ~NEED_LAST;
+        if (!(m & M_VALID) || (m & M_DONE)) continue;
+        if (seen[k] >= need) {
+          ready.set(k, true);
+        } else {
+          pending = true;
+          const uint32_t d = need - seen[k];
+          gap = d < gap ? d : gap;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const uint32_t need = (uint32_t)c.st[k] & ~NEED_LAST;
+        const bool poll = ((c.meta[k] & (M_VALID | M_DONE)) == M_VALID) & (need != 0);
+        seen[k] = poll ? ld32(turn_counter(a, c.row[k])) : 0u;
+      }
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const uint32_t need = (uint32_t)c.st[k] & ~NEED_LAST;
+        const bool waiting = (c.meta[k] & (M_VALID | M_DONE)) == M_VALID;
+        const bool now_ready = waiting & (seen[k] >= need), waits = waiting & !now_ready;
+        ready.set(k, now_ready);
+        pending |= waits;
+        const uint32_t d = waits ? need - seen[k] : 0xffffffffu;
         gap = d < gap ? d : gap;
       }
     }
-    if (any) {
+    if (ready.any(0, K)) {
       order_acquire();
-      uint64_t v[K];
+      constexpr int C = K < CHUNK ? K : CHUNK;
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const uint32_t m = c.meta[k];
-        const uint32_t j = op_index<G>(k);
-        v[k] = 0;
-        if (!ready[k]) continue;
-        if (m & M_WRITE)
-          op_store(a, c.row[k], m, c.tx, j, c.op0 + j);
-        else
-          v[k] = op_load(a, c.row[k], m);
-      }
+      for (int b = 0; b < K; b += C) {
+        if (K > C && !ready.any(b, C)) continue;
+        uint64_t v[C];
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        if (!ready[k]) continue;
-        if (!(c.meta[k] & M_WRITE)) a.reads[c.op0 + op_index<G>(k)] = v[k];
-        ev_op<G>(c, a, k);
-        c.meta[k] |= M_DONE;
-      }
-      if (pass) {
+        for (int i = 0; i < C; ++i) {
+          const int k = b + i;
+          v[i] = 0;
+          if (!ready.has(k)) continue;
+          const uint32_t m = c.meta[k], j = op_index<G>(k);
+          if (m & M_WRITE)
+            op_store(a, c.row[k], m, c.tx, j, c.op0 + j);
+          else
+            v[i] = op_load(a, c.row[k], m);
+          ev_op<G>(c, a, k);
+        }
         order_release();
 #pragma unroll
-        for (int k = 0; k < K; ++k)
-          if (ready[k] && !((uint32_t)c.st[k] & NEED_LAST)) fetch_add32(turn_counter(a, c.row[k]), 1u);
+        for (int i = 0; i < C; ++i)
+          if (ready.has(b + i) && !((uint32_t)c.st[b + i] & NEED_LAST)) fetch_add32(turn_counter(a, c.row[b + i]), 1u);
+#pragma unroll
+        for (int i = 0; i < C; ++i) {
+          const int k = b + i;
+          if (!ready.has(k)) continue;
+          if (!(c.meta[k] & M_WRITE)) a.reads[c.op0 + op_index<G>(k)] = v[i];
+          c.meta[k] |= M_DONE;
+        }
       }
     }
     if (group_all<G>(!pending)) {
