@@ -279,19 +279,28 @@ __device__ __forceinline__ void report_error(const ExecArgs& a, uint64_t flag) {
 // wait, and 1024 such units would idle a transaction for seconds.
 //
 // A young plain launch (until 300 us + 4 ns per transaction after its
-// counters were reset) spans at most 4 units of at most 4 us and does not
-// raise e: the conflicts of a low-contention batch are over within that time,
-// and delays of 8 and 16 units, or of units as long as the first, crowded
-// attempt (50 us and more), were half of such a launch.  65,536 transactions
-// of 16 ops on 1,048,576 rows, theta 0.1, read ratio 0.9, 8 lanes each, us
+// counters were reset) spans at most 4 units of at most 4 us (no-wait 2PL 8
+// after a third of that time) and does not raise e: the conflicts of a
+// low-contention batch are over within that time, and delays of 8 and 16
+// units, or of units as long as the first, crowded attempt (50 us and more),
+// were half of such a launch.  65,536 transactions of 16 ops on 1,048,576 rows, theta 0.1, read ratio 0.9, 8 lanes each, us
 // with growing delays, with 4 units, with 4 units of at most 4 us: 2PL 800,
 // 435, 383; T/O 290, 300, 197; MVCC 420, 430, 330; Silo 520, 463, 383; TicToc
 // 510, 445, 367.  Units of at most 2 us: 1-4% less there, but 2PL 232 -> 296
 // on 6,007 transactions of 4 to 32 ops on 131,071 rows, read ratio 0.5.
 // A contended launch runs for tens of ms, so the aborts of its first 300 us do
-// not count (theta 0.99, read ratio 0.5 and 0.9: within 2% either way).  By
-// the age of the transaction instead, the waves that start late would each
+// not count (theta 0.99, read ratio 0.5 and 0.9: within 2% either way).
+// By the age of the transaction instead, the waves that start late would each
 // bring a burst of retries of their own: 2PL 1.5x slower at theta 0.99.
+// No-wait 2PL aborts on every lock that another holds, so a batch that covers
+// its table drowns in retries within 4 units.  12,000 transactions of 32 ops on
+// 65,536 rows, theta 0.3, read ratio 0.9, batches of 4,000, 32 lanes each: 1.05-1.27
+// ms with growing delays, 1.74 with 4 units, .80 now; 32,000 of 16 ops, theta 0,
+// read ratio 0.5, batches of 8,000: 2.31, 3.06, 1.06; 6,007 of 4 to 32 ops on
+// 131,071 rows in one static call 510, 245, 240 us.  8 units from the start: a
+// tenth more where the batch is over before the line; with the line at half
+// the time 1.25 ms in the second example.  The other schemes lose 5 to 20% to
+// longer delays.
 // Urgent state (persistent form).  A transaction that has aborted
 // ExecArgs::urgent_attempts times (256 by default: a safety net, far beyond
 // the abort counts of a healthy run) adds itself to the urgent count of every
@@ -309,7 +318,7 @@ constexpr uint64_t BACKOFF_UNIT_MAX = 5000;  // 50 us of the 100 MHz wall clock
 constexpr uint64_t YOUNG_UNIT_MAX = 400;     // 4 us, while a plain launch is young
 
 template <int G>
-__device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, uint64_t now) {
+__device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, uint64_t now, uint32_t late_exp = 2) {
   (void)now;
   const uint64_t t = now_ticks();
   const uint64_t dur = t - c.t_attempt;
@@ -319,8 +328,9 @@ __device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, ui
   uint64_t unit = dur > a.backoff_ticks ? dur : a.backoff_ticks;
   if (unit > BACKOFF_UNIT_MAX) unit = BACKOFF_UNIT_MAX;
   const uint64_t h = hash3(a.seed ^ TAG_BACKOFF, c.tx, c.attempts);
-  const bool young = a.young_ticks && t - ld(a.ctrs + CTR_T0) < a.young_ticks;
-  if (c.backoff < 2 || !young) c.backoff++;
+  const uint64_t age = a.young_ticks ? t - ld(a.ctrs + CTR_T0) : 0;
+  const bool young = age < a.young_ticks;
+  if (c.backoff < (3 * age > a.young_ticks ? late_exp : 2u) || !young) c.backoff++;
   if (young && unit > YOUNG_UNIT_MAX) unit = YOUNG_UNIT_MAX;
   const uint32_t span = 1u << (c.backoff < a.backoff_exp ? c.backoff : a.backoff_exp);
   c.t_resume = t + (h % span) * unit;
@@ -393,6 +403,7 @@ template <bool WAIT_DIE>
 struct TwoPL {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
   static constexpr uint32_t kTailShare = 2;
+  static constexpr uint32_t kLateExp = WAIT_DIE ? 2 : 3;  // exponent of a young launch's delays after its first third
   static constexpr bool kBulkRefill = true;
   static constexpr bool kSlotStash = false;
   // lock_shared (twopl.cuh:233-267), continuing from an observed word `cur`
@@ -490,7 +501,7 @@ struct TwoPL {
 #pragma unroll
           for (int k = 0; k < K; ++k)
             if (c.meta[k] & M_HELD) unlock(cc_word(a, c.row[k]), c.meta[k] & M_WRITE);
-          abort_attempt(c, a, now);
+          abort_attempt(c, a, now, kLateExp);
         } else if (group_all<G>(!pending)) {
           c.ph = PH_COMMIT;
         } else {

@@ -328,7 +328,7 @@ struct ExecArgs {
   uint32_t launch_no;      // plain form: 1 for the run's first launch, 2 for the second, ... (0 in the other forms)
   uint32_t urgent_attempts; // persistent form: aborts that make a transaction urgent (0 = never)
   uint32_t backoff_exp;     // retry delay spans at most 2^backoff_exp units
-  uint32_t young_ticks;     // plain form: until this long after CTR_T0 it spans at most 4 units (young_ticks())
+  uint32_t young_ticks;     // plain form: until this long after CTR_T0 it spans few units (young_ticks())
   uint32_t poll_ticks;      // ordered schemes: expected ticks per handoff on a row (rest pacing)
   uint32_t deep_turns;      // ordered schemes, persistent form: a wait of this many turns counts as long
   uint64_t* tcommit;       // optional, per tx: wall-clock tick of its commit (serving form)
