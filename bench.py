@@ -319,7 +319,7 @@ def main():
     b_ms = b_kern = p_ms = p_kern = 0.0
     b_launch = 0
     for s in schemes:
-        shape = autotune.lookup(s, args.theta, args.read_ratio, table)
+        shape = autotune.lookup(s, args.theta, args.read_ratio, table, rows=args.rows)
         wd = args.wd if args.wd >= 0 else shape["warp_density"]
         bs = args.bs if args.bs >= 0 else shape["block_size"]
         # the plain form runs at its own best low-contention shape

@@ -72,14 +72,29 @@ def load_table(path: str = TABLE_PATH) -> dict:
         return json.load(f)
 
 
-def lookup(scheme: str, theta: float, read_ratio: float, table: dict | None = None, key: str | None = None) -> dict:
+# Below this many rows 2PL's t0-rw and t0-ro entries, swept on 700,000 rows and
+# more, give way to t1-rw and t1-ro: a few thousand transactions cover such a
+# table, and narrow groups with wide windows then wait for one another's locks.
+# 200,000 transactions, t0 / t1 shape, ms.  Half written, 4 to 32 ops, theta
+# 0.3, no-wait: 65,536 rows 9.48 / 3.90, 131,072 5.26 / 2.25, 262,144 3.03 / 1.84,
+# 700,000 1.54 / 1.53, 1,400,000 1.07 / 1.42; 16 ops, theta 0.1: 3.78 / 2.26,
+# 2.19 / 1.88, 1.36 / 1.59, .86 / 1.44, .72 / 1.36.  Read only, theta 0.3: 65,536
+# rows 1.06 / .81, 131,072 .63 / .50, 262,144 .47 / .47, 700,000 .42 / .46.
+SMALL_TABLE = 262144
+
+
+def lookup(scheme: str, theta: float, read_ratio: float, table: dict | None = None, key: str | None = None,
+           rows: int | None = None) -> dict:
     """Tuned {warp_density, block_size, window, adaptive} for a workload (or
     for the named bucket `key`, e.g. "stream", when the table has it); the
-    default shape with a device-filling window when the table has no entry."""
+    default shape with a device-filling window when the table has no entry.
+    `rows`: the key-value table's rows, when the caller knows them (SMALL_TABLE)."""
     table = load_table() if table is None else table
     ent = table.get(scheme, {})
     if key is None or key not in ent:
         key = bucket(theta, read_ratio)
+        if rows is not None and rows < SMALL_TABLE and scheme in ("tpl_nw", "tpl_wd") and key in ("t0-rw", "t0-ro"):
+            key = "t1" + key[2:]
     if key not in ent and ent:
         # nearest measured skew with the same read bucket, else any
         buckets = [k for k in ent if k.startswith("t")]

@@ -44,7 +44,7 @@ def sweep(args) -> None:
         for rr in reads:
             w = generate(args.rows, args.txs, theta=th, read_ratio=rr)
             for scheme in args.schemes.split(","):
-                shape = autotune.lookup(scheme, th, rr)
+                shape = autotune.lookup(scheme, th, rr, rows=args.rows)
                 for b in batches:
                     with Context(scheme, rows=args.rows, warp_density=shape["warp_density"],
                                  block_size=shape["block_size"], batch_size=b) as c:
