@@ -109,6 +109,8 @@ struct CombArgs {
   uint64_t* reads;
   uint32_t* need;
   unsigned long long* combined;
+  uint32_t launch_no;      // TPC-C: the batch's launch (ExecArgs::launch_no), and
+  const uint64_t* failed;  // the launch before it that reported an error (Metrics::failed; 0: none)
 };
 constexpr uint32_t COMB_CHUNKS = 0, COMB_SUMS = 1, COMB_MULTI = 2, COMB_WORDS = 4;
 uint64_t comb_chunk_cap(uint64_t nops, uint32_t min);
@@ -154,7 +156,8 @@ hipError_t ord_filter(const IndexView& ix, const uint64_t* ops, const uint32_t* 
 // cells (cols <= 64), store its reads' results, mark its ops need = NEED_DONE
 // and add the ops run to *combined.  srow, sop: the sorted accesses.
 hipError_t gacco_combine(const CombArgs& c, const uint32_t* srow, const uint32_t* sop, hipStream_t s);
-// TPC-C, GaccO: the same for queues of updates (c.whole), one wave per queue.
+// TPC-C, GaccO: the same for queues of updates (c.whole), one wave per queue;
+// nothing once an earlier launch of the run reported an error.
 hipError_t tpcc_combine(const CombArgs& c, const uint32_t* srow, const uint32_t* sop, hipStream_t s);
 // Open form, one admitted batch sorted by (row, op) with group starts gstart
 // and row starts rstart: need[op] = base[row] + gstart[p] - rstart[p]; then

@@ -512,6 +512,8 @@ class GaccoHost : public SchemeHost {
     c.reads = ctx.reads.p;
     c.need = ctx.need.p;
     c.combined = reinterpret_cast<unsigned long long*>(ctx.comb_ctr.p + launch::COMB_WORDS / 2);
+    c.launch_no = ctx.launch_no;
+    c.failed = &ctx.metrics.p->failed;
     return c;
   }
   // per-row access queues for ops [o0, o1) in (row, transaction id) order;

@@ -26,6 +26,8 @@ int blocks(size_t bytes) {
 }
 int launched = 0;              // execution launches over some transactions
 int fail_launch = 0;           // this one fails
+int error_at = 0;              // this one reports an error
+int combined = 0;              // batches whose TPC-C queues were applied
 bool waited = true;            // the host has waited since the last launch
 std::string found;
 void expect(bool ok, const char* what) {
@@ -137,7 +139,36 @@ hipError_t exec(const ExecArgs& a, uint64_t n) {
   launched += n != 0;
   if (fail_launch && launched == fail_launch) return hipErrorLaunchFailure;
   waited = false;
+  if (a.launch_no > 1 && a.metrics->failed != 0 && a.metrics->failed != a.launch_no) return hipSuccess;  // as txn_exec
+  if (error_at && launched == error_at) {
+    a.metrics->error_flags |= ERR_WATCHDOG;
+    a.metrics->failed = a.launch_no;
+    return hipSuccess;
+  }
   a.metrics->committed += n;
+  return hipSuccess;
+}
+hipError_t exec_tpcc(int, int, const ExecArgs& a, uint64_t n, int, hipStream_t) { return exec(a, n); }
+hipError_t probe(const IndexView&, const uint64_t*, uint64_t, uint32_t*, hipStream_t, uint32_t*, uint32_t*, uint32_t,
+                 const uint32_t*, uint32_t*, uint64_t*, uint32_t) {
+  return hipSuccess;
+}
+hipError_t radix_sort_u32(uint32_t* k0, uint32_t* v0, uint32_t*, uint32_t*, uint64_t, int, uint32_t*, uint32_t** k,
+                          uint32_t** v, hipStream_t, const uint32_t*) {
+  *k = k0;
+  *v = v0;
+  return hipSuccess;
+}
+hipError_t seg_turns(const uint32_t*, const uint32_t*, uint64_t, int, uint32_t*, uint32_t*, uint32_t*, uint64_t,
+                     const CombArgs&, uint64_t*, hipStream_t, const uint32_t*) {
+  return hipSuccess;
+}
+hipError_t tpcc_combine(const CombArgs& c, const uint32_t*, const uint32_t*, hipStream_t) {
+  combined += !(c.launch_no > 1 && *c.failed != 0);  // as k_tpcc_combine
+  return hipSuccess;
+}
+hipError_t fill_u64(uint64_t* v, uint64_t n, uint64_t x, hipStream_t) {
+  for (uint64_t i = 0; i < n; ++i) v[i] = x;
   return hipSuccess;
 }
 hipError_t exec_tpl(bool, int, const ExecArgs& a, uint64_t n, int, bool, hipStream_t) { return exec(a, n); }
@@ -152,11 +183,12 @@ hipError_t exec_ordered(int, const ExecArgs& a, uint64_t n, int, bool, hipStream
 namespace {
 using namespace gcctb;
 
-gcctb_ctx* make(const char* scheme, uint64_t rows) {
+gcctb_ctx* make(const char* scheme, uint64_t rows, bool tpcc = false) {
   gcctb_config cfg{};
   cfg.cc_scheme = scheme;
   cfg.rows = rows;
-  cfg.cols = 1;
+  cfg.cols = tpcc ? TPCC_COLS : 1;
+  cfg.tpcc = tpcc;
   cfg.warp_density = 3;
   cfg.block_size = 8;
   cfg.batch_size = 1 << 16;
@@ -223,6 +255,24 @@ void failed_launch(const char* scheme) {
   expect(gcctb_run_plain(c, &st) == GCCTB_OK && st.committed == 100 && st.batches == 4, "the next run");
   gcctb_destroy(c);
 }
+
+// TPC-C under GaccO, four batches, the second reports an error: the queues of
+// the two behind it are not applied; the next run is whole.
+void tpcc_error() {
+  gcctb_ctx* c = make("gacco", 1000, true);
+  const uint64_t sizes[4] = {10, 20, 30, 40};
+  expect(load(c, 100) == GCCTB_OK, "load");
+  const std::vector<uint32_t> params(100);
+  expect(gcctb_load_params(c, params.data(), 100) == GCCTB_OK, "parameters");
+  expect(gcctb_set_batches(c, sizes, 4) == GCCTB_OK, "batches");
+  error_at = 2;
+  gcctb_stats st{};
+  expect(gcctb_run_plain(c, &st) == GCCTB_EKERNEL && st.committed == 10, "the error is reported");
+  expect(combined == 2, "the queues behind the error are left alone");
+  combined = launched = error_at = 0;
+  expect(gcctb_run_plain(c, &st) == GCCTB_OK && st.committed == 100 && combined == 4, "the next run");
+  gcctb_destroy(c);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -232,6 +282,7 @@ int main(int argc, char** argv) {
   if (what == "alloc") load_after_failed_alloc(scheme, std::atoi(argv[3]));
   if (what == "run") run_after_failed_load(scheme, !std::strcmp(argv[3], "first"));
   if (what == "launch") failed_launch(scheme);
+  if (what == "tpcc") tpcc_error();
   std::printf("%s\n", found.empty() ? "ok" : found.c_str());
   return found.empty() ? 0 : 1;
 }

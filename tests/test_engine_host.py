@@ -44,3 +44,8 @@ def test_run_after_failed_load(engine, scheme, when):
 def test_run_waits_for_queued_batches(engine, scheme):
     """A plain run whose launch fails returns with no batch still running."""
     engine("launch", scheme)
+
+
+def test_tpcc_queues_behind_an_error(engine):
+    """Each batch's combiner is told its launch and where an error shows."""
+    engine("tpcc")
