@@ -208,7 +208,7 @@ hipError_t run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, bool co
 // (pinned, read after the stream is waited for).  conflicts, combined and
 // defer (the deferral's state words) may be null.
 struct RunResult {
-  Metrics metrics;  // sums over the slots (error_flags: or)
+  Metrics metrics;  // sums over the slots (error_flags: or; failed: slot 0's)
   uint64_t conflicts, combined, deferred;
 };
 hipError_t run_end(const Metrics* metrics, const uint64_t* conflicts, const uint64_t* combined, const uint32_t* defer,

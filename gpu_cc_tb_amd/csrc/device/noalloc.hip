@@ -283,7 +283,7 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
       st.tick_khz = khz;
   }
   st.tot_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  st.batches = launches;
+  st.batches = m.failed ? m.failed : launches;  // the launches behind a failed one did nothing
   st.index_miss = m.index_miss;
   st.error_flags = m.error_flags;
   st.total_ops = r->nops;

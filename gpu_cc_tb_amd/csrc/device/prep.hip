@@ -1512,8 +1512,9 @@ __global__ void k_run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, 
 // sums field t mod 16 of every 16th slot, all its loads (whole lines per 16
 // threads) issued at once, and 16 threads add 16 sums each out of LDS.  An LDS
 // atomic per slot and field took 15-22 us.
-constexpr int RUN_FIELDS = 10;  // Metrics fields in use; the last is error_flags
-static_assert(offsetof(Metrics, error_flags) == 8 * (RUN_FIELDS - 1) && METRICS_WORDS == 16, "the fields k_run_end sums");
+constexpr int RUN_FIELDS = 11;  // Metrics fields in use: error_flags, then failed (of slot 0 alone) are the last
+static_assert(offsetof(Metrics, error_flags) == 8 * (RUN_FIELDS - 2) && offsetof(Metrics, failed) == 8 * (RUN_FIELDS - 1) &&
+                  METRICS_WORDS == 16, "the fields k_run_end sums");
 __global__ __launch_bounds__(256) void k_run_end(const Metrics* metrics, const uint64_t* conflicts,
                                                  const uint64_t* combined, const uint32_t* defer,
                                                  launch::RunResult* out) {
@@ -1522,7 +1523,7 @@ __global__ __launch_bounds__(256) void k_run_end(const Metrics* metrics, const u
   static_assert(METRIC_SLOTS % STEP == 0 && launch::CONFLICT_SLOTS == METRICS_WORDS, "no remainder");
   __shared__ uint64_t part[STEP + 1][METRICS_WORDS];
   const uint32_t f = threadIdx.x % METRICS_WORDS, g = threadIdx.x / METRICS_WORDS;
-  const bool flags = f == RUN_FIELDS - 1;
+  const bool flags = f == RUN_FIELDS - 2;
   const uint64_t* m = reinterpret_cast<const uint64_t*>(metrics) + threadIdx.x;
   uint64_t v[N];
 #pragma unroll

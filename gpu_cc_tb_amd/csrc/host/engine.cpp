@@ -1374,7 +1374,7 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
     st.pre_ms = pre;
     st.proc_ms = proc;
     st.exec_kernel_ms = proc;
-    st.batches = launches;
+    st.batches = m.failed ? m.failed : launches;  // the launches behind a failed one did nothing
     if (m.error_flags) clear_cc_state(*c);
     if (c->scheme == SCHEME_GPUTX) {
       st.ranks = c->nranks;

@@ -71,7 +71,8 @@ typedef struct gcctb_stats {
   double proc_ms;          /* execution kernels (reference "proc") */
   double tot_ms;           /* whole timed region (reference "tot") */
   double exec_kernel_ms;   /* sum of execution-kernel durations (HIP events) */
-  uint64_t batches;        /* launches of the execution kernel */
+  uint64_t batches;        /* launches of the execution kernel; after an error those up to the one
+                              that reported it */
   uint64_t ranks;          /* gputx: number of rank levels */
   uint64_t same_rank_conflicts; /* gputx: adjacent conflicting same-rank accesses */
   uint64_t index_miss;     /* ops whose key was absent from the index */
@@ -138,9 +139,11 @@ int gcctb_check_ops(const uint64_t* ops, const uint64_t* tx_off, uint64_t ntx, u
 /* Run every loaded transaction with the reference's launch structure: Init0
  * splits into batches, then per batch Init (reset / preprocess) + one kernel
  * launch, one batch after the other (benchmark_cpu/ycsb.cu:249-291, include/cc.cuh:29-36,
- * benchmark/ycsb.cu:21-111).  The host queues the batches and waits at the end.  The table keeps the result; run again to
- * continue on it.  A batch whose kernel reports an error (GCCTB_EKERNEL, e.g.
- * the per-wave watchdog, GCCTB_WATCHDOG_S seconds) ends the run; every CC
+ * benchmark/ycsb.cu:21-111).  The host queues the batches and waits at the
+ * end.  The table keeps the result; run again to continue on it.  A batch
+ * whose kernel reports an error (GCCTB_EKERNEL, e.g. the per-wave watchdog,
+ * GCCTB_WATCHDOG_S seconds) ends the run: its own transactions that the error
+ * does not concern still commit, the batches behind it do nothing.  Every CC
  * word is then cleared, so no lock or mark of an unfinished transaction
  * outlives the call (the same holds for every run and serve entry point). */
 int gcctb_run_plain(gcctb_ctx* ctx, gcctb_stats* out);

@@ -268,9 +268,10 @@ void tpcc_error() {
   error_at = 2;
   gcctb_stats st{};
   expect(gcctb_run_plain(c, &st) == GCCTB_EKERNEL && st.committed == 10, "the error is reported");
+  expect(st.batches == 2, "the count ends at the launch that reported it");
   expect(combined == 2, "the queues behind the error are left alone");
   combined = launched = error_at = 0;
-  expect(gcctb_run_plain(c, &st) == GCCTB_OK && st.committed == 100 && combined == 4, "the next run");
+  expect(gcctb_run_plain(c, &st) == GCCTB_OK && st.committed == 100 && st.batches == 4 && combined == 4, "the next run");
   gcctb_destroy(c);
 }
 }  // namespace
