@@ -10,6 +10,7 @@ import pytest
 
 import gpu_cc_tb_amd as g
 import oracle_lib as orc
+from test_zz_no_alloc import COLS, SCHEMES6, run_static
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -79,3 +80,71 @@ def test_tpcc_combiner_after_an_error(combine, launch_no, failed):
             reads[i] = orc.lib().orc_tpcc_apply(int(g.op_col(ops[i:i + 1])[0]), int(params[i]), row)
         need[:] = 0xFFFFFFFF
     assert np.array_equal(out_c, cells) and np.array_equal(out_r, reads) and np.array_equal(out_n, need)
+
+
+def _hot_first_batch(rows, n, later):
+    """One write each: n transactions on row 0, then 3 x later, each on a row of its own."""
+    keys = np.concatenate([np.zeros(n, dtype=np.uint64), 1 + np.arange(3 * later, dtype=np.uint64)])
+    return g.Ops(g.make_ops(keys, np.full(keys.size, 2), np.ones(keys.size, dtype=bool)),
+                 np.arange(keys.size + 1, dtype=np.uint64))
+
+
+HOT, LATER = 4096, 512  # 4,096 commits on one row, at least a memory latency each, outlast a wait of 50 us
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["plain", "graph"])
+@pytest.mark.parametrize("scheme", ["tpl_nw", "tpl_wd", "to", "mvcc", "silo", "tictoc", "gacco"])
+def test_batches_behind_an_error(scheme, form, monkeypatch):
+    """The first of four batches runs into its bounded wait: the three behind
+    it write nothing, commit nothing and are not counted, and once the wait is
+    long enough the next context commits them all."""
+    rows = 1 + 3 * LATER
+    w = _hot_first_batch(rows, HOT, LATER)
+    init = orc.seed_table(g.SEED, rows, 10).reshape(rows, 10)
+    for wait in ("0.00005", None):
+        if wait:
+            monkeypatch.setenv("GCCTB_WATCHDOG_S", wait)
+        else:
+            monkeypatch.delenv("GCCTB_WATCHDOG_S")
+        print(f"[error-stop] scheme={scheme} form={form} wait={wait}", flush=True)
+        with g.Context(scheme, rows=rows, warp_density=3, block_size=8) as ctx:
+            ctx.seed_table()
+            ctx.load_ops(w)
+            ctx.set_batches([HOT, LATER, LATER, LATER])
+            st = ctx.run(form, check=False)
+            table = ctx.fetch()["table"].reshape(rows, 10)
+            changed = np.any(table != init, axis=1)[1:]
+            if wait:
+                assert st["rc"] == -6 and st["error_flags"] & 16
+                assert st["batches"] == 1 and st["committed"] < HOT
+                assert not np.any(changed), "a batch behind the error ran"
+                assert not np.any(ctx.fetch_cc())
+            else:
+                assert st["rc"] == 0 and st["batches"] == 4 and st["committed"] == w.ntx and np.all(changed)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme", SCHEMES6)
+def test_static_batches_behind_an_error(scheme, monkeypatch):
+    """The same through gcctb_run_plain_static, whose calls share their words:
+    the batches behind the error leave the table alone, and the call
+    after it runs whole."""
+    rows = 1 + 3 * LATER
+    w = _hot_first_batch(rows, HOT, LATER)
+    init = orc.seed_table(g.SEED, rows, COLS).reshape(rows, COLS)
+    call = g.run_plain_static
+    monkeypatch.setattr(g, "run_plain_static", lambda *a, **k: call(*a, **k, check=False))
+    for wait in ("0.00005", None):
+        if wait:
+            monkeypatch.setenv("GCCTB_WATCHDOG_S", wait)
+        else:
+            monkeypatch.delenv("GCCTB_WATCHDOG_S")
+        print(f"[error-stop] static scheme={scheme} wait={wait}", flush=True)
+        st, res = run_static(scheme, rows, w, HOT, 3, 8)
+        changed = np.any(res["table"].reshape(rows, COLS) != init, axis=1)[1:]
+        if wait:
+            assert st["rc"] == -6 and st["error_flags"] & 16 and st["batches"] == 1 and st["committed"] < HOT
+            assert not np.any(changed)
+        else:
+            assert st["rc"] == 0 and st["batches"] == 2 and st["committed"] == w.ntx and np.all(changed)
