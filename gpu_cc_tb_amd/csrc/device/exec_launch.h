@@ -33,7 +33,8 @@ hipError_t launch_one(const ExecArgs& a, uint64_t nslots, int threads, hipStream
     int per_cu = 0, cus = 0, dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    // a constant of the kernel and the block size (0: not asked for yet)
+    // a constant of the kernel and the block size, on every device that the
+    // library's one code object (gfx950) runs on (0: not asked for yet)
     static std::atomic<int> occupancy[MAXT / 32 + 1];
     std::atomic<int>& known = occupancy[(threads + 31) / 32];
     per_cu = known.load(std::memory_order_relaxed);

@@ -971,12 +971,6 @@ __global__ __launch_bounds__(BT) void k_seg_tiles(const KT* key, const uint32_t*
   if (threadIdx.x == 0) summ[blockIdx.x] = make_uint4(total.row, total.group, total.cnt, 0u);
 }
 
-// need[op] (op = val & OPID_MASK) of every access that waits or is waited
-// for; the others keep NEED_FREE.  The counter of a row where that happens is
-// set to 0 at the row's first access.  comb.min > 0: every row queue of at
-// least comb.min accesses is listed for its combiner (comb_list).
-// conflicts (GPUTx): same-row neighbours of equal key (row and rank) where
-// either writes, added to CONFLICT_SLOTS counters on lines of their own.
 // The row queues of a thread's accesses that end in it, filed block by block:
 // one add per counter and block (a queue per atomic would pile onto them).
 __device__ __forceinline__ uint32_t block_file(uint32_t n, uint32_t* ctr) {  // n places for this thread
@@ -1003,6 +997,12 @@ __device__ __forceinline__ uint32_t block_file(uint32_t n, uint32_t* ctr) {  // 
 }
 constexpr uint32_t CB_BT = 256;  // accesses per combiner chunk, one per thread
 
+// need[op] (op = val & OPID_MASK) of every access that waits or is waited
+// for; the others keep NEED_FREE.  The counter of a row where that happens is
+// set to 0 at the row's first access.  comb.min > 0: every row queue of at
+// least comb.min accesses is listed for its combiner (CombArgs).
+// conflicts (GPUTx): same-row neighbours of equal key (row and rank) where
+// either writes, added to CONFLICT_SLOTS counters on lines of their own.
 template <class KT, int TT_ITEMS>
 __global__ __launch_bounds__(BT) void k_seg_turns(const KT* key, const uint32_t* val, uint64_t n, int rb,
                                                   const uint4* summ, uint32_t* need, uint32_t* counters,
@@ -1470,8 +1470,6 @@ __global__ void k_reset_rows(const uint32_t* rows, uint64_t n, uint64_t nrows_ta
     if (vprev) dev::st32(vprev + w, 0);
   }
 }
-// Start of a run: metrics (and the hot-key counts of a persistent run) to
-// zero, and, with `counters`, what k_batch_begin and k_persist_begin set.
 __device__ __forceinline__ void reset_batch(uint64_t* ctrs) {
   const int i = threadIdx.x;
   if (i == 0) {
@@ -1495,6 +1493,8 @@ __device__ __forceinline__ void reset_admission(uint64_t* ctrs) {
 }
 __global__ void k_batch_begin(uint64_t* ctrs) { reset_batch(ctrs); }
 __global__ void k_persist_begin(uint64_t* ctrs) { reset_admission(ctrs); }
+// Start of a run: metrics (and the hot-key counts of a persistent run) to
+// zero, and, with `counters`, what k_batch_begin and k_persist_begin set.
 __global__ void k_run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, int counters) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
   for (uint32_t k = i; k < (uint32_t)METRIC_SLOTS * METRICS_WORDS; k += step) metrics[k] = 0;
@@ -1655,11 +1655,6 @@ namespace launch {
 #define GC_LAUNCH(kern, n, ...)                                                    \
   do {                                                                            \
     hipLaunchKernelGGL(kern, dim3(grid_stride_blocks(n)), dim3(BT), 0, s, __VA_ARGS__); \
-    return hipGetLastError();                                                     \
-  } while (0)
-#define GC_LAUNCH_REDUCE(kern, n, ...)                                            \
-  do {                                                                            \
-    hipLaunchKernelGGL(kern, dim3(reduce_blocks(n)), dim3(BT), 0, s, __VA_ARGS__); \
     return hipGetLastError();                                                     \
   } while (0)
 

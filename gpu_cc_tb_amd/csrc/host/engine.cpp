@@ -243,12 +243,6 @@ class SchemeHost {
   virtual void PrepStream() {}
   // Persistent form: restore the words every transaction of the stream touched.
   virtual void PostStream() { Post(0, 0, ctx.ntx); }
-  // Serving form: prepare one launch over transactions whose ops are [o0, o1).
-  virtual void PrepLaunch(uint64_t o0, uint64_t o1) {
-    (void)o0;
-    (void)o1;
-    HIP_TRY(launch::batch_begin(ctx.ctrs.p, ctx.stream));
-  }
   // Serving form, open launch: reset the counters of a launch whose
   // transactions are admitted while it runs (on the launch's stream).
   virtual void PrepOpen() {
@@ -264,8 +258,8 @@ class SchemeHost {
   }
   // True when the open launch reads every op's row from rows_out (PrepAdmit wrote it).
   virtual bool OpenRowsProbed() const { return ctx.probe_pass >= 0 ? ctx.probe_pass != 0 : WantsProbePass(); }
-  // True when PrepStream / PrepLaunch leave the row of every op they cover in
-  // rows_out, so the persistent and serving forms need no probe pass of their own.
+  // True when PrepStream leaves the row of every op in rows_out, so the
+  // persistent form needs no probe pass of its own.
   virtual bool ProbesRows() const { return false; }
   // Persistent and serving forms: whether a probe pass before the launch
   // beats looking rows up in the index as each transaction is taken (one
@@ -466,7 +460,6 @@ class GaccoHost : public SchemeHost {
   // the same as batch after batch.
   void PrepStream() override { prep_range(0, ctx.nops, true); }
   void PostStream() override {}
-  void PrepLaunch(uint64_t o0, uint64_t o1) override { prep_range(o0, o1, false); }
   bool ProbesRows() const override { return !ctx.ix.dense; }
   // Open launch: every row's queue starts empty; each admitted batch's
   // accesses queue behind those of the batches admitted before it, in
