@@ -109,8 +109,7 @@ struct CombArgs {
   uint64_t* reads;
   uint32_t* need;
   unsigned long long* combined;
-  uint32_t launch_no;      // TPC-C: the batch's launch (ExecArgs::launch_no), and
-  const uint64_t* failed;  // the launch before it that reported an error (Metrics::failed; 0: none)
+  const uint64_t* failed;  // TPC-C: the run's launch that reported an error (Metrics::failed; 0: none)
 };
 constexpr uint32_t COMB_CHUNKS = 0, COMB_SUMS = 1, COMB_MULTI = 2, COMB_WORDS = 4;
 uint64_t comb_chunk_cap(uint64_t nops, uint32_t min);

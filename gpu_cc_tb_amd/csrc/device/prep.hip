@@ -1354,9 +1354,8 @@ __device__ __forceinline__ uint64_t tpcc_run(uint32_t kind, uint32_t param, uint
   return mine;
 }
 __global__ __launch_bounds__(TC_BT) void k_tpcc_combine(launch::CombArgs c, const uint32_t* srow, const uint32_t* sop) {
-  // the batch's launch will do nothing either (txn_exec)
-  if (c.launch_no > 1 && dev::ld(c.failed) != 0) return;
-  const uint32_t nq = min(c.ctr[launch::COMB_CHUNKS], c.chunk_cap);
+  // after an error no queue counts, as the batch's launch will do nothing either (txn_exec)
+  const uint32_t nq = min(c.ctr[launch::COMB_CHUNKS], *c.failed ? 0u : c.chunk_cap);
   const uint32_t lane = threadIdx.x % 64;
   for (uint32_t x = (blockIdx.x * TC_BT + threadIdx.x) / 64; x < nq; x += gridDim.x * (TC_BT / 64)) {
     const uint4 q = c.chunks[x];

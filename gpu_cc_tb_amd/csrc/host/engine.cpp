@@ -505,7 +505,6 @@ class GaccoHost : public SchemeHost {
     c.reads = ctx.reads.p;
     c.need = ctx.need.p;
     c.combined = reinterpret_cast<unsigned long long*>(ctx.comb_ctr.p + launch::COMB_WORDS / 2);
-    c.launch_no = ctx.launch_no;
     c.failed = &ctx.metrics.p->failed;
     return c;
   }

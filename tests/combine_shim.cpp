@@ -26,7 +26,7 @@ struct Dev {
 // nrows rows of TPCC_COLS.  Returns a HIP error, cells / reads / need changed in place.
 extern "C" int combine_queues(uint32_t nq, const uint32_t* lens, const uint32_t* srow, const uint32_t* sop, uint32_t nops,
                               const uint64_t* ops, const uint32_t* params, uint64_t nrows, uint64_t* cells,
-                              uint64_t* reads, uint32_t* need, uint32_t launch_no, uint64_t failed) {
+                              uint64_t* reads, uint32_t* need, uint64_t failed) {
   std::vector<uint4> chunks(nq);
   for (uint32_t q = 0, at = 0; q < nq; at += lens[q++]) chunks[q] = make_uint4(at, lens[q], 0u, 0u);
   const uint32_t ctr[launch::COMB_WORDS] = {nq};
@@ -58,7 +58,6 @@ extern "C" int combine_queues(uint32_t nq, const uint32_t* lens, const uint32_t*
   c.cols = TPCC_COLS;
   c.reads = static_cast<uint64_t*>(d_reads.p);
   c.need = static_cast<uint32_t*>(d_need.p);
-  c.launch_no = launch_no;
   c.failed = static_cast<uint64_t*>(d_failed.p);
   e = launch::tpcc_combine(c, static_cast<uint32_t*>(d_srow.p), static_cast<uint32_t*>(d_sop.p), nullptr);
   if (e == hipSuccess) e = hipDeviceSynchronize();

@@ -164,7 +164,7 @@ hipError_t seg_turns(const uint32_t*, const uint32_t*, uint64_t, int, uint32_t*,
   return hipSuccess;
 }
 hipError_t tpcc_combine(const CombArgs& c, const uint32_t*, const uint32_t*, hipStream_t) {
-  combined += !(c.launch_no > 1 && *c.failed != 0);  // as k_tpcc_combine
+  combined += *c.failed == 0;  // as k_tpcc_combine
   return hipSuccess;
 }
 hipError_t fill_u64(uint64_t* v, uint64_t n, uint64_t x, hipStream_t) {

@@ -47,5 +47,5 @@ def test_run_waits_for_queued_batches(engine, scheme):
 
 
 def test_tpcc_queues_behind_an_error(engine):
-    """Each batch's combiner is told its launch and where an error shows."""
+    """Each batch's combiner is told where an error shows."""
     engine("tpcc")

@@ -54,13 +54,13 @@ def combine(tmp_path_factory):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("launch_no,failed", [(1, 0), (2, 0), (2, 1), (7, 3)])
-def test_tpcc_combiner_after_an_error(combine, launch_no, failed):
+@pytest.mark.parametrize("failed", [0, 1, 3])
+def test_tpcc_combiner_after_an_error(combine, failed):
     """TPC-C under GaccO applies a batch's queues before its launch: not once an
     earlier launch has reported an error."""
     lens = np.array([70, 3], dtype=np.uint32)
     nops, rows = int(lens.sum()), 4
-    rng = np.random.default_rng(launch_no * 10 + failed)
+    rng = np.random.default_rng(failed)
     w = g.tpcc_generate(1, nops, new_order=False, seed=3)
     first = w.tx_off[:-1].astype(np.int64)  # each payment's warehouse update
     ops, params = np.ascontiguousarray(w.ops[first]), np.ascontiguousarray(w.params[first])
@@ -70,9 +70,9 @@ def test_tpcc_combiner_after_an_error(combine, launch_no, failed):
     reads, need = np.full(nops, 7, dtype=np.uint64), np.full(nops, 5, dtype=np.uint32)
     out_c, out_r, out_n = cells.copy(), reads.copy(), need.copy()
     ptr = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
-    print(f"[error-stop] combiner launch={launch_no} failed={failed}", flush=True)
+    print(f"[error-stop] combiner failed={failed}", flush=True)
     rc = combine(C.c_uint32(2), ptr(lens), ptr(srow), ptr(sop), C.c_uint32(nops), ptr(ops), ptr(params), C.c_uint64(rows),
-                 ptr(out_c), ptr(out_r), ptr(out_n), C.c_uint32(launch_no), C.c_uint64(failed))
+                 ptr(out_c), ptr(out_r), ptr(out_n), C.c_uint64(failed))
     assert rc == 0
     if not failed:
         for i in range(nops):
