@@ -259,9 +259,13 @@ __device__ __forceinline__ void ev_commit(const TxCtx<G>& c, const ExecArgs& a) 
 // already: they do nothing once its number is there (txn_exec).  Its own waves
 // go on, those that start later too: every transaction of the batch runs, and
 // under the ordered schemes has its turn, as far as the error lets it.
-__device__ __forceinline__ void report_error(const ExecArgs& a, uint64_t flag) {
-  atomicOr((unsigned long long*)&a.metrics->error_flags, flag);
-  if (a.launch_no) st(&a.metrics->failed, a.launch_no);
+// Flags and number are the halves of one word, each written by itself: as one
+// 64-bit value they took MVCC's persistent kernels past 256 and 168 registers,
+// a wave per SIMD less (4 lanes: 1,540 -> 1,850 us).
+__device__ __forceinline__ void report_error(const ExecArgs& a, uint32_t flag) {
+  uint32_t* w = reinterpret_cast<uint32_t*>(&a.metrics->error_flags);
+  atomicOr(w, flag);
+  st32(w + 1, a.launch_no);
 }
 
 // Abort bookkeeping, identical on every lane of the group (the wall clock is a
@@ -317,8 +321,8 @@ __device__ __forceinline__ void urgent_add(const ExecArgs& a, uint64_t delta) {
 constexpr uint64_t BACKOFF_UNIT_MAX = 5000;  // 50 us of the 100 MHz wall clock
 constexpr uint64_t YOUNG_UNIT_MAX = 400;     // 4 us, while a plain launch is young
 
-template <int G>
-__device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, uint64_t now, uint32_t late_exp = 2) {
+template <bool NO_WAIT_2PL = false, int G>
+__device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, uint64_t now) {
   (void)now;
   const uint64_t t = now_ticks();
   const uint64_t dur = t - c.t_attempt;
@@ -328,9 +332,15 @@ __device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, ui
   uint64_t unit = dur > a.backoff_ticks ? dur : a.backoff_ticks;
   if (unit > BACKOFF_UNIT_MAX) unit = BACKOFF_UNIT_MAX;
   const uint64_t h = hash3(a.seed ^ TAG_BACKOFF, c.tx, c.attempts);
-  const uint64_t age = a.young_ticks ? t - ld(a.ctrs + CTR_T0) : 0;
-  const bool young = age < a.young_ticks;
-  if (c.backoff < (3 * age > a.young_ticks ? late_exp : 2u) || !young) c.backoff++;
+  bool young, late = false;
+  if constexpr (NO_WAIT_2PL) {
+    const uint64_t age = a.young_ticks ? t - ld(a.ctrs + CTR_T0) : 0;
+    young = age < a.young_ticks;
+    late = 3 * age > a.young_ticks;
+  } else {  // (no age to keep: two registers more are a wave per SIMD less in MVCC's persistent kernels)
+    young = a.young_ticks && t - ld(a.ctrs + CTR_T0) < a.young_ticks;
+  }
+  if (c.backoff < (late ? 3u : 2u) || !young) c.backoff++;
   if (young && unit > YOUNG_UNIT_MAX) unit = YOUNG_UNIT_MAX;
   const uint32_t span = 1u << (c.backoff < a.backoff_exp ? c.backoff : a.backoff_exp);
   c.t_resume = t + (h % span) * unit;
@@ -403,7 +413,6 @@ template <bool WAIT_DIE>
 struct TwoPL {
   static constexpr bool kRestInOps = false;  // t_resume paces restarts only (PH_START)
   static constexpr uint32_t kTailShare = 2;
-  static constexpr uint32_t kLateExp = WAIT_DIE ? 2 : 3;  // exponent of a young launch's delays after its first third
   static constexpr bool kBulkRefill = true;
   static constexpr bool kSlotStash = false;
   // lock_shared (twopl.cuh:233-267), continuing from an observed word `cur`
@@ -501,7 +510,7 @@ struct TwoPL {
 #pragma unroll
           for (int k = 0; k < K; ++k)
             if (c.meta[k] & M_HELD) unlock(cc_word(a, c.row[k]), c.meta[k] & M_WRITE);
-          abort_attempt(c, a, now, kLateExp);
+          abort_attempt<!WAIT_DIE>(c, a, now);
         } else if (group_all<G>(!pending)) {
           c.ph = PH_COMMIT;
         } else {
@@ -1984,7 +1993,7 @@ __global__ __launch_bounds__(MAXT) void txn_exec(ExecArgs a) {
     // plain form: one transaction per group; nothing once a launch before this
     // one reported an error (the host queues the batches without a wait each)
     if (a.launch_no > 1) {
-      const uint32_t failed = (uint32_t)__builtin_amdgcn_readfirstlane((int)ld(&a.metrics->failed));
+      const uint32_t failed = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ld(&a.metrics->error_flags) >> 32));
       if (failed != 0 && failed != a.launch_no) return;
     }
     const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;

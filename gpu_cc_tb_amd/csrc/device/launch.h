@@ -109,7 +109,7 @@ struct CombArgs {
   uint64_t* reads;
   uint32_t* need;
   unsigned long long* combined;
-  const uint64_t* failed;  // TPC-C: the run's launch that reported an error (Metrics::failed; 0: none)
+  const uint64_t* error;   // TPC-C: the run's error word (Metrics::error_flags; 0: none so far)
 };
 constexpr uint32_t COMB_CHUNKS = 0, COMB_SUMS = 1, COMB_MULTI = 2, COMB_WORDS = 4;
 uint64_t comb_chunk_cap(uint64_t nops, uint32_t min);
@@ -207,8 +207,9 @@ hipError_t run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, bool co
 // (pinned, read after the stream is waited for).  conflicts, combined and
 // defer (the deferral's state words) may be null.
 struct RunResult {
-  Metrics metrics;  // sums over the slots (error_flags: or; failed: slot 0's)
+  Metrics metrics;  // sums over the slots (error_flags: or, flags alone)
   uint64_t conflicts, combined, deferred;
+  uint64_t failed;  // plain form: the launch that reported an error, from 1 (0: none)
 };
 hipError_t run_end(const Metrics* metrics, const uint64_t* conflicts, const uint64_t* combined, const uint32_t* defer,
                    RunResult* out, hipStream_t s);

@@ -175,7 +175,7 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
   const auto t0 = std::chrono::steady_clock::now();
   hipStream_t s = static_cast<hipStream_t>(r->stream);
   Metrics m{};
-  uint64_t launches = 0;
+  uint64_t launches = 0, failed = 0;
   try {
     uint64_t* base = nullptr;
     NA_TRY(scratch_ptr(&base));
@@ -265,6 +265,7 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
     NA_TRY(hipMemcpyAsync(&res, metrics, sizeof res, hipMemcpyDeviceToHost, s));
     NA_TRY(hipStreamSynchronize(s));
     m = res.metrics;
+    failed = res.failed;
   } catch (const NaFail& f) {
     return set_error(GCCTB_EDEVICE, std::string("HIP error: ") + hipGetErrorString(f.err) + " in " + f.where);
   }
@@ -283,7 +284,7 @@ extern "C" int gcctb_run_plain_static(const gcctb_static_run* r, gcctb_stats* ou
       st.tick_khz = khz;
   }
   st.tot_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  st.batches = m.failed ? m.failed : launches;  // the launches behind a failed one did nothing
+  st.batches = failed ? failed : launches;  // the launches behind a failed one did nothing
   st.index_miss = m.index_miss;
   st.error_flags = m.error_flags;
   st.total_ops = r->nops;

@@ -1355,7 +1355,7 @@ __device__ __forceinline__ uint64_t tpcc_run(uint32_t kind, uint32_t param, uint
 }
 __global__ __launch_bounds__(TC_BT) void k_tpcc_combine(launch::CombArgs c, const uint32_t* srow, const uint32_t* sop) {
   // after an error no queue counts, as the batch's launch will do nothing either (txn_exec)
-  const uint32_t nq = min(c.ctr[launch::COMB_CHUNKS], *c.failed ? 0u : c.chunk_cap);
+  const uint32_t nq = min(c.ctr[launch::COMB_CHUNKS], *c.error ? 0u : c.chunk_cap);
   const uint32_t lane = threadIdx.x % 64;
   for (uint32_t x = (blockIdx.x * TC_BT + threadIdx.x) / 64; x < nq; x += gridDim.x * (TC_BT / 64)) {
     const uint4 q = c.chunks[x];
@@ -1511,9 +1511,8 @@ __global__ void k_run_begin(uint64_t* metrics, uint32_t* defer, uint64_t* ctrs, 
 // sums field t mod 16 of every 16th slot, all its loads (whole lines per 16
 // threads) issued at once, and 16 threads add 16 sums each out of LDS.  An LDS
 // atomic per slot and field took 15-22 us.
-constexpr int RUN_FIELDS = 11;  // Metrics fields in use: error_flags, then failed (of slot 0 alone) are the last
-static_assert(offsetof(Metrics, error_flags) == 8 * (RUN_FIELDS - 2) && offsetof(Metrics, failed) == 8 * (RUN_FIELDS - 1) &&
-                  METRICS_WORDS == 16, "the fields k_run_end sums");
+constexpr int RUN_FIELDS = 10;  // Metrics fields in use; the last is error_flags
+static_assert(offsetof(Metrics, error_flags) == 8 * (RUN_FIELDS - 1) && METRICS_WORDS == 16, "the fields k_run_end sums");
 __global__ __launch_bounds__(256) void k_run_end(const Metrics* metrics, const uint64_t* conflicts,
                                                  const uint64_t* combined, const uint32_t* defer,
                                                  launch::RunResult* out) {
@@ -1522,7 +1521,7 @@ __global__ __launch_bounds__(256) void k_run_end(const Metrics* metrics, const u
   static_assert(METRIC_SLOTS % STEP == 0 && launch::CONFLICT_SLOTS == METRICS_WORDS, "no remainder");
   __shared__ uint64_t part[STEP + 1][METRICS_WORDS];
   const uint32_t f = threadIdx.x % METRICS_WORDS, g = threadIdx.x / METRICS_WORDS;
-  const bool flags = f == RUN_FIELDS - 2;
+  const bool flags = f == RUN_FIELDS - 1;
   const uint64_t* m = reinterpret_cast<const uint64_t*>(metrics) + threadIdx.x;
   uint64_t v[N];
 #pragma unroll
@@ -1542,7 +1541,8 @@ __global__ __launch_bounds__(256) void k_run_end(const Metrics* metrics, const u
     uint64_t y = 0;
 #pragma unroll
     for (int i = 0; i < STEP; ++i) y = flags ? y | part[i][f] : y + part[i][f];
-    dev::st(o + f, y);
+    dev::st(o + f, flags ? (uint32_t)y : y);
+    if (flags) dev::st(&out->failed, y >> 32);
   }
   if (threadIdx.x == 0) {
     uint64_t c = 0;

@@ -177,9 +177,8 @@ struct Metrics {
   uint64_t index_duration;
   uint64_t committed;
   uint64_t index_miss;
-  uint64_t error_flags;
-  uint64_t failed;  // slot 0, plain form: the launch_no of the launch that reported an error (0: none)
-  uint64_t pad[5];
+  uint64_t error_flags;  // on the device, plain form: the launch_no of the launch that reported them in the high half
+  uint64_t pad[6];
 };
 constexpr int METRICS_WORDS = 16;
 // Device counters (u64 indices into ExecArgs::ctrs, each on its own 128-byte
@@ -216,11 +215,11 @@ constexpr uint32_t ADMIT_CLOSED = 1u << 31;
 constexpr int METRIC_SLOTS = 256;
 
 // error_flags bits
-constexpr uint64_t ERR_TS_OVERFLOW = 1;     // 31-bit timestamp space exhausted
-constexpr uint64_t ERR_POOL_OVERFLOW = 2;   // MVCC version pool full
-constexpr uint64_t ERR_CHAIN_BROKEN = 4;    // MVCC chain ended before a visible version
-constexpr uint64_t ERR_TXLEN = 8;           // transaction longer than the kernel's slots
-constexpr uint64_t ERR_WATCHDOG = 16;       // a wave exceeded the watchdog time and gave up
+constexpr uint32_t ERR_TS_OVERFLOW = 1;     // 31-bit timestamp space exhausted
+constexpr uint32_t ERR_POOL_OVERFLOW = 2;   // MVCC version pool full
+constexpr uint32_t ERR_CHAIN_BROKEN = 4;    // MVCC chain ended before a visible version
+constexpr uint32_t ERR_TXLEN = 8;           // transaction longer than the kernel's slots
+constexpr uint32_t ERR_WATCHDOG = 16;       // a wave exceeded the watchdog time and gave up
 
 // ---------------------------------------------------------------------------
 // Key -> row index with Find's contract (include/index.cuh:74-91): a key's

@@ -505,7 +505,7 @@ class GaccoHost : public SchemeHost {
     c.reads = ctx.reads.p;
     c.need = ctx.need.p;
     c.combined = reinterpret_cast<unsigned long long*>(ctx.comb_ctr.p + launch::COMB_WORDS / 2);
-    c.failed = &ctx.metrics.p->failed;
+    c.error = &ctx.metrics.p->error_flags;
     return c;
   }
   // per-row access queues for ops [o0, o1) in (row, transaction id) order;
@@ -1366,7 +1366,7 @@ static int run_form(gcctb_ctx* c, gcctb_stats* out, RunForm form) {
     st.pre_ms = pre;
     st.proc_ms = proc;
     st.exec_kernel_ms = proc;
-    st.batches = m.failed ? m.failed : launches;  // the launches behind a failed one did nothing
+    st.batches = c->h_run->failed ? c->h_run->failed : launches;  // the launches behind a failed one did nothing
     if (m.error_flags) clear_cc_state(*c);
     if (c->scheme == SCHEME_GPUTX) {
       st.ranks = c->nranks;

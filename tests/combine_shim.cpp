@@ -26,11 +26,11 @@ struct Dev {
 // nrows rows of TPCC_COLS.  Returns a HIP error, cells / reads / need changed in place.
 extern "C" int combine_queues(uint32_t nq, const uint32_t* lens, const uint32_t* srow, const uint32_t* sop, uint32_t nops,
                               const uint64_t* ops, const uint32_t* params, uint64_t nrows, uint64_t* cells,
-                              uint64_t* reads, uint32_t* need, uint64_t failed) {
+                              uint64_t* reads, uint32_t* need, uint64_t error) {
   std::vector<uint4> chunks(nq);
   for (uint32_t q = 0, at = 0; q < nq; at += lens[q++]) chunks[q] = make_uint4(at, lens[q], 0u, 0u);
   const uint32_t ctr[launch::COMB_WORDS] = {nq};
-  Dev d_chunks, d_ctr, d_srow, d_sop, d_ops, d_params, d_cells, d_reads, d_need, d_failed;
+  Dev d_chunks, d_ctr, d_srow, d_sop, d_ops, d_params, d_cells, d_reads, d_need, d_error;
   hipError_t e = hipSuccess;
   auto put = [&](Dev& d, const void* p, size_t n) {
     if (e == hipSuccess) e = d.put(p, n);
@@ -44,7 +44,7 @@ extern "C" int combine_queues(uint32_t nq, const uint32_t* lens, const uint32_t*
   put(d_cells, cells, nrows * TPCC_COLS * 8);
   put(d_reads, reads, nops * 8ull);
   put(d_need, need, nops * 4ull);
-  put(d_failed, &failed, 8);
+  put(d_error, &error, 8);
   if (e != hipSuccess) return (int)e;
   launch::CombArgs c{};
   c.min = 2;
@@ -58,7 +58,7 @@ extern "C" int combine_queues(uint32_t nq, const uint32_t* lens, const uint32_t*
   c.cols = TPCC_COLS;
   c.reads = static_cast<uint64_t*>(d_reads.p);
   c.need = static_cast<uint32_t*>(d_need.p);
-  c.failed = static_cast<uint64_t*>(d_failed.p);
+  c.error = static_cast<uint64_t*>(d_error.p);
   e = launch::tpcc_combine(c, static_cast<uint32_t*>(d_srow.p), static_cast<uint32_t*>(d_sop.p), nullptr);
   if (e == hipSuccess) e = hipDeviceSynchronize();
   if (e == hipSuccess) e = hipMemcpy(cells, d_cells.p, nrows * TPCC_COLS * 8, hipMemcpyDeviceToHost);

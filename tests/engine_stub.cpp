@@ -127,6 +127,8 @@ hipError_t run_begin(uint64_t* m, uint32_t*, uint64_t*, bool, hipStream_t) {
 hipError_t run_end(const Metrics* m, const uint64_t*, const uint64_t*, const uint32_t*, RunResult* out, hipStream_t) {
   *out = RunResult{};
   out->metrics = m[0];
+  out->metrics.error_flags &= 0xffffffffu;
+  out->failed = m[0].error_flags >> 32;
   return hipSuccess;
 }
 uint32_t defer_threshold(uint64_t, uint64_t, uint32_t) { return 2; }
@@ -139,10 +141,10 @@ hipError_t exec(const ExecArgs& a, uint64_t n) {
   launched += n != 0;
   if (fail_launch && launched == fail_launch) return hipErrorLaunchFailure;
   waited = false;
-  if (a.launch_no > 1 && a.metrics->failed != 0 && a.metrics->failed != a.launch_no) return hipSuccess;  // as txn_exec
+  const uint64_t failed = a.metrics->error_flags >> 32;
+  if (a.launch_no > 1 && failed != 0 && failed != a.launch_no) return hipSuccess;  // as txn_exec
   if (error_at && launched == error_at) {
-    a.metrics->error_flags |= ERR_WATCHDOG;
-    a.metrics->failed = a.launch_no;
+    a.metrics->error_flags |= (uint64_t)a.launch_no << 32 | ERR_WATCHDOG;
     return hipSuccess;
   }
   a.metrics->committed += n;
@@ -164,7 +166,7 @@ hipError_t seg_turns(const uint32_t*, const uint32_t*, uint64_t, int, uint32_t*,
   return hipSuccess;
 }
 hipError_t tpcc_combine(const CombArgs& c, const uint32_t*, const uint32_t*, hipStream_t) {
-  combined += *c.failed == 0;  // as k_tpcc_combine
+  combined += *c.error == 0;  // as k_tpcc_combine
   return hipSuccess;
 }
 hipError_t fill_u64(uint64_t* v, uint64_t n, uint64_t x, hipStream_t) {
