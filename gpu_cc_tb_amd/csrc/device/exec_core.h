@@ -334,10 +334,13 @@ __device__ __forceinline__ void abort_attempt(TxCtx<G>& c, const ExecArgs& a, ui
   const uint64_t h = hash3(a.seed ^ TAG_BACKOFF, c.tx, c.attempts);
   bool young, late = false;
   if constexpr (NO_WAIT_2PL) {
-    const uint64_t age = a.young_ticks ? t - ld(a.ctrs + CTR_T0) : 0;
-    young = age < a.young_ticks;
-    late = 3 * age > a.young_ticks;
-  } else {  // (no age to keep: two registers more are a wave per SIMD less in MVCC's persistent kernels)
+    young = false;
+    if (a.young_ticks) {  // the plain form
+      const uint64_t age = t - ld(a.ctrs + CTR_T0);
+      young = age < a.young_ticks;
+      late = 3 * age > a.young_ticks;
+    }
+  } else {  // (no age to keep)
     young = a.young_ticks && t - ld(a.ctrs + CTR_T0) < a.young_ticks;
   }
   if (c.backoff < (late ? 3u : 2u) || !young) c.backoff++;
