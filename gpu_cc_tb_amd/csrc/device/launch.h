@@ -82,7 +82,8 @@ hipError_t access_group_flags(const uint32_t* srow, const uint32_t* sop, uint64_
 // op id (op_ids).  need[op] (NEED_*) of every access that waits for another or
 // is waited for (the caller fills need with NEED_FREE first), counters[row] =
 // 0 for the rows where that happens.  With comb.min > 0 every row queue of at
-// least comb.min accesses is listed for gacco_combine.  conflicts (may be
+// least comb.min accesses is listed for gacco_combine or tpcc_combine, none
+// once a launch of the run reported an error.  conflicts (may be
 // null): neighbours with equal keys where either writes, added to
 // CONFLICT_SLOTS counters 16 words apart.  tmp holds seg_tmp_words(n) u32.
 constexpr uint32_t CONFLICT_SLOTS = 16;
@@ -109,7 +110,7 @@ struct CombArgs {
   uint64_t* reads;
   uint32_t* need;
   unsigned long long* combined;
-  const uint64_t* error;   // TPC-C: the run's error word (Metrics::error_flags; 0: none so far)
+  const uint64_t* error;   // the run's error word (Metrics::error_flags; 0: none so far)
 };
 constexpr uint32_t COMB_CHUNKS = 0, COMB_SUMS = 1, COMB_MULTI = 2, COMB_WORDS = 4;
 uint64_t comb_chunk_cap(uint64_t nops, uint32_t min);
@@ -155,8 +156,7 @@ hipError_t ord_filter(const IndexView& ix, const uint64_t* ops, const uint32_t* 
 // cells (cols <= 64), store its reads' results, mark its ops need = NEED_DONE
 // and add the ops run to *combined.  srow, sop: the sorted accesses.
 hipError_t gacco_combine(const CombArgs& c, const uint32_t* srow, const uint32_t* sop, hipStream_t s);
-// TPC-C, GaccO: the same for queues of updates (c.whole), one wave per queue;
-// nothing once an earlier launch of the run reported an error.
+// TPC-C, GaccO: the same for queues of updates (c.whole), one wave per queue.
 hipError_t tpcc_combine(const CombArgs& c, const uint32_t* srow, const uint32_t* sop, hipStream_t s);
 // Open form, one admitted batch sorted by (row, op) with group starts gstart
 // and row starts rstart: need[op] = base[row] + gstart[p] - rstart[p]; then

@@ -1000,7 +1000,8 @@ constexpr uint32_t CB_BT = 256;  // accesses per combiner chunk, one per thread
 // need[op] (op = val & OPID_MASK) of every access that waits or is waited
 // for; the others keep NEED_FREE.  The counter of a row where that happens is
 // set to 0 at the row's first access.  comb.min > 0: every row queue of at
-// least comb.min accesses is listed for its combiner (CombArgs).
+// least comb.min accesses is listed for its combiner (CombArgs), unless an
+// earlier launch of the run reported an error.
 // conflicts (GPUTx): same-row neighbours of equal key (row and rank) where
 // either writes, added to CONFLICT_SLOTS counters on lines of their own.
 template <class KT, int TT_ITEMS>
@@ -1086,7 +1087,10 @@ __global__ __launch_bounds__(BT) void k_seg_turns(const KT* key, const uint32_t*
       if (q == n || (k1 >> rb) != (t.k[i] >> rb)) qlen[i] = p + 2 - at.row;
     }
   }
-  if (comb.min) {
+  // After an error no queue is listed: a batch's launch will do nothing either
+  // (txn_exec).  Asked here, in a kernel of many blocks: in k_tpcc_combine's own
+  // few first instructions it moved the update loop, 61 -> 65 ns per payment.
+  if (comb.min && *comb.error == 0) {
     // file the queues long enough: their chunks, and those of more than one
     // chunk once more for the carry between their chunks
     const uint32_t step = comb.whole ? 0x7fffffffu : CB_BT;
@@ -1354,8 +1358,7 @@ __device__ __forceinline__ uint64_t tpcc_run(uint32_t kind, uint32_t param, uint
   return mine;
 }
 __global__ __launch_bounds__(TC_BT) void k_tpcc_combine(launch::CombArgs c, const uint32_t* srow, const uint32_t* sop) {
-  // after an error no queue counts, as the batch's launch will do nothing either (txn_exec)
-  const uint32_t nq = min(c.ctr[launch::COMB_CHUNKS], *c.error ? 0u : c.chunk_cap);
+  const uint32_t nq = min(c.ctr[launch::COMB_CHUNKS], c.chunk_cap);
   const uint32_t lane = threadIdx.x % 64;
   for (uint32_t x = (blockIdx.x * TC_BT + threadIdx.x) / 64; x < nq; x += gridDim.x * (TC_BT / 64)) {
     const uint4 q = c.chunks[x];

@@ -162,13 +162,11 @@ hipError_t radix_sort_u32(uint32_t* k0, uint32_t* v0, uint32_t*, uint32_t*, uint
   return hipSuccess;
 }
 hipError_t seg_turns(const uint32_t*, const uint32_t*, uint64_t, int, uint32_t*, uint32_t*, uint32_t*, uint64_t,
-                     const CombArgs&, uint64_t*, hipStream_t, const uint32_t*) {
+                     const CombArgs& c, uint64_t*, hipStream_t, const uint32_t*) {
+  combined += c.min && *c.error == 0;  // as k_seg_turns
   return hipSuccess;
 }
-hipError_t tpcc_combine(const CombArgs& c, const uint32_t*, const uint32_t*, hipStream_t) {
-  combined += *c.error == 0;  // as k_tpcc_combine
-  return hipSuccess;
-}
+hipError_t tpcc_combine(const CombArgs&, const uint32_t*, const uint32_t*, hipStream_t) { return hipSuccess; }
 hipError_t fill_u64(uint64_t* v, uint64_t n, uint64_t x, hipStream_t) {
   for (uint64_t i = 0; i < n; ++i) v[i] = x;
   return hipSuccess;

@@ -54,31 +54,34 @@ def combine(tmp_path_factory):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("failed", [0, 1, 3])
-def test_tpcc_combiner_after_an_error(combine, failed):
+@pytest.mark.parametrize("error", [0, 16, (3 << 32) | 16])
+def test_tpcc_combiner_after_an_error(combine, error):
     """TPC-C under GaccO applies a batch's queues before its launch: not once an
     earlier launch has reported an error."""
-    lens = np.array([70, 3], dtype=np.uint32)
+    lens = np.array([70, 1, 3])
     nops, rows = int(lens.sum()), 4
-    rng = np.random.default_rng(failed)
+    rng = np.random.default_rng(5)
     w = g.tpcc_generate(1, nops, new_order=False, seed=3)
     first = w.tx_off[:-1].astype(np.int64)  # each payment's warehouse update
     ops, params = np.ascontiguousarray(w.ops[first]), np.ascontiguousarray(w.params[first])
-    srow = np.repeat(np.array([1, 3], dtype=np.uint32), lens)
+    srow = np.repeat(np.array([0, 1, 3], dtype=np.uint32), lens)
     sop = np.arange(nops, dtype=np.uint32) | np.uint32(1 << 31)
     cells = rng.integers(0, 1 << 30, rows * 5).astype(np.uint64)
-    reads, need = np.full(nops, 7, dtype=np.uint64), np.full(nops, 5, dtype=np.uint32)
-    out_c, out_r, out_n = cells.copy(), reads.copy(), need.copy()
+    reads, need = np.full(nops, 7, dtype=np.uint64), np.full(nops, 1 << 31, dtype=np.uint32)
+    out_c, out_r, out_n, listed = cells.copy(), reads.copy(), need.copy(), C.c_uint32(9)
     ptr = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
-    print(f"[error-stop] combiner failed={failed}", flush=True)
-    rc = combine(C.c_uint32(2), ptr(lens), ptr(srow), ptr(sop), C.c_uint32(nops), ptr(ops), ptr(params), C.c_uint64(rows),
-                 ptr(out_c), ptr(out_r), ptr(out_n), C.c_uint64(failed))
-    assert rc == 0
-    if not failed:
-        for i in range(nops):
+    print(f"[error-stop] combiner error={error}", flush=True)
+    rc = combine(ptr(srow), ptr(sop), C.c_uint32(nops), ptr(ops), ptr(params), C.c_uint64(rows), ptr(out_c), ptr(out_r),
+                 ptr(out_n), C.c_uint64(error), C.byref(listed))
+    assert rc == 0 and listed.value == (0 if error else 2)
+    for i in np.flatnonzero(srow != 1):
+        if error:  # the queues keep their turns
+            at = i if srow[i] == 0 else i - 71
+            need[i] = at | (1 << 31 if at == lens[srow[i] if srow[i] == 0 else 2] - 1 else 0)
+        else:
             row = cells[5 * int(srow[i]):5 * int(srow[i]) + 5]
             reads[i] = orc.lib().orc_tpcc_apply(int(g.op_col(ops[i:i + 1])[0]), int(params[i]), row)
-        need[:] = 0xFFFFFFFF
+            need[i] = 0xFFFFFFFF
     assert np.array_equal(out_c, cells) and np.array_equal(out_r, reads) and np.array_equal(out_n, need)
 
 
